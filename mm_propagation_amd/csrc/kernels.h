@@ -124,6 +124,8 @@ struct HeadArgs {
   int update_prev;     // 1 when this head is the last reader of e_prev in the step
   int chain_next;      // with final_stage: also build stage 0 of the next step (E_0 in e_cur, no a terms)
   int advance_z;       // with final_stage: z += h, steps += 1 on the fiber's StepState
+  int n_stash;         // of the a_ij below, those whose N_j is read from the stash (the first ones)
+  int prev_term;       // 1 when the last of them is a_i,i-1 (N_{i-1} comes from registers)
   int n_a;             // number of nonzero a_ij, j < i, in increasing j
   int a_idx[kMaxStages];    // j (N_{i-1} comes from registers, earlier N_j from stash)
   double a_coef[kMaxStages];  // a_ij (the fiber's a_ij h come from Batch::coef)

@@ -99,7 +99,12 @@ __device__ __forceinline__ cd cmul_exact(cd a, cd b) {
 
 // RE: Lawson factors computed from Im L and the fiber's z (HeadArgs::recompute_e) instead of
 // read from the tables; they are formed where they are used, so no table registers stay live.
-template <int L, class W, bool RE>
+// ST: stage i's argument takes stashed N_j (the tableaux beyond RK4). In FP64 two of them are requested
+// together, since each trip to memory is exposed (a lone fiber's head has one wavefront per SIMD at
+// most), and RK4 runs without that code: 5 modes, NT = 8192, sixth order 176.2 -> 164.6 us per step, RK4
+// of two modes 71.2 -> 70.2. The table-free form has no registers for two (its second wavefront per SIMD
+// would go), and without the loop its batched heads measured 3 % slower, so it keeps one form.
+template <int L, class W, bool RE, bool ST>
 __global__ void __launch_bounds__(RowCfg<L>::THREADS) k_row_head(Geometry g, const cpx<W>* __restrict__ rowtw, HeadArgs a, Batch b) {
   using C = RowCfg<L>;
   using cw = cpx<W>;
@@ -108,7 +113,7 @@ __global__ void __launch_bounds__(RowCfg<L>::THREADS) k_row_head(Geometry g, con
   const int gl = tid / C::T, t = tid % C::T;
   const int row = blockIdx.x * C::G + gl;
   const bool valid = row < g.M * g.N1;
-  const size_t base = valid ? (size_t)row * g.N2 + t : t;
+  const size_t base = valid ? (size_t)row * g.N2 + t : t;  // (lanes without a row: in bounds, not stored)
   cw* sm = smem + gl * C::SLOTS;
   const size_t MN = (size_t)g.M * g.N;
   // fiber blockIdx.y of the batch: its arrays and scalars
@@ -171,17 +176,30 @@ __global__ void __launch_bounds__(RowCfg<L>::THREADS) k_row_head(Geometry g, con
   }
   // stage i's argument psi + sum_j a_ij h N_j over j < i in increasing j: the stashed N_j now,
   // N_{i-1} (the largest j, from this head's transform) last
-  const bool prev_term = a.n_a > 0 && a.a_idx[a.n_a - 1] == a.prev_stage;
-  if (!a.final_stage) {
+  if constexpr (ST) {
+    int e = 0;
+    if constexpr (!RE) {
+#pragma unroll 1
+      for (; e + 2 <= a.n_stash; e += 2) {
+        const cd* n0 = stash + (size_t)a.a_idx[e] * MN + base;
+        const cd* n1 = stash + (size_t)a.a_idx[e + 1] * MN + base;
+        cd t0[8], t1[8];
 #pragma unroll
-    for (int e = 0; e < kMaxStages; e++) {
-      if (e >= a.n_a - (prev_term ? 1 : 0)) break;
-      const int j = a.a_idx[e];
+        for (int i = 0; i < 8; i++) t0[i] = n0[i * C::T];
 #pragma unroll
-      for (int i = 0; i < 8; i++) {
-        const cd nj = valid ? stash[(size_t)j * MN + base + i * C::T] : zero;
-        x[i] = cadd(x[i], cscale(nj, hc[1 + e]));
+        for (int i = 0; i < 8; i++) t1[i] = n1[i * C::T];
+#pragma unroll
+        for (int i = 0; i < 8; i++) x[i] = cadd(cadd(x[i], cscale(t0[i], hc[1 + e])), cscale(t1[i], hc[2 + e]));
       }
+    }
+#pragma unroll 1
+    for (; e < a.n_stash; e++) {
+      const cd* n0 = stash + (size_t)a.a_idx[e] * MN + base;
+      cd t0[8];
+#pragma unroll
+      for (int i = 0; i < 8; i++) t0[i] = n0[i * C::T];
+#pragma unroll
+      for (int i = 0; i < 8; i++) x[i] = cadd(x[i], cscale(t0[i], hc[1 + e]));
     }
   }
   // the Lawson table of stage i-1 moves on by E1 (it is not read again in this step)
@@ -193,7 +211,7 @@ __global__ void __launch_bounds__(RowCfg<L>::THREADS) k_row_head(Geometry g, con
   }
   if (a.has_prev) {
     const double bh = hc[0];
-    const double cprev = prev_term ? hc[a.n_a] : 0.;
+    const double cprev = a.prev_term ? hc[a.n_a] : 0.;
     line_fft<L, -1, 1, 1>(v, sm, lt, t);
     bool finite = true;
 #pragma unroll
@@ -213,7 +231,7 @@ __global__ void __launch_bounds__(RowCfg<L>::THREADS) k_row_head(Geometry g, con
         if (a.stash_prev) store_stream(stash + (size_t)a.prev_stage * MN + idx, nh);
       }
       if (a.final_stage) x[i] = acc;  // chain_next: stage 0 of the next step from the new psi_hat
-      else if (prev_term) x[i] = cadd(x[i], cscale(nh, cprev));
+      else if (a.prev_term) x[i] = cadd(x[i], cscale(nh, cprev));
       if constexpr (RE) {
         if (same) x[i] = cmul(epi, x[i]);  // E_i x_i
       }
@@ -1513,13 +1531,17 @@ static hipError_t row_head_impl(const Geometry& g, const Twiddles& tw, const Hea
   using C = RowCfg<L>;
   const int rows = g.M * g.N1;
   dim3 grid((rows + C::G - 1) / C::G, F);
-  // the table-free form only for FP32 work arrays (mixed precision)
-  if (a.recompute_e && !std::is_same<W, float>::value) return hipErrorInvalidValue;
-  if (a.recompute_e)
-    MMP_LAUNCH((k_row_head<L, W, std::is_same<W, float>::value>), grid, dim3(C::THREADS), 0, s, g,
-               TwOf<W>::row(tw), a, b);
-  else
-    MMP_LAUNCH((k_row_head<L, W, false>), grid, dim3(C::THREADS), 0, s, g, TwOf<W>::row(tw), a, b);
+  // FP32 work arrays (mixed precision) take the table-free form, FP64 ones the tables
+  constexpr bool RE = std::is_same<W, float>::value;
+  if ((a.recompute_e != 0) != RE) return hipErrorInvalidValue;
+#define MMP_HEAD(ST) MMP_LAUNCH((k_row_head<L, W, RE, ST>), grid, dim3(C::THREADS), 0, s, g, TwOf<W>::row(tw), a, b)
+  if constexpr (RE) {
+    MMP_HEAD(true);
+  } else {
+    if (a.n_stash > 0) MMP_HEAD(true);
+    else MMP_HEAD(false);
+  }
+#undef MMP_HEAD
   return hipGetLastError();
 }
 template <class W>

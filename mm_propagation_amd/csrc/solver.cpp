@@ -487,7 +487,7 @@ void release(mmp_solver* s) {
 
 // Lawson tables E_u (one per distinct c_u, advanced by E1 each step) exist in FP64 only: the
 // mixed-precision stage heads form E_u from Im L and the fiber's z where they use it.
-bool lawson_tables(const Problem& P, bool mixed) { return !(mixed && P.rk.s >= 2); }
+bool lawson_tables(bool mixed) { return !mixed; }
 
 // Device bytes create_impl allocates for F fibers of problem P (kept in step with its dalloc calls).
 size_t planned_device_bytes(const Problem& P, const mmp_options& opt, size_t F) {
@@ -498,7 +498,7 @@ size_t planned_device_bytes(const Problem& P, const mmp_options& opt, size_t F) 
   for (int j = 0; j < P.rk.s; j++) any_stash = any_stash || P.stash_needed[j];
   size_t b = 16 * MN * (2 * F + 2 * Fw) + 8 * MN * F + 16 * (P.N2 + P.N1 + P.N) + sizeof(StepState) * F +
              sizeof(FiberParams) * F + 8 * kHeadCoef * ((size_t)P.rk.s + 1) * F + 8 * c(P.M);
-  if (lawson_tables(P, mixed)) b += 16 * MN * F * (2 * P.c_unique.size() + 1);
+  if (lawson_tables(mixed)) b += 16 * MN * F * (2 * P.c_unique.size() + 1);
   if (any_stash) b += 16 * (size_t)P.rk.s * MN * F;
   if (P.raman) b += (mixed ? 8 : 16) * c(L) * P.N * F + 16 * (size_t)P.N * F + 8 * (size_t)P.N;
   b += 4 * c(P.coff.size()) + 4 * c(P.nnz) + 8 * c(P.nnz) + 4 * 4 * c(P.P) + 4 * 3 * c(L);
@@ -721,7 +721,7 @@ mmp_status create_impl(mmp_ctx* ctx, uint32_t n_fibers, const mmp_params* params
   A(dalloc(s, &s->ybuf, Fw * MN));
   A(dalloc(s, &s->U, Fw * MN));
   A(dalloc(s, &s->imL, F * MN));
-  if (lawson_tables(P, s->mixed)) {
+  if (lawson_tables(s->mixed)) {
     A(dalloc(s, &s->etab, F * s->batch.se));
     A(dalloc(s, &s->etab0, F * s->batch.se));
     A(dalloc(s, &s->e1, F * MN));
@@ -907,7 +907,7 @@ mmp_status create_impl(mmp_ctx* ctx, uint32_t n_fibers, const mmp_params* params
     a.final_stage = (i == P.rk.s);
     // mixed precision: Lawson factors from Im L and the step count (no tables exist); the close
     // head takes the count at the step's start from StepState::n0, which head 1 records
-    if (!lawson_tables(P, s->mixed)) {
+    if (!lawson_tables(s->mixed)) {
       a.recompute_e = 1;
       a.imL = s->imL;
       a.set_n0 = (i == 1);
@@ -936,6 +936,8 @@ mmp_status create_impl(mmp_ctx* ctx, uint32_t n_fibers, const mmp_params* params
           a.a_coef[a.n_a] = P.rk.a[i][j];
           a.n_a++;
         }
+      a.prev_term = a.n_a > 0 && a.a_idx[a.n_a - 1] == a.prev_stage;
+      a.n_stash = a.n_a - a.prev_term;
     }
     s->heads.push_back(a);
   }
