@@ -94,7 +94,7 @@ struct Batch {
   size_t sl;              // Raman line arrays (lines x NT)
   size_t se;              // Lawson table sets (tables x M x NT)
   size_t ss;              // stage stash (s x M x NT)
-  size_t sq;              // dense coupling blocks (P x M x M coefficients)
+  size_t sq;              // coupling blocks (coefficients)
   size_t sh;              // Raman spectra (NT)
 };
 
@@ -165,36 +165,66 @@ struct PairLineArgs {
   const uint32_t* line_self;  // [n_lines] 1 = packed self pairs, 0 = cross pair a, b
 };
 
-// Column-stage kernels (one workgroup per column, Raman on, N1 = 64, M <= 16): Raman lines
-// are processed in chunks; chunk c covers lines [chunk_line[c], chunk_line[c+1]) and their
-// slots [chunk_slot[c], chunk_slot[c+1]) (slots are numbered by line).
-struct FusedArgs {
+// Column-stage kernels (one workgroup per column, Raman on, N1 = 64, M <= 16). A Raman line carries
+// two real products as its real and imaginary parts, each Re or Im of U_a conj(U_b); lines are
+// processed in chunks, chunk c covers lines [chunk_line[c], chunk_line[c+1]).
+// line_prod: the two products of a line, a | b << 8 | im << 16 | absent << 17.
+
+// FP64 sums the real products themselves (setup.h).
+struct ProductArgs {
+  const uint32_t* chunk_line;  // [n_chunks + 1]
+  const uint2* line_prod;      // [lines]
+  int n_chunks, max_chunk_lines;
+  int first_lines;             // chunk_line[1]
+  int n_lines;                 // lines in use (those of the Re products, or of all)
+  int n_products;              // products in use
+  const uint32_t* steps;       // first product | segment << 28 | another step of the chunk follows << 30 | last
+                               // of its segment in the chunk << 31 of each step, padded to a multiple
+                               // of 64 + 64
+  int n_steps;                 // steps in use
+  int odd_step;                // with one chunk: the first step of the odd parity class
+  int stride;                  // steps per mode of the coupling blocks (16 coefficients each)
+  int parity;                  // coupling rows hold only the entries (p, k) with (p + k) % 2 == the
+                               // segment's parity: ceil(M/2) per p, k = 2 kk + ((p + parity) % 2)
+  int waves;                   // wavefronts of the gather workgroup: 4; 8 (one column); 12 (one column at 5
+                               // and 6 modes with parity rows and one chunk)
+  int cols;                    // neighbouring columns per gather workgroup (colstage_cols_ok; more than
+                               // one with 4 wavefronts); same arithmetic, same results
+};
+
+// FP32 (mixed precision) sums the complex slots X_s = kv U_a conj(U_b) + kr (its line as is, conjugated,
+// or its real or imaginary part); slots are numbered by line.
+struct SlotArgs {
   const uint32_t* chunk_line;  // [n_chunks + 1]
   const uint32_t* chunk_slot;  // [n_chunks + 1]
   const uint32_t* slot_meta;   // [P] a | b << 8 | kind << 16 | parity << 18 | line << 19 of each slot
   int n_chunks, max_chunk_lines, max_chunk_slots;
+  int first_lines, first_slots;  // chunk_line[1], chunk_slot[1]
   int parity;                  // coupling blocks hold only the entries (p, k) with (p + k) % 2 == the
                                // slot's parity: M x ceil(M/2) per slot, k = 2 kk + ((p + parity) % 2)
   int waves;                   // wavefronts of the gather workgroup: 4, or 8 (colstage_wide_ok)
   int hi_occupancy;            // with 4 wavefronts: the three-workgroups-per-CU variant where it
-                               // exists (FP32, 7 to 10 modes); same arithmetic, same results
+                               // exists (7 to 10 modes); same arithmetic, same results
   int matrix_cores;            // with 4 wavefronts: the slot sums on the matrix cores where that
                                // variant exists (colstage_matrix_cores_ok); FP32 rounding differs
 };
 
-// Limits of one column-stage chunk: Raman lines, slots, and coupling coefficients
-// (slots x M x M) held in LDS; and the largest mode count.
 int colstage_max_modes();
-// Whether the 8-wavefront gather workgroup exists for M modes in this precision.
-bool colstage_wide_ok(int M, bool mixed);
-// Whether the three-workgroups-per-CU 4-wavefront gather exists (FusedArgs::hi_occupancy).
+bool colstage_cols_ok(int M, int cols);
+// Coefficients per mode and product of the FP64 coupling blocks: 16 / that many products a step.
+int colstage_coef_pad(int M, bool parity);
+// FP32: whether the 8-wavefront and the three-workgroups-per-CU 4-wavefront gathers exist.
+bool colstage_wide_ok(int M);
 bool colstage_hi_occupancy_ok(int M, bool mixed, bool parity);
-// Whether the matrix-core gather exists (FusedArgs::matrix_cores): FP32, 4 to 16 modes with
+// Whether the matrix-core gather exists (SlotArgs::matrix_cores): FP32, 4 to 16 modes with
 // parity-structured coupling blocks, 4 to 10 without.
 bool colstage_matrix_cores_ok(int M, bool mixed, bool parity);
-int colstage_lines_per_chunk(int M);
+int colstage_lines_per_chunk(int M);  // Raman lines of one LDS chunk at most
+// FP32: slots and coupling coefficients of one chunk at most.
 int colstage_slots_per_chunk();
 int colstage_coefficients_per_chunk(int M, bool mixed);
+constexpr size_t kColStageLds = 65536;      // dynamic LDS of one gather workgroup at most
+size_t colstage_products_lds_bytes(int M, int cols, int lines, int steps);
 constexpr size_t kColStagePairsLds = 65536;
 size_t colstage_pairs_lds_bytes(int M, int columns, bool mixed);
 // C1 layout for F fibers: four columns per workgroup where the LDS allows (else two, else
@@ -240,13 +270,16 @@ hipError_t launch_gather(const Geometry& g, const cpx<W>* U, const cpx<W>* VR, c
 // conv_cols: store the Raman lines in column order (for launch_row_raman_cols with in_cols).
 template <class W>
 hipError_t launch_colstage_fields_pairs(const Geometry& g, const Twiddles& tw, const cpx<W>* yin, cpx<W>* U,
-                                        cpx<W>* conv, int n_lines, const PairLineArgs& pl, double scale,
-                                        const Batch& b, int F, int columns, int groups, int conv_cols,
+                                        cpx<W>* conv, const uint2* line_prod, int n_lines, double scale,
+                                        const Batch& b, int F, int columns, int groups, int conv_cols, hipStream_t s);
+// Qp: the products' coupling blocks [p][step][16] (product_blocks).
+hipError_t launch_colstage_products(const Geometry& g, const Twiddles& tw, const cd* U, const cd* conv, cd* yout,
+                                    const ProductArgs& fa, const double* Qp, double scale, const Batch& b, int F,
+                                    hipStream_t s);
+// Qd: [slot][M][M] (or parity-compact) coupling blocks.
+hipError_t launch_colstage_raman_gather(const Geometry& g, const Twiddles& tw, const cf* U, const cf* conv, cf* yout,
+                                        const SlotArgs& fa, const float* Qd, double scale, const Batch& b, int F,
                                         hipStream_t s);
-template <class W>
-hipError_t launch_colstage_raman_gather(const Geometry& g, const Twiddles& tw, const cpx<W>* U, const cpx<W>* conv,
-                                        cpx<W>* yout, const GatherArgs& ga, const FusedArgs& fa, const W* Qd,
-                                        double scale, const Batch& b, int F, hipStream_t s);
 // Dense-block gather (M <= 16): Qd is [P][M][M] with Qd[s][p][k] = sum of Q/max|Q| over the
 // nonzeros (k, slot s) of Q^(p). dense_gather_chunk(M) is 0 when M is out of range.
 int dense_gather_chunk(int M);

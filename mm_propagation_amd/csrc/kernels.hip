@@ -836,14 +836,20 @@ struct ColStageCfg {
 
 int colstage_max_modes() { return kColStageMaxM; }
 
-// 8-wavefront gather workgroups: up to 12 modes in FP32, 6 in FP64 (beyond, the registers of
-// a 512-lane workgroup would spill)
-template <int M, class W>
-constexpr bool kColStageWide = std::is_same<W, float>::value ? M <= 12 : M <= 6;
-bool colstage_wide_ok(int M, bool mixed) { return mixed ? M <= 12 : M <= 6; }
+// Columns per C2 workgroup: one, two up to 10 modes (a wavefront pair per column; beyond, the sums'
+// registers leave one wavefront per SIMD), four up to 4 modes in the vector form
+constexpr int kColStageMaxM2 = 10, kColStageMaxM4 = 4;
+bool colstage_cols_ok(int M, int cols) {
+  return cols == 1 || (cols == 2 && M <= kColStageMaxM2) || (cols == 4 && M <= kColStageMaxM4);
+}
 int colstage_lines_per_chunk(int M) { return colstage_lines_cap(M); }
 int colstage_coefficients_per_chunk(int M, bool mixed) { return colstage_qcap(M, mixed); }
 int colstage_slots_per_chunk() { return kColStageSCap; }
+// FP32: 8-wavefront gather workgroups up to 12 modes (beyond, the registers of a 512-lane
+// workgroup would spill)
+template <int M, class W>
+constexpr bool kColStageWide = M <= 12;
+bool colstage_wide_ok(int M) { return M <= 12; }
 
 // C1 over CW neighbouring columns per workgroup, the column block's Raman lines dealt to
 // `groups` workgroups (each transforms every field of the block, group 0 stores them to U).
@@ -857,8 +863,8 @@ __global__ void __launch_bounds__(256) k_colstage_fields_pairs(Geometry g, const
                                                                const cpx<W>* __restrict__ fourtw,
                                                                const cpx<W>* __restrict__ yin, cpx<W>* __restrict__ U,
                                                                cpx<W>* __restrict__ conv, int n_lines,
-                                                               PairLineArgs pl, double scale, Batch b, int groups,
-                                                               int conv_cols) {
+                                                               const uint2* __restrict__ line_prod, double scale,
+                                                               Batch b, int groups, int conv_cols) {
   using F = ColStageCfg;
   using cw = cpx<W>;
   constexpr int L = F::L;
@@ -882,34 +888,31 @@ __global__ void __launch_bounds__(256) k_colstage_fields_pairs(Geometry g, const
   const int lend = lbeg + lpg < n_lines ? lbeg + lpg : n_lines;
   cw* fsm = sh + (jl * CW + c) * F::SLOTS;
   cw w4[8], v[8];
-  // the first round's field samples are requested before the twiddles, and the first round's
-  // line descriptors with them (each later round's during the round before)
-  {
-    const bool valid = jl < g.M;
-    const size_t base = (size_t)(valid ? jl : 0) * g.N + n2;
-#pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = valid ? yin[base + (size_t)(t + i * F::T) * g.N2] : cw{0, 0};
-  }
-  uint32_t la_n = 0, lb_n = 0, self_n = 0;
-  if (lbeg + jl < lend) {
-    la_n = pl.line_a[lbeg + jl];
-    lb_n = pl.line_b[lbeg + jl];
-    self_n = pl.line_self[lbeg + jl];
-  }
   LineTw<L, W> lt;
-  load_line_tw<L>(lt, coltw, t);
+  const int wave_jl0 = __builtin_amdgcn_readfirstlane(tid / 64) * (64 / (F::T * CW));  // first row job of this wavefront
+  // the first round's field samples are requested before the twiddles, and the first round's
+  // line descriptors with them (each later round's during the round before); wavefronts without a
+  // field or line load nothing (see C2)
+  if (wave_jl0 < g.M) {
+    const size_t base = (size_t)(jl < g.M ? jl : g.M - 1) * g.N + n2;
 #pragma unroll
-  for (int i = 0; i < 8; i++) w4[i] = fourtw[n2 * (t + i * F::T)];
+    for (int i = 0; i < 8; i++) v[i] = yin[base + (size_t)(t + i * F::T) * g.N2];
+  }
+  uint2 d_n = line_prod[lbeg + jl < n_lines ? lbeg + jl : n_lines - 1];
+  if (wave_jl0 < (lend - lbeg > g.M ? lend - lbeg : g.M)) {
+    load_line_tw<L>(lt, coltw, t);
+#pragma unroll
+    for (int i = 0; i < 8; i++) w4[i] = fourtw[n2 * (t + i * F::T)];
+  }
   const W sc = (W)scale;
-  const int wave_jl0 = (tid / 64) * (64 / (F::T * CW));  // first row job of this wavefront
   for (int r0 = 0; r0 < g.M; r0 += JL) {
     const int q = r0 + jl;
     const bool valid = q < g.M;
-    const size_t base = (size_t)(valid ? q : 0) * g.N + n2;
+    const size_t base = (size_t)(valid ? q : g.M - 1) * g.N + n2;
     if (r0 + wave_jl0 >= g.M) continue;  // no field of this wavefront in the round
     if (r0 > 0) {
 #pragma unroll
-      for (int i = 0; i < 8; i++) v[i] = valid ? yin[base + (size_t)(t + i * F::T) * g.N2] : cw{0, 0};
+      for (int i = 0; i < 8; i++) v[i] = yin[base + (size_t)(t + i * F::T) * g.N2];
     }
 #pragma unroll
     for (int i = 0; i < 8; i++) v[i] = cmulc(v[i], w4[i]);
@@ -929,23 +932,16 @@ __global__ void __launch_bounds__(256) k_colstage_fields_pairs(Geometry g, const
     const int q = r0 + jl;
     const bool valid = q < lend;
     if (r0 + wave_jl0 >= lend) continue;  // no line of this wavefront in this round or later
-    // cross line: U_a conj(U_b); self line: |U_a|^2 + i |U_b|^2 (b absent: 0)
-    const uint32_t la = la_n, lb = lb_n, self = self_n;  // lanes past the last line read line 0's
-    if (q + JL < lend) {
-      la_n = pl.line_a[q + JL];
-      lb_n = pl.line_b[q + JL];
-      self_n = pl.line_self[q + JL];
-    }
-    const bool has_b = lb != 0xffffffffu;
-    const int ia = (int)la * L * CW + c, ib = (int)(has_b ? lb : la) * L * CW + c;
-    const W bmask = has_b ? (W)1 : (W)0;
+    const uint2 d = d_n;
+    d_n = line_prod[q + JL < n_lines ? q + JL : n_lines - 1];
+    const int i0 = (int)(d.x & 255u) * L * CW + c, j0 = (int)((d.x >> 8) & 255u) * L * CW + c;
+    const int i1 = (int)(d.y & 255u) * L * CW + c, j1 = (int)((d.y >> 8) & 255u) * L * CW + c;
+    const bool im0 = (d.x >> 16) & 1u, im1 = (d.y >> 16) & 1u, has1 = !((d.y >> 17) & 1u);
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-      const int n1 = t + i * F::T;
-      const cw ua = Ush[ia + n1 * CW], ub = Ush[ib + n1 * CW];
-      const cw cross = cmulc(ua, ub);
-      const cw selfv = {ua.re * ua.re + ua.im * ua.im, bmask * (ub.re * ub.re + ub.im * ub.im)};
-      v[i] = !valid ? cw{0, 0} : (self ? selfv : cross);
+      const int o = (t + i * F::T) * CW;
+      const cw x0 = cmulc(Ush[i0 + o], Ush[j0 + o]), x1 = cmulc(Ush[i1 + o], Ush[j1 + o]);
+      v[i] = {im0 ? x0.im : x0.re, has1 ? (im1 ? x1.im : x1.re) : (W)0};
     }
     line_fft<L, -1, 1, 1, W, true>(v, fsm, lt, t);
     if (valid) {
@@ -962,6 +958,392 @@ __global__ void __launch_bounds__(256) k_colstage_fields_pairs(Geometry g, const
   }
 }
 
+// Coupling coefficients of the vector gather: 16 to a register (pair), those of mode p for
+// G = 16 / QP consecutive products, QP each (the QROW coefficients padded to 4, 8 or 16). Lane l of
+// each row of 16 lanes holds the l-th, and an FMAC takes its coefficient by DPP row broadcast: no
+// scalar load or LDS read per coefficient. A step is one such register for every mode; the steps go
+// through the segments in order, and a group of products that two segments share has a step in
+// each, the other segment's products with zeros.
+constexpr int coef_pad(int q) { return q <= 4 ? 4 : (q <= 8 ? 8 : 16); }
+int colstage_coef_pad(int M, bool parity) { return coef_pad(parity ? (M + 1) / 2 : M); }
+
+// B[k] += c[N + k] x for k < Q, c[n] being lane n of each row of 16 lanes. The s_nop covers the two
+// wait states a DPP operand needs after a VALU write of it (a register copy that the compiler may
+// place before the block).
+#define MMP_BC(OP, K, N) "\n\t" OP " %" #K ", %[c], %[x] row_newbcast:%c[" #N "] row_mask:0xf bank_mask:0xf"
+#define MMP_FMAC_BCAST(OP)                                                                                             \
+  if constexpr (Q == 1)                                                                                                \
+    asm("s_nop 1" MMP_BC(OP, 0, n0) : "+v"(B[0]) : [c] "v"(c), [x] "v"(x), [n0] "n"(N));                               \
+  if constexpr (Q == 2)                                                                                                \
+    asm("s_nop 1" MMP_BC(OP, 0, n0) MMP_BC(OP, 1, n1)                                                                  \
+        : "+v"(B[0]), "+v"(B[1])                                                                                       \
+        : [c] "v"(c), [x] "v"(x), [n0] "n"(N), [n1] "n"(N + 1));                                                       \
+  if constexpr (Q == 3)                                                                                                \
+    asm("s_nop 1" MMP_BC(OP, 0, n0) MMP_BC(OP, 1, n1) MMP_BC(OP, 2, n2)                                                \
+        : "+v"(B[0]), "+v"(B[1]), "+v"(B[2])                                                                           \
+        : [c] "v"(c), [x] "v"(x), [n0] "n"(N), [n1] "n"(N + 1), [n2] "n"(N + 2));                                      \
+  if constexpr (Q >= 4)                                                                                                \
+    asm("s_nop 1" MMP_BC(OP, 0, n0) MMP_BC(OP, 1, n1) MMP_BC(OP, 2, n2) MMP_BC(OP, 3, n3)                              \
+        : "+v"(B[0]), "+v"(B[1]), "+v"(B[2]), "+v"(B[3])                                                               \
+        : [c] "v"(c), [x] "v"(x), [n0] "n"(N), [n1] "n"(N + 1), [n2] "n"(N + 2), [n3] "n"(N + 3));
+template <int Q, int N, class W>
+__device__ __forceinline__ void fmac_bcast(W* B, W c, W x) {
+  static_assert(Q >= 1 && N + Q <= 16, "coefficients of one register");
+  if constexpr (std::is_same<W, float>::value) {
+    MMP_FMAC_BCAST("v_fmac_f32_dpp")
+  } else {
+    MMP_FMAC_BCAST("v_fmac_f64_dpp")
+  }
+  if constexpr (Q > 4) fmac_bcast<Q - 4, N + 4>(B + 4, c, x);
+}
+#undef MMP_FMAC_BCAST
+#undef MMP_BC
+
+// LDS of the products' C2: field rows (whole wavefronts of line slots, so that the transform of sigma has its
+// rows there), then the rows of a chunk's lines, which sigma takes over.
+// Steps of the vector gather whose coefficients are preloaded in registers (up to 6 modes): every
+// product once, and a shared group per further segment.
+constexpr int steps_cap(int M, bool parity) {
+  const int G = 16 / coef_pad(parity ? (M + 1) / 2 : M);
+  return (M * M + G - 1) / G + 3;
+}
+template <int M, int COLS, class W, bool PAR>
+struct C2Cfg {
+  static constexpr int UR = (M + 7) / 8 * 8;
+  static constexpr int STEPS = steps_cap(M, PAR);
+  static __host__ __device__ size_t q_offset(int lines) {
+    const int jw = 8 / COLS, rows = (lines + jw - 1) / jw * jw, sig = 2 * M;
+    return (size_t)(UR + (OWN ? rows + sig : (rows > sig ? rows : sig))) * COLS * kColStageRS * sizeof(cpx<W>);
+  }
+  // sigma in rows of its own (one barrier less) where one column's LDS leaves room for them
+  static constexpr bool OWN = COLS == 1 && M <= 6;
+  // vector form with two wavefronts per mode and column, one for each parity class
+  template <int NW>
+  static constexpr bool cs() { return PAR && M <= 6 && NW / COLS >= 2 * M; }
+};
+size_t colstage_products_lds_bytes(int M, int cols, int lines, int steps) {
+  const int jw = 8 / cols, rows = (lines + jw - 1) / jw * jw, sig = 2 * M;
+  const bool own = cols == 1 && M <= 6;
+  return (size_t)((M + 7) / 8 * 8 + (own ? rows + sig : (rows > sig ? rows : sig))) * cols * kColStageRS * sizeof(cd) +
+         (M <= 6 ? ((size_t)M * steps + 4) * 16 * sizeof(double) : 0);  // (+ 4: steps read ahead)
+}
+
+// B[kk] += over the G = 16 / QP products of one coefficient register
+template <int QROW, int QP, int I = 0, class W>
+__device__ __forceinline__ void group_fmac(W* B, W c, const W* x) {
+  fmac_bcast<QROW, I * QP>(B, c, x[I]);
+  if constexpr ((I + 1) * QP < 16) group_fmac<QROW, QP, I + 1>(B, c, x);
+}
+
+// The vector gather's steps over the products [xc0, xc1) of one chunk, for the modes
+// p = sub + j WPC < M of this wavefront and the sample of this lane: B[p][kk] per segment, then
+// acc (even parity class) or acc2 (odd) += U_k B. Xc: the sample in the chunk's first X row (rows of
+// RS reals, the two products of a line together, COLS columns per line); Uc: in field row 0. The
+// coefficients come from LDS (QL) or by `coefs`, PD steps ahead. CS: parity class `cls` only.
+template <int QROW, int NP, int PD, int WPC, int COLS, int RS, bool PAR, bool QL, bool CS, class W, class Coefs, int PQ,
+          int P2>
+__device__ __forceinline__ void product_sums(const ProductArgs& fa, const W* Qsh, const W* Xc, const cpx<W>* Uc, int xc0,
+                                             int xc1, int M, int sub, int cls, bool busy, int lane, int& step,
+                                             uint32_t& sdesc, W (&cq)[PQ][NP], const Coefs& coefs, cpx<W> (&acc)[NP],
+                                             cpx<W> (&acc2)[P2]) {
+  using cw = cpx<W>;
+  constexpr int QP = coef_pad(QROW), G = 16 / QP;
+  auto xrow = [&](int x) { return ((x >> 1) * COLS * 2 + (x & 1)) * RS; };  // of product xc0 + x
+  W B[NP][QROW];
+#pragma unroll
+  for (int j = 0; j < NP; j++)
+#pragma unroll
+    for (int kk = 0; kk < QROW; kk++) B[j][kk] = (W)0;
+  // PD steps with their coefficients in PD fixed registers, each loaded again for the step PD
+  // further on as soon as it is used
+  // lane i: step i of its 64: offset of its X values (G products of one line, or of two neighbouring
+  // ones) in place of its first product (steps of other chunks: any valid place)
+  uint32_t sx = 0;
+  auto describe = [&]() {
+    const int x = (int)(sdesc & 0xffffu);
+    sx = (sdesc & 0xf0000000u) | (uint32_t)xrow(x >= xc0 && x < xc1 ? x - xc0 : 0);
+  };
+  describe();
+  W xv[PD][G], cl[PD][NP];
+  uint32_t sd[PD];
+  const W* ql[NP];  // QL: step's coefficients
+#pragma unroll
+  for (int j = 0; j < NP; j++)
+    ql[j] = Qsh + ((sub + j * WPC < M ? sub + j * WPC : 0) * fa.stride + step) * 16 + (lane & 15);
+  auto operands = [&](int s, int u, int qo) {
+    if constexpr (!QL) {  // (QL: fewer than 64 steps)
+      if (s > 0 && (s & 63) == 0) {
+        sdesc = fa.steps[s + lane];
+        describe();
+      }
+    }
+    sd[u] = __builtin_amdgcn_readlane(sx, QL ? s : s & 63);
+    const W* xs = Xc + (sd[u] & 0xfffffffu);
+#pragma unroll
+    for (int i = 0; i < G; i++) xv[u][i] = xs[xrow(i)];
+    if constexpr (QL) {
+#pragma unroll
+      for (int j = 0; j < NP; j++) cl[u][j] = ql[j][qo];
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < PD; u++) operands(step + u, u, u * 16);
+  // (CS: wavefronts beyond the modes' and classes with no product have nothing to sum)
+  bool more = !CS || (busy && (cls ? fa.odd_step < fa.n_steps : fa.odd_step > 0));
+#pragma unroll 1
+  while (more) {
+#pragma unroll
+    for (int u = 0; u < PD; u++) {
+      const uint32_t sdu = sd[u];
+#pragma unroll
+      for (int j = 0; j < NP; j++) group_fmac<QROW, QP>(B[j], QL ? cl[u][j] : cq[QL ? 0 : u][j], xv[u]);
+      if constexpr (!QL) coefs(step + PD, cq[u]);
+      operands(step + PD, u, (PD + u) * 16);  // (past the last step: any valid place)
+      step++;
+      if (!(sdu >> 31)) continue;
+      // the segment (or the chunk's part of it) is complete
+      const int sg = (sdu >> 28) & 3u;
+#pragma unroll
+      for (int j = 0; j < NP; j++) {
+        const int par = PAR ? ((sub + j * WPC + sg) & 1) : 0;
+        cw sum = {0, 0};
+#pragma unroll
+        for (int kk = 0; kk < QROW; kk++) {
+          sum = cadd(sum, cscale(Uc[((PAR ? 2 * kk : kk) + par) * COLS * RS], B[j][kk]));
+          B[j][kk] = (W)0;
+        }
+        if (sg >= 2) sum = {-sum.im, sum.re};
+        if constexpr (!CS && PAR) {  // (selects of values: of places would put the sums in scratch memory)
+          const bool odd = sg & 1;
+          const cw even = cadd(acc[j], sum), odds = cadd(acc2[CS || !PAR ? 0 : j], sum);
+          acc[j] = {odd ? acc[j].re : even.re, odd ? acc[j].im : even.im};
+          cw& o = acc2[CS || !PAR ? 0 : j];
+          o = {odd ? odds.re : o.re, odd ? odds.im : o.im};
+        } else {
+          acc[j] = cadd(acc[j], sum);
+        }
+      }
+      more = ((sdu >> 30) & 1u) && !(CS && !cls && step == fa.odd_step);
+      if (!more) break;
+    }
+#pragma unroll
+    for (int j = 0; j < NP; j++) ql[j] += PD * 16;
+  }
+}
+
+// C2 over COLS neighbouring columns per workgroup. Lanes are ordered column-fastest as in C1, each
+// line transform runs inside one wavefront, in place in its padded LDS row, and wavefronts without
+// a line skip it. Each line's row is then mixed into its two real products' slot mixes
+// X = kv Re|Im(U_a conj U_b) + kr (the line's real|imaginary part), in its place (two X rows of RS
+// reals), by whole wavefronts. NW / COLS wavefronts then sum each column: wavefront `sub` of a column
+// takes the modes p = sub, sub + NW / COLS, ... (product_sums). The sum over the products runs in
+// their order whatever NW and COLS are.
+// Bound by latency for one fiber (a workgroup per CU or two: loads, line transform, mix, sums and
+// transform follow one another), by the FP64 units from 10 modes on. Summing complex slots took 18 Raman lines
+// instead of 11 at 6 modes and 4 to 5 times the coupling sums. Whole step on one MI355X, before and after: 6 modes,
+// NT = 16384, RK4 111.5 -> 101.7 us; 2 modes, NT = 4096 71.1 -> 68.3 us; 5 modes without the
+// symmetric couplings (all products), NT = 8192, sixth order 164.6 -> 165.2 us (the one form kept).
+template <int M, int NW, int COLS, class W, bool PAR>
+__global__ void __launch_bounds__(NW * 64) k_colstage_products(
+    Geometry g, const cpx<W>* __restrict__ coltw, const cpx<W>* __restrict__ fourtw, const cpx<W>* __restrict__ U,
+    const cpx<W>* __restrict__ conv, cpx<W>* __restrict__ yout, ProductArgs fa, const W* __restrict__ Qp, double scale,
+    Batch b) {
+  using cw = cpx<W>;
+  using C2 = C2Cfg<M, COLS, W, PAR>;
+  const int fib = blockIdx.y;
+  const FiberParams fp = b.fp[fib];
+  if (!fp.live) return;  // uniform over the workgroup
+  U += fib * b.sf;
+  yout += fib * b.sf;
+  conv += fib * b.sl;
+  constexpr int L = kColStageL, T = L / 8, RS = kColStageRS, UR = C2::UR;
+  constexpr int NT = NW * 64;
+  constexpr int JL = NT / (T * COLS);  // lines of every column per round
+  constexpr int JW = 64 / (T * COLS);  // of which one wavefront holds
+  constexpr int WPC = NW / COLS;       // wavefronts per column
+  constexpr int QROW = PAR ? (M + 1) / 2 : M;  // coefficients per product and mode p
+  constexpr int UIN = (M * COLS * L + NT - 1) / NT;
+  static_assert(M >= 1 && M <= kColStageMaxM && JW >= 1 && WPC >= 1 && JL >= M, "modes or columns out of range");
+  extern __shared__ __align__(16) unsigned char c2_lds[];
+  cw* const Ush = reinterpret_cast<cw*>(c2_lds);  // field rows [UR][COLS] (zeros beyond M); transform rows of sigma
+  cw* const Rsh = Ush + UR * COLS * RS;           // line rows [lines][COLS], then their X rows; then sigma
+  W* const Xsh = reinterpret_cast<W*>(Rsh);
+  W* const Qsh = reinterpret_cast<W*>(c2_lds + C2::q_offset(fa.max_chunk_lines));  // coefficients (QL)
+  cw* const Ssh = C2::OWN ? Rsh + (fa.max_chunk_lines + 7) / 8 * 8 * RS : Rsh;  // sigma rows
+  const int tid = threadIdx.x;
+  const int c = tid % COLS, t = (tid / COLS) % T, jl = tid / (T * COLS);
+  const int lane = tid % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int n20 = xcd_block(blockIdx.x, gridDim.x) * COLS, n2 = n20 + c;
+  // The first chunk's lines, the field samples and the coefficients are requested before anything
+  // waits on memory, each by the wavefronts that use it only: the vector memory pipe takes a
+  // wavefront's 16-byte loads at 64 bytes a cycle, and eight wavefronts loading every twiddle kept
+  // a lone workgroup's first line waiting for 3000 cycles.
+  cw v[8], uin[UIN], w4[8];
+  LineTw<L, W> lt;
+  int l0 = 0, l1 = fa.first_lines;
+  if (wave * JW < l1) {
+    const int q = jl < l1 ? jl : l1 - 1;  // lanes without a line read the last one's
+    const size_t base = (size_t)q * g.N + (size_t)n2 * L;
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] = conv[base + t + i * T];
+  }
+#pragma unroll
+  for (int r = 0; r < UIN; r++) {
+    const int e = tid + r * NT;
+    if (wave * 64 + r * NT < M * COLS * L)  // (whole wavefronts)
+      uin[r] = U[(size_t)(e / (COLS * L)) * g.N + (size_t)n20 * L + e % (COLS * L)];
+  }
+  if (wave * JW < (l1 > M ? l1 : M)) {
+    load_line_tw<L>(lt, coltw, t);
+#pragma unroll
+    for (int i = 0; i < 8; i++) w4[i] = fourtw[n2 * (t + i * T)];
+  }
+  const int col = wave % COLS, sub = wave / COLS;  // column of this wavefront's sums, its place there
+  // with two wavefronts per mode each takes one parity class (CS), else a wavefront takes the modes
+  // sub, sub + WPC, ... in both; the classes' sums are added last either way
+  constexpr bool CS = C2::template cs<NW>();
+  constexpr int NP = CS ? 1 : (M + WPC - 1) / WPC;  // modes of this wavefront
+  const int cls = CS && sub >= M ? 1 : 0, sub0 = CS ? (sub < M ? sub : (sub < 2 * M ? sub - M : 0)) : sub;
+  constexpr int QP = coef_pad(QROW), G = 16 / QP;   // products per coefficient register
+  // the steps' coefficients go through LDS where all of them fit (up to 6 modes), else
+  // each wavefront reads its modes' ahead of use, from cache lines requested here
+  constexpr bool QL = M <= 6;
+  constexpr int PD = QL ? 2 : 4;          // steps read ahead
+  const W* qf = Qp + fib * b.sq + (lane & 15);
+  auto coefs = [&](int s, W (&q)[NP]) {  // step s's coefficients of this wavefront's modes
+#pragma unroll
+    for (int j = 0; j < NP; j++) {
+      const int p = sub0 + j * WPC < M ? sub0 + j * WPC : 0;
+      q[j] = qf[((size_t)p * fa.stride + (s < fa.stride ? s : 0)) * 16];
+    }
+  };
+  constexpr int QIN = QL ? (M * C2::STEPS * 16 + NT - 1) / NT : 1;
+  W cq[QL ? 1 : PD][NP], qin[QIN], touch[QL ? 1 : NP];
+  uint32_t sdesc = fa.steps[lane];
+  {
+    if constexpr (QL) {
+      const int last = M * fa.stride * 16 - 1;
+#pragma unroll
+      for (int r = 0; r < QIN; r++)
+        if (wave * 64 + r * NT <= last) qin[r] = Qp[fib * b.sq + (tid + r * NT < last ? tid + r * NT : last)];
+    } else {
+#pragma unroll
+      for (int u = 0; u < PD; u++) coefs(u, cq[u]);
+#pragma unroll
+      for (int j = 0; j < NP; j++) {
+        const int p = sub0 + j * WPC < M ? sub0 + j * WPC : 0, e = lane * (128 / (int)sizeof(W));
+        touch[j] = Qp[fib * b.sq + (size_t)p * fa.stride * 16 + (e < fa.stride * 16 ? e : 0)];
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < UIN; r++) {
+    const int e = tid + r * NT;
+    if (wave * 64 + r * NT < M * COLS * L) Ush[(e / L) * RS + e % L] = uin[r];
+  }
+  // the field row after the last one, which the coupling rows of an odd number of modes read with
+  // zero coefficients
+  constexpr int UZ = M % 2 && PAR ? M + 1 : M;
+  for (int e = M * COLS * L + tid; e < UZ * COLS * L; e += NT) Ush[(e / L) * RS + e % L] = cw{0, 0};
+  if constexpr (QL) {
+#pragma unroll
+    for (int r = 0; r < QIN; r++)
+      if (tid + r * NT < M * fa.stride * 16) Qsh[tid + r * NT] = qin[r];
+    for (int e = tid + QIN * NT; e < M * fa.stride * 16; e += NT) Qsh[e] = Qp[fib * b.sq + e];
+  }
+  const W sc = (W)scale, kv = (W)fp.kv, kr = (W)fp.kr;
+  cw acc[NP], acc2[CS || !PAR ? 1 : NP];  // sums of the even (CS: its own) and of the odd parity class
+#pragma unroll
+  for (int p = 0; p < NP; p++) acc[p] = {0, 0};
+#pragma unroll
+  for (int p = 0; p < (CS || !PAR ? 1 : NP); p++) acc2[p] = {0, 0};
+  int step = cls ? fa.odd_step : 0;  // steps taken
+  for (int ch = 0; ch < fa.n_chunks; ch++) {
+    if (ch > 0) {
+      __syncthreads();  // X rows of the previous chunk consumed
+      l0 = l1;
+      l1 = (int)fa.chunk_line[ch + 1];
+      sdesc = fa.steps[(step & ~63) + lane];
+      if constexpr (!QL) {
+#pragma unroll
+        for (int u = 0; u < PD; u++) coefs(step + u, cq[u]);
+      }
+    }
+    // lane i: the products of the wavefront's i-th (line, column) row to mix
+    const int rows = (l1 - l0) * COLS;
+    const uint2 dl = fa.line_prod[l0 + (wave + NW * lane < rows ? (wave + NW * lane) / COLS : 0)];
+    for (int r0 = l0; r0 < l1; r0 += JL) {
+      if (r0 + wave * JW >= l1) break;  // no line of this wavefront in the round
+      const int q = r0 + jl;
+      const bool valid = q < l1;
+      if (ch > 0 || r0 > l0) {
+        const size_t base = (size_t)(valid ? q : l1 - 1) * g.N + (size_t)n2 * L;
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = conv[base + t + i * T];
+      }
+#pragma unroll
+      for (int i = 0; i < 8; i++) v[i] = cmulc(v[i], w4[i]);
+      cw* row = Rsh + ((q - l0) * COLS + c) * RS;
+      line_fft<L, 1, 1, 1, W, true>(v, row, lt, t);
+#pragma unroll
+      for (int i = 0; i < 8; i++) row[t + i * T] = v[i];
+    }
+    __syncthreads();  // the lines' and the fields' rows
+    // slot mixes, a row at a time by whole wavefronts (lane = sample): the two products of a line
+    // take the place of its samples
+#pragma unroll 1
+    for (int i = 0, r = wave; r < rows; i++, r += NW) {
+      const uint32_t d0 = __builtin_amdgcn_readlane(dl.x, i), d1 = __builtin_amdgcn_readlane(dl.y, i);
+      const cw* uc = Ush + (COLS > 1 ? r % COLS : 0) * RS + lane;
+      const cw V0 = cmulc(uc[(d0 & 255u) * COLS * RS], uc[((d0 >> 8) & 255u) * COLS * RS]);
+      const cw V1 = cmulc(uc[(d1 & 255u) * COLS * RS], uc[((d1 >> 8) & 255u) * COLS * RS]);
+      W* x0 = Xsh + r * 2 * RS + lane;
+      const cw vr = Rsh[r * RS + lane];
+      x0[0] = kv * ((d0 >> 16) & 1u ? V0.im : V0.re) + kr * (vr.re * sc);
+      x0[RS] = kv * ((d1 >> 16) & 1u ? V1.im : V1.re) + kr * (vr.im * sc);
+    }
+    if constexpr (!QL) {
+#pragma unroll
+      for (int j = 0; j < NP; j++) asm volatile("" ::"v"(touch[j]));
+    }
+    __syncthreads();
+    const int xc0 = 2 * l0, xc1 = 2 * l1 < fa.n_products ? 2 * l1 : fa.n_products;  // products of the chunk
+    const W* const Xc = Xsh + col * 2 * RS + lane;  // this lane's sample of the chunk's first X row
+    const cw* const Uc = Ush + col * RS + lane;     // this lane's sample of field k: Uc[k * COLS * RS]
+    product_sums<QROW, NP, PD, WPC, COLS, RS, PAR, QL, CS>(fa, Qsh, Xc, Uc, xc0, xc1, M, sub0, cls, sub < 2 * M, lane, step,
+                                                           sdesc, cq, coefs, acc, acc2);
+  }
+  if constexpr (!C2::OWN) __syncthreads();  // every lane done with the X rows, whose place sigma takes
+  // sigma rows [modes][COLS]; CS: a set for each parity class
+  constexpr int SETS = CS ? 2 : 1;
+#pragma unroll
+  for (int j = 0; j < NP; j++) {
+    if (CS ? sub < 2 * M : sub + j * WPC < M)
+      Ssh[((sub + j * WPC) * COLS + col) * RS + lane] = !CS && PAR ? cadd(acc[j], acc2[CS || !PAR ? 0 : j]) : acc[j];
+  }
+  __syncthreads();
+  if (wave * JW < M) {
+    const int q = jl;
+    const bool valid = q < M;
+    const cw* in = Ssh + ((valid ? q : 0) * COLS + c) * RS;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      v[i] = in[t + i * T];
+      if constexpr (SETS == 2) v[i] = cadd(v[i], in[M * COLS * RS + t + i * T]);
+    }
+    line_fft<L, -1, 1, 1, W, true>(v, Ush + (q * COLS + c) * RS, lt, t);
+    if (valid) {
+      const size_t base = (size_t)q * g.N + n2;
+#pragma unroll
+      for (int i = 0; i < 8; i++) store_stream64(yout + base + (size_t)(t + i * T) * g.N2, cmul(v[i], w4[i]));
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// C2 in FP32 (mixed precision): complex slots X_s and complex Raman lines
+// ---------------------------------------------------------------------------
 // 4-wavefront FP32 gathers of 7 to 10 modes also come in a variant held to 168 VGPRs, so
 // that three workgroups share a CU (their LDS is under 50 KB); it reads the coupling rows in
 // 64-byte groups to make room, and spills at most 12 dwords. Measured on one MI355X it pays
@@ -1011,8 +1393,7 @@ __global__ void __launch_bounds__(NW * 64, HI ? 3 : (MF ? (MfmaRows<M, PAR>::RT 
                                                                    const cpx<W>* __restrict__ fourtw,
                                                                    const cpx<W>* __restrict__ U,
                                                                    const cpx<W>* __restrict__ conv,
-                                                                   cpx<W>* __restrict__ yout, GatherArgs a,
-                                                                   FusedArgs fa, const W* __restrict__ Qd,
+                                                                   cpx<W>* __restrict__ yout, SlotArgs fa, const W* __restrict__ Qd,
                                                                    double scale, Batch b) {
   using cw = cpx<W>;
   const int fib = blockIdx.y;
@@ -1049,17 +1430,19 @@ __global__ void __launch_bounds__(NW * 64, HI ? 3 : (MF ? (MfmaRows<M, PAR>::RT 
   // the first chunk's lines, this lane's field samples, coupling blocks and slot metadata are
   // all requested before anything waits on memory
   cw v[8], uin[UIN];
-  int l0 = 0, l1 = (int)fa.chunk_line[1], s0 = 0, s1 = (int)fa.chunk_slot[1];
-  {
-    const bool valid = job < l1;
-    const size_t base = (size_t)(valid ? job : 0) * g.N + (size_t)n2 * L;
+  // (each by the wavefronts that use it only: see the products' C2)
+  int l0 = 0, l1 = fa.first_lines, s0 = 0, s1 = fa.first_slots;
+  LineTw<L, W> lt;
+  cw w4[8];
+  if (wave * (64 / T) < l1) {
+    const size_t base = (size_t)(job < l1 ? job : l1 - 1) * g.N + (size_t)n2 * L;
 #pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = valid ? conv[base + t + i * T] : cw{0, 0};
+    for (int i = 0; i < 8; i++) v[i] = conv[base + t + i * T];
+  }
 #pragma unroll
-    for (int r = 0; r < UIN; r++) {
-      const int e = tid + r * NT;
-      uin[r] = e < M * L ? U[(size_t)(e / L) * g.N + (size_t)n2 * L + e % L] : cw{0, 0};
-    }
+  for (int r = 0; r < UIN; r++) {
+    const int e = tid + r * NT;
+    if (wave * 64 + r * NT < M * L) uin[r] = U[(size_t)(e / L) * g.N + (size_t)n2 * L + e % L];
   }
   constexpr int QIN = kColStageQPreOf<M, W> / NT;
   W qin[QIN];
@@ -1070,15 +1453,15 @@ __global__ void __launch_bounds__(NW * 64, HI ? 3 : (MF ? (MfmaRows<M, PAR>::RT 
     qin[r] = e < (s1 - s0) * MM ? Qd[(size_t)s0 * MM + e] : (W)0;
   }
   if (tid < s1 - s0) min_ = fa.slot_meta[s0 + tid];
-  LineTw<L, W> lt;
-  load_line_tw<L>(lt, coltw, t);
-  cw w4[8];
+  if (wave * (64 / T) < (l1 > M ? l1 : M)) {
+    load_line_tw<L>(lt, coltw, t);
 #pragma unroll
-  for (int i = 0; i < 8; i++) w4[i] = fourtw[n2 * (t + i * T)];
+    for (int i = 0; i < 8; i++) w4[i] = fourtw[n2 * (t + i * T)];
+  }
 #pragma unroll
   for (int r = 0; r < UIN; r++) {
     const int e = tid + r * NT;
-    if (e < M * L) Ush[(e / L) * RS + e % L] = uin[r];
+    if (wave * 64 + r * NT < M * L) Ush[(e / L) * RS + e % L] = uin[r];
   }
   const W sc = (W)scale, kv = (W)fp.kv, kr = (W)fp.kr;
   cw u[MF ? 1 : M], acc[M];
@@ -1153,9 +1536,9 @@ __global__ void __launch_bounds__(NW * 64, HI ? 3 : (MF ? (MfmaRows<M, PAR>::RT 
       const bool valid = q < l1;
       if (r0 + wave * (64 / T) >= l1) continue;  // no line of this wavefront in the round
       if (c > 0 || r0 > l0) {
-        const size_t base = (size_t)(valid ? q : 0) * g.N + (size_t)n2 * L;
+        const size_t base = (size_t)(valid ? q : l1 - 1) * g.N + (size_t)n2 * L;
 #pragma unroll
-        for (int i = 0; i < 8; i++) v[i] = valid ? conv[base + t + i * T] : cw{0, 0};
+        for (int i = 0; i < 8; i++) v[i] = conv[base + t + i * T];
       }
 #pragma unroll
       for (int i = 0; i < 8; i++) v[i] = cmulc(v[i], w4[i]);
@@ -1716,7 +2099,7 @@ void colstage_pairs_plan(int M, int N2, int n_lines, int F, bool mixed, int& col
 
 template <class W>
 hipError_t launch_colstage_fields_pairs(const Geometry& g, const Twiddles& tw, const cpx<W>* yin, cpx<W>* U,
-                                        cpx<W>* conv, int n_lines, const PairLineArgs& pl, double scale,
+                                        cpx<W>* conv, const uint2* line_prod, int n_lines, double scale,
                                         const Batch& b, int F, int columns, int groups, int conv_cols, hipStream_t s) {
   if (g.N1 != kColStageL || g.M < 1 || g.M > kColStageMaxM || F < 1 || F > 65535 || n_lines < 1) return hipErrorInvalidValue;
   if (columns < 1 || g.N2 % columns || groups < 1 || groups > n_lines) return hipErrorInvalidValue;
@@ -1725,55 +2108,100 @@ hipError_t launch_colstage_fields_pairs(const Geometry& g, const Twiddles& tw, c
   const dim3 grid((unsigned)(g.N2 / columns * groups), F);
   switch (columns) {
     case 1: MMP_LAUNCH((k_colstage_fields_pairs<W, 1>), grid, dim3(256), lds, s, g, TwOf<W>::col(tw),
-                       TwOf<W>::four(tw), yin, U, conv, n_lines, pl, scale, b, groups, conv_cols); break;
+                       TwOf<W>::four(tw), yin, U, conv, n_lines, line_prod, scale, b, groups, conv_cols); break;
     case 2: MMP_LAUNCH((k_colstage_fields_pairs<W, 2>), grid, dim3(256), lds, s, g, TwOf<W>::col(tw),
-                       TwOf<W>::four(tw), yin, U, conv, n_lines, pl, scale, b, groups, conv_cols); break;
+                       TwOf<W>::four(tw), yin, U, conv, n_lines, line_prod, scale, b, groups, conv_cols); break;
     case 4: MMP_LAUNCH((k_colstage_fields_pairs<W, 4>), grid, dim3(256), lds, s, g, TwOf<W>::col(tw),
-                       TwOf<W>::four(tw), yin, U, conv, n_lines, pl, scale, b, groups, conv_cols); break;
+                       TwOf<W>::four(tw), yin, U, conv, n_lines, line_prod, scale, b, groups, conv_cols); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
 
-#define MMP_COLSTAGE_LAUNCH(MV, PARV)                                                                             \
-  if constexpr (kColStageMfma<MV, W, PARV>)                                                                       \
-    if (fa.waves == 4 && fa.matrix_cores) {                                                                       \
-      MMP_LAUNCH((k_colstage_raman_gather<MV, 4, W, PARV, false, true>), dim3(g.N2, F), dim3(256), 0, s, g,      \
-                 TwOf<W>::col(tw), TwOf<W>::four(tw), U, conv, yout, ga, fa, Qd, scale, b);                        \
-      break;                                                                                                      \
-    }                                                                                                             \
-  if constexpr (kColStageHiOcc<MV, W, PARV>)                                                                      \
-    if (fa.waves == 4 && fa.hi_occupancy) {                                                                       \
-      MMP_LAUNCH((k_colstage_raman_gather<MV, 4, W, PARV, true>), dim3(g.N2, F), dim3(256), 0, s, g,             \
-                 TwOf<W>::col(tw), TwOf<W>::four(tw), U, conv, yout, ga, fa, Qd, scale, b);                        \
-      break;                                                                                                      \
-    }                                                                                                             \
-  if constexpr (kColStageWide<MV, W>)                                                                             \
-    if (fa.waves == 8) {                                                                                          \
-      MMP_LAUNCH((k_colstage_raman_gather<MV, 8, W, PARV>), dim3(g.N2, F), dim3(512), 0, s, g, TwOf<W>::col(tw), \
-                 TwOf<W>::four(tw), U, conv, yout, ga, fa, Qd, scale, b);                                         \
-      break;                                                                                                      \
-    }                                                                                                             \
-  MMP_LAUNCH((k_colstage_raman_gather<MV, 4, W, PARV>), dim3(g.N2, F), dim3(256), 0, s, g, TwOf<W>::col(tw),     \
-             TwOf<W>::four(tw), U, conv, yout, ga, fa, Qd, scale, b);
-#define MMP_COLSTAGE_CASE(MV)                                                                                    \
-  case MV:                                                                                                        \
-    if (fa.parity) {                                                                                              \
-      MMP_COLSTAGE_LAUNCH(MV, true)                                                                               \
-    } else {                                                                                                      \
-      MMP_COLSTAGE_LAUNCH(MV, false)                                                                              \
-    }                                                                                                             \
-    break;
+// C2 in FP64, on the real products
+template <int M, int NW, int COLS, bool PAR>
+static hipError_t c2_launch(const Geometry& g, const Twiddles& tw, const cd* U, const cd* conv, cd* yout,
+                            const ProductArgs& fa, const double* Qp, double scale, const Batch& b, int F, hipStream_t s) {
+  const size_t lds = colstage_products_lds_bytes(M, COLS, fa.max_chunk_lines, fa.stride);
+  if (g.N2 % COLS || lds > kColStageLds) return hipErrorInvalidValue;
+  MMP_LAUNCH((k_colstage_products<M, NW, COLS, double, PAR>), dim3(g.N2 / COLS, F), dim3(NW * 64), lds, s, g, tw.coltw,
+             tw.fourtw, U, conv, yout, fa, Qp, scale, b);
+  return hipGetLastError();
+}
+template <int M, bool PAR>
+static hipError_t c2_variant(const Geometry& g, const Twiddles& tw, const cd* U, const cd* conv, cd* yout,
+                             const ProductArgs& fa, const double* Qp, double scale, const Batch& b, int F, hipStream_t s) {
+  if constexpr (M <= kColStageMaxM4) {
+    if (fa.cols == 4) return c2_launch<M, 4, 4, PAR>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
+  }
+  if constexpr (M <= kColStageMaxM2) {
+    if (fa.cols == 2) return c2_launch<M, 4, 2, PAR>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
+  }
+  if (fa.cols != 1) return hipErrorInvalidValue;
+  if constexpr (PAR && (M == 5 || M == 6)) {
+    if (fa.waves == 12) {
+      if (fa.n_chunks != 1) return hipErrorInvalidValue;
+      return c2_launch<M, 12, 1, PAR>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
+    }
+  }
+  if (fa.waves == 8 && M <= 4 && PAR && fa.n_chunks != 1) return hipErrorInvalidValue;
+  if (fa.waves == 8) return c2_launch<M, 8, 1, PAR>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
+  return c2_launch<M, 4, 1, PAR>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
+}
+#define MMP_PRODUCTS_CASE(MV)                                                                  \
+  case MV:                                                                                      \
+    return fa.parity ? c2_variant<MV, true>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s)       \
+                     : c2_variant<MV, false>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
+hipError_t launch_colstage_products(const Geometry& g, const Twiddles& tw, const cd* U, const cd* conv, cd* yout,
+                                    const ProductArgs& fa, const double* Qp, double scale, const Batch& b, int F,
+                                    hipStream_t s) {
+  if (g.N1 != kColStageL || F < 1 || F > 65535) return hipErrorInvalidValue;
+  if (fa.n_chunks < 1 || fa.max_chunk_lines < 1 || fa.max_chunk_lines > colstage_lines_per_chunk(g.M) ||
+      fa.first_lines > fa.max_chunk_lines || fa.n_products > 2 * fa.n_lines || fa.stride < 1 || fa.n_steps > fa.stride)
+    return hipErrorInvalidValue;
+  switch (g.M) {
+    MMP_PRODUCTS_CASE(1) MMP_PRODUCTS_CASE(2) MMP_PRODUCTS_CASE(3) MMP_PRODUCTS_CASE(4) MMP_PRODUCTS_CASE(5)
+    MMP_PRODUCTS_CASE(6) MMP_PRODUCTS_CASE(7) MMP_PRODUCTS_CASE(8) MMP_PRODUCTS_CASE(9) MMP_PRODUCTS_CASE(10)
+    MMP_PRODUCTS_CASE(11) MMP_PRODUCTS_CASE(12) MMP_PRODUCTS_CASE(13) MMP_PRODUCTS_CASE(14) MMP_PRODUCTS_CASE(15)
+    MMP_PRODUCTS_CASE(16)
+    default: return hipErrorInvalidValue;
+  }
+}
 
-template <class W>
-hipError_t launch_colstage_raman_gather(const Geometry& g, const Twiddles& tw, const cpx<W>* U, const cpx<W>* conv,
-                                        cpx<W>* yout, const GatherArgs& ga, const FusedArgs& fa, const W* Qd,
-                                        double scale, const Batch& b, int F, hipStream_t s) {
+// C2 in FP32, on the complex slots
+#define MMP_COLSTAGE_GO(MV, NWV, PARV, ...)                                                                        \
+  MMP_LAUNCH((k_colstage_raman_gather<MV, NWV, float, PARV __VA_ARGS__>), dim3(g.N2, F), dim3(NWV * 64), 0, s, g,  \
+             tw.coltw32, tw.fourtw32, U, conv, yout, fa, Qd, scale, b);                                            \
+  break;
+#define MMP_COLSTAGE_LAUNCH(MV, PARV)                                                                              \
+  if constexpr (kColStageMfma<MV, float, PARV>)                                                                    \
+    if (fa.waves == 4 && fa.matrix_cores) {                                                                        \
+      MMP_COLSTAGE_GO(MV, 4, PARV, , false, true)                                                                  \
+    }                                                                                                              \
+  if constexpr (kColStageHiOcc<MV, float, PARV>)                                                                   \
+    if (fa.waves == 4 && fa.hi_occupancy) {                                                                        \
+      MMP_COLSTAGE_GO(MV, 4, PARV, , true)                                                                         \
+    }                                                                                                              \
+  if constexpr (kColStageWide<MV, float>)                                                                          \
+    if (fa.waves == 8) {                                                                                           \
+      MMP_COLSTAGE_GO(MV, 8, PARV)                                                                                 \
+    }                                                                                                              \
+  MMP_COLSTAGE_GO(MV, 4, PARV)
+#define MMP_COLSTAGE_CASE(MV)                                                                                      \
+  case MV:                                                                                                         \
+    if (fa.parity) {                                                                                               \
+      MMP_COLSTAGE_LAUNCH(MV, true)                                                                                \
+    } else {                                                                                                       \
+      MMP_COLSTAGE_LAUNCH(MV, false)                                                                               \
+    }
+hipError_t launch_colstage_raman_gather(const Geometry& g, const Twiddles& tw, const cf* U, const cf* conv, cf* yout,
+                                        const SlotArgs& fa, const float* Qd, double scale, const Batch& b, int F,
+                                        hipStream_t s) {
   if (g.N1 != kColStageL || F < 1 || F > 65535) return hipErrorInvalidValue;
   const int block = fa.parity ? g.M * ((g.M + 1) / 2) : g.M * g.M;
   if (fa.n_chunks < 1 || fa.max_chunk_lines < 1 || fa.max_chunk_lines > colstage_lines_per_chunk(g.M) ||
       fa.max_chunk_slots < 1 || fa.max_chunk_slots > colstage_slots_per_chunk() ||
-      fa.max_chunk_slots * block > colstage_coefficients_per_chunk(g.M, std::is_same<W, float>::value))
+      fa.max_chunk_slots * block > colstage_coefficients_per_chunk(g.M, true))
     return hipErrorInvalidValue;
   switch (g.M) {
     MMP_COLSTAGE_CASE(1) MMP_COLSTAGE_CASE(2) MMP_COLSTAGE_CASE(3) MMP_COLSTAGE_CASE(4) MMP_COLSTAGE_CASE(5)
@@ -1878,11 +2306,8 @@ hipError_t launch_photon_number(const Geometry& g, const cd* spectra, double* ou
   template hipError_t launch_row_raman_cols<W>(const Geometry&, const Twiddles&, const cpx<W>*, cpx<W>*, int,         \
                                                const cpx<W>*, const Batch&, int, int, hipStream_t);                 \
   template hipError_t launch_colstage_fields_pairs<W>(const Geometry&, const Twiddles&, const cpx<W>*, cpx<W>*,     \
-                                                      cpx<W>*, int, const PairLineArgs&, double, const Batch&, int, \
-                                                      int, int, int, hipStream_t);                                 \
-  template hipError_t launch_colstage_raman_gather<W>(const Geometry&, const Twiddles&, const cpx<W>*,             \
-                                                      const cpx<W>*, cpx<W>*, const GatherArgs&, const FusedArgs&, \
-                                                      const W*, double, const Batch&, int, hipStream_t);
+                                                      cpx<W>*, const uint2*, int, double, const Batch&, int, int,  \
+                                                      int, int, hipStream_t);
 MMP_INSTANTIATE_W(double)
 MMP_INSTANTIATE_W(float)
 

@@ -125,6 +125,128 @@ static bool all_finite(const double* x, size_t n) {
   return true;
 }
 
+// Real products of the pair slots (setup.h), the Re products ordered by parity class, then the Im
+// products, and whether the Im products have a nonzero coefficient.
+static void plan_products(Problem& P) {
+  const uint32_t M = P.M, none = 0xffffffffu;
+  // the slots of each unordered pair: [0] (lo, hi) or a self pair, [1] (hi, lo)
+  std::vector<uint32_t> pair_slot((size_t)M * M * 2, none);
+  std::vector<uint32_t> pairs;  // lo * M + hi in slot order
+  for (uint32_t j = 0; j < P.P; j++) {
+    const uint32_t a = P.slot_a[j], b = P.slot_b[j], lo = std::min(a, b), hi = std::max(a, b), key = lo * M + hi;
+    if (pair_slot[2 * key] == none && pair_slot[2 * key + 1] == none) pairs.push_back(key);
+    pair_slot[2 * key + (a > b ? 1 : 0)] = j;
+  }
+  // parity classes of a pair's couplings: 1 even, 2 odd, 3 both (its slots differ); no structure: 1
+  auto classes = [&](uint32_t key) {
+    uint32_t c = 0;
+    for (int r = 0; r < 2; r++)
+      if (pair_slot[2 * key + r] != none) c |= 1u << (P.parity ? P.slot_parity[pair_slot[2 * key + r]] : 0);
+    return c;
+  };
+  P.slot_re.assign(P.P, none);
+  P.slot_im.assign(P.P, none);
+  P.prod_a.clear();
+  P.prod_b.clear();
+  P.prod_im.clear();
+  for (uint32_t im = 0; im < 2; im++) {
+    for (uint32_t c : {1u, 3u, 2u}) {
+      if (c == 1) P.seg_b[2 * im] = P.n_products();
+      if (c == 3) P.seg_b[2 * im + 1] = P.n_products();
+      for (uint32_t key : pairs) {
+        const uint32_t lo = key / M, hi = key % M;
+        if ((im && lo == hi) || classes(key) != c) continue;
+        for (int r = 0; r < 2; r++)
+          if (pair_slot[2 * key + r] != none) (im ? P.slot_im : P.slot_re)[pair_slot[2 * key + r]] = P.n_products();
+        P.prod_a.push_back(lo);
+        P.prod_b.push_back(hi);
+        P.prod_im.push_back(im);
+      }
+      if (c == 3) P.seg_e[2 * im] = P.n_products();
+    }
+    P.seg_e[2 * im + 1] = P.n_products();
+    if (!im) P.n_re = P.n_products();
+  }
+  // Q1 - Q2 of every cross pair: a slot alone in its pair, or with a partner of other values
+  P.need_im = false;
+  std::vector<double> d(M);
+  for (uint32_t p = 0; p < M && !P.need_im; p++) {
+    for (uint32_t key : pairs)
+      if (key / M != key % M) {
+        const uint32_t s0 = pair_slot[2 * key], s1 = pair_slot[2 * key + 1];
+        std::fill(d.begin(), d.end(), 0.);
+        for (int r = 0; r < 2; r++) {
+          const uint32_t s = r ? s1 : s0;
+          if (s == none) continue;
+          // the nonzeros of Q^(p) are sorted by slot
+          uint32_t e = (uint32_t)(std::lower_bound(P.slot.begin() + P.off[p], P.slot.begin() + P.off[p + 1], s) -
+                                  P.slot.begin());
+          for (; e < P.off[p + 1] && P.slot[e] == s; e++) d[P.k[e]] += r ? -P.q[e] : P.q[e];
+        }
+        for (uint32_t k = 0; k < M; k++) P.need_im = P.need_im || d[k] != 0.;
+        if (P.need_im) break;
+      }
+  }
+}
+
+std::vector<double> product_coefficients(const Problem& P) {
+  const uint32_t M = P.M, none = 0xffffffffu;
+  const size_t NX = P.n_products();
+  std::vector<double> q(M * NX * M, 0.);
+  for (uint32_t p = 0; p < M; p++)
+    for (uint32_t e = P.off[p]; e < P.off[p + 1]; e++) {
+      const uint32_t s = P.slot[e];
+      q[(p * NX + P.slot_re[s]) * M + P.k[e]] += P.q[e];
+      if (P.slot_im[s] != none) q[(p * NX + P.slot_im[s]) * M + P.k[e]] += P.slot_a[s] < P.slot_b[s] ? P.q[e] : -P.q[e];
+    }
+  return q;
+}
+
+uint32_t Problem::product_steps() const {
+  const uint32_t G = 16 / (uint32_t)colstage_coef_pad((int)M, parity);
+  uint32_t steps = 0;
+  for (int sg = 0; sg < 4; sg++)
+    if (seg_b[sg] < seg_e[sg]) steps += (seg_e[sg] + G - 1) / G - seg_b[sg] / G;
+  return steps;
+}
+
+std::vector<uint32_t> product_step_table(const Problem& P, bool im) {
+  const uint32_t G = 16 / (uint32_t)colstage_coef_pad((int)P.M, P.parity), n = P.active_products(im);
+  std::vector<uint32_t> out;
+  for (int c = 0; c < P.fused_chunks; c++)
+    for (uint32_t sg : {0u, 2u, 1u, 3u}) {
+      const uint32_t c1 = std::min(2 * P.fused_line[c + 1], n);
+      const uint32_t b = std::max(P.seg_b[sg], 2 * P.fused_line[c]), e = std::min(P.seg_e[sg], c1);
+      if (b >= e) continue;
+      for (uint32_t x = b / G * G; x < e; x += G) out.push_back(x | sg << 28 | (x + G >= e ? 1u << 31 : 0u));
+    }
+  // whether another step of the chunk follows
+  for (size_t i = 0; i + 1 < out.size(); i++) {
+    int c = 0;
+    while (2 * P.fused_line[c + 1] <= (out[i] & 0xffffu)) c++;
+    if ((out[i + 1] & 0xffffu) < 2 * P.fused_line[c + 1]) out[i] |= 1u << 30;
+  }
+  return out;
+}
+
+std::vector<double> product_blocks(const Problem& P, const std::vector<double>& q, const std::vector<uint32_t>& steps) {
+  const uint32_t M = P.M, pad = (uint32_t)colstage_coef_pad((int)M, P.parity), G = 16 / pad;
+  const uint32_t row = P.parity ? (M + 1) / 2 : M;
+  const size_t NX = P.n_products(), stride = P.product_steps();
+  std::vector<double> out(M * stride * 16, 0.);
+  for (size_t step = 0; step < steps.size(); step++) {
+    const uint32_t x0 = steps[step] & 0xffffu;
+    const int sg = (int)(steps[step] >> 28 & 3u);
+    for (uint32_t x = std::max(P.seg_b[sg], x0); x < std::min(P.seg_e[sg], x0 + G); x++)
+      for (uint32_t p = 0; p < M; p++)
+        for (uint32_t kk = 0; kk < row; kk++) {
+          const uint32_t k = product_k(P, p, sg, kk);
+          if (k < M) out[(p * stride + step) * 16 + (x - x0) * pad + kk] = q[(p * NX + x) * M + k];
+        }
+  }
+  return out;
+}
+
 mmp_status prepare_problem(const mmp_params* in, const mmp_options& opt, Problem& P, std::string& err) {
   if (!in) { err = "params is NULL"; return MMP_ERR_INVALID_ARGUMENT; }
   const uint32_t M = in->n_modes, nt = in->nt, nb = in->n_beta;
@@ -141,7 +263,6 @@ mmp_status prepare_problem(const mmp_params* in, const mmp_options& opt, Problem
   }
   if (in->n_steps == 0) { err = "n_steps must be >= 1"; return MMP_ERR_INVALID_ARGUMENT; }
   if (in->raman && !in->raman_response) { err = "raman_response is required with Raman on"; return MMP_ERR_INVALID_ARGUMENT; }
-  P.mixed = opt.precision == MMP_PRECISION_MIXED;
   if (opt.precision != MMP_PRECISION_FP64 && opt.precision != MMP_PRECISION_MIXED) {
     err = "unknown precision";
     return MMP_ERR_INVALID_ARGUMENT;
@@ -181,6 +302,7 @@ mmp_status prepare_problem(const mmp_params* in, const mmp_options& opt, Problem
   P.nnz = nnz;
   P.n_steps = in->n_steps;
   P.rk = make_tableau(in->method_order);
+  P.mixed = opt.precision == MMP_PRECISION_MIXED;
   P.raman = in->raman ? 1 : 0;
   P.fR = in->raman_proportion;
 
@@ -395,6 +517,7 @@ mmp_status prepare_problem(const mmp_params* in, const mmp_options& opt, Problem
     P.parity = ok;
     for (uint32_t j = 0; j < P.P; j++) P.slot_parity[j] = (uint8_t)(par[j] > 0 ? 1 : 0);
   }
+  plan_products(P);
   gather_plan((int)M, (int)P.P, P.gather_cap, P.gather_chunk);
   if (!P.gather_cap || P.gather_chunk <= 0) {
     err = "the Kerr gather tile does not fit (n_modes too large)";
@@ -412,7 +535,7 @@ mmp_status prepare_problem(const mmp_params* in, const mmp_options& opt, Problem
   }
   P.kv = P.raman ? 1 - P.fR : 1.;
   P.kr = P.raman ? P.fR * P.T0 : 0.;
-  plan_colstage_chunks(P, colstage_lines_per_chunk((int)M));
+  plan_colstage_chunks(P, colstage_lines_per_chunk((int)M), P.need_im);
   // a stage result N_j needs a stash slot when a stage i > j + 1 reads it
   P.stash_needed.assign(P.rk.s, 0);
   for (int i = 0; i < P.rk.s; i++)
@@ -421,20 +544,12 @@ mmp_status prepare_problem(const mmp_params* in, const mmp_options& opt, Problem
   return MMP_OK;
 }
 
-// Column-stage kernels (Raman on, N1 = 64, M <= 16, dense coupling blocks): Raman lines are
-// processed in chunks that respect the LDS limits on lines, slots and coupling blocks;
-// chunk c covers lines [fused_line[c], fused_line[c+1]) and slots [fused_slot[c], fused_slot[c+1]).
-bool plan_colstage_chunks(Problem& P, int max_lines) {
+// The mixed-precision chunks: lines with their slots, within the LDS limits on both and on the
+// coupling coefficients.
+static bool plan_slot_chunks(Problem& P, int max_lines) {
   const uint32_t M = P.M;
-  P.fused_chunks = 0;
-  P.fused_max_lines = 0;
-  P.fused_max_slots = 0;
-  P.fused_line.clear();
-  P.fused_slot.clear();
   const int nl = (int)P.line_a.size();
-  if (max_lines < 1 || max_lines > colstage_lines_per_chunk((int)M)) return false;
-  if (P.raman && P.N1 == 64 && (int)M <= colstage_max_modes() && nl > 0 &&
-      P.line_slot0.size() == (size_t)nl + 1 && P.line_slot0[0] == 0 && P.line_slot0[nl] == P.P) {
+  if (nl > 0 && P.line_slot0.size() == (size_t)nl + 1 && P.line_slot0[0] == 0 && P.line_slot0[nl] == P.P) {
     const int block = P.parity ? (int)(M * ((M + 1) / 2)) : (int)(M * M);  // coefficients per slot
     const int max_slots =
         std::min(colstage_slots_per_chunk(), colstage_coefficients_per_chunk((int)M, P.mixed) / block);
@@ -466,6 +581,31 @@ bool plan_colstage_chunks(Problem& P, int max_lines) {
     P.fused_max_lines = P.fused_max_slots = 0;
   }
   return false;
+}
+
+
+// Column-stage kernels (Raman on, N1 = 64, M <= 16): Raman lines are processed in chunks of at
+// most max_lines (their LDS rows); chunk c covers lines [fused_line[c], fused_line[c+1]). The
+// lines of the Re products alone are chunked as the first lines of all products are.
+bool plan_colstage_chunks(Problem& P, int max_lines, bool im) {
+  P.fused_chunks = 0;
+  P.fused_max_lines = 0;
+  P.fused_line.clear();
+  if (max_lines < 1 || max_lines > colstage_lines_per_chunk((int)P.M)) return false;
+  P.fused_max_slots = 0;
+  P.fused_slot.clear();
+  if (!P.raman || P.N1 != 64 || (int)P.M > colstage_max_modes()) return false;
+  if (P.mixed) return plan_slot_chunks(P, max_lines);
+  const int nl = (int)P.active_lines(im);
+  if (nl < 1) return false;
+  P.fused_line.push_back(0);
+  for (int l = 0; l < nl; l += max_lines) {
+    const int lines = std::min(max_lines, nl - l);
+    P.fused_line.push_back((uint32_t)(l + lines));
+    P.fused_max_lines = std::max(P.fused_max_lines, lines);
+  }
+  P.fused_chunks = (int)P.fused_line.size() - 1;
+  return true;
 }
 
 }  // namespace mmp

@@ -56,12 +56,31 @@ struct Problem {
   // half zeros in a fixed checkerboard
   bool parity = false;
   std::vector<uint8_t> slot_parity;  // [P]
-  // column-stage kernels: chunks of Raman lines (0 chunks: not eligible), their line and slot
-  // bounds, and the largest chunk's line and slot counts
-  bool mixed = false;  // FP32 work arrays (the column-stage LDS limits depend on it)
-  int fused_chunks = 0, fused_max_lines = 0, fused_max_slots = 0;
+  bool mixed = false;  // FP32 work arrays
+  // Real products of the FP64 gathers. A cross pair's slots X(a,b) and X(b,a) = conj X(a,b)
+  // (h_R is real) enter as (Q1 + Q2) Re X + i (Q1 - Q2) Im X, so the kernels work on real products:
+  // Re U_a conj(U_b) of every pair (a <= b), then Im U_a conj(U_b) of the cross pairs. Each complex
+  // Raman line carries two consecutive products as its real and imaginary parts. Where every coupling
+  // is symmetric in the pair (Q1 = Q2, overlap integrals of real mode profiles) the Im products
+  // drop out: the Re products' lines are a prefix of the list.
+  std::vector<uint32_t> prod_a, prod_b, prod_im;    // [n_products]
+  std::vector<uint32_t> slot_re, slot_im;           // [P] products of a slot (slot_im: none for self pairs)
+  uint32_t n_re = 0;                                // Re products (the first ones)
+  // Segments [b, e): Re products with couplings of even and of odd parity, Im products of even and
+  // of odd parity. A pair whose two slots differ in parity lies in both (the segments then overlap).
+  // Without the parity structure all products lie in the even segments.
+  uint32_t seg_b[4] = {0, 0, 0, 0}, seg_e[4] = {0, 0, 0, 0};
+  uint32_t seg_products() const { return seg_e[0] - seg_b[0] + seg_e[1] - seg_b[1] + seg_e[2] - seg_b[2] + seg_e[3] - seg_b[3]; }
+  bool need_im = false;                             // some Q1 - Q2 is not zero
+  // chunks of Raman lines (0 chunks: the column-stage kernels do not apply) and the largest chunk
+  int fused_chunks = 0, fused_max_lines = 0;
   std::vector<uint32_t> fused_line;                 // [fused_chunks + 1]
+  int fused_max_slots = 0;                          // mixed: slots of the chunks
   std::vector<uint32_t> fused_slot;                 // [fused_chunks + 1]
+  uint32_t n_products() const { return (uint32_t)prod_a.size(); }
+  uint32_t product_steps() const;                   // steps of the vector gather over all products
+  uint32_t active_products(bool im) const { return im ? n_products() : n_re; }
+  uint32_t active_lines(bool im) const { return (active_products(im) + 1) / 2; }
   // Kerr gather: nonzeros of each Q^(p) sorted by (slot, k), with per-chunk ranges
   std::vector<uint32_t> off, k, slot;  // [M+1], [nnz], [nnz]
   int gather_cap = 0, gather_chunk = 0, gather_chunks = 0;
@@ -79,9 +98,23 @@ mmp_status prepare_problem(const mmp_params* in, const mmp_options& opt, Problem
 // rows would exceed 1024 samples; false if NT is unsupported.
 bool split_length(uint32_t nt, uint32_t& n1, uint32_t& n2);
 
-// Chunks of Raman lines (at most max_lines each, within the column-stage LDS limits) for the
-// column-stage kernels: fills P.fused_*; false (and no chunks) when those kernels do not apply.
-bool plan_colstage_chunks(Problem& P, int max_lines);
+// Chunks of Raman lines (at most max_lines each) for the column-stage kernels: fills P.fused_*; false
+// (and no chunks) when those kernels do not apply. FP64: over the lines of the Re products or (im) of
+// all products. Mixed precision: over line_a/b/self, within the LDS limits on slots and coefficients.
+bool plan_colstage_chunks(Problem& P, int max_lines, bool im);
+
+// Coupling coefficients of the real products: Re products Q1 + Q2, Im products Q1 - Q2, as [p][x][k].
+std::vector<double> product_coefficients(const Problem& P);
+// Index k of coefficient kk of mode p in segment sg (>= P.M: none).
+inline uint32_t product_k(const Problem& P, uint32_t p, int sg, uint32_t kk) {
+  return P.parity ? 2 * kk + ((p + (uint32_t)sg) & 1u) : kk;
+}
+// Step descriptors (ProductArgs::steps) of the vector gather for the chunks of P.fused_line, over the
+// Re products or (im) all: chunk by chunk, the even parity class's segments, then the odd one's; a step takes the
+// 16 / colstage_coef_pad products from its first one on.
+std::vector<uint32_t> product_step_table(const Problem& P, bool im);
+// The coefficients in those steps, [p][step][16] (zeros for products outside the step's segment).
+std::vector<double> product_blocks(const Problem& P, const std::vector<double>& q, const std::vector<uint32_t>& steps);
 
 // Sets the calling thread's mmp_last_error() text and returns st.
 mmp_status record_error(mmp_status st, const std::string& msg);

@@ -11,6 +11,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/mmprop.h"
@@ -105,7 +106,10 @@ struct mmp_solver {
   std::vector<HeadArgs> heads;  // s + 1 entries
   GatherArgs gather{};
   PairLineArgs pairs{};
-  FusedArgs fused{};
+  // column-stage step: the FP64 products' arguments (n_lines, line_prod also serve the pair pass in mixed
+  // precision), the mixed-precision slots'
+  ProductArgs fused{};
+  SlotArgs slots{};
   bool use_fused = false;
   int chunk_lines = 0;       // column-stage gather: Raman lines per LDS chunk at most
   bool tuned = false;        // MMP_FLAG_AUTOTUNE chose fused.waves and chunk_lines
@@ -113,7 +117,13 @@ struct mmp_solver {
   int pair_groups = 1;
   int conv_cols = 0;         // the pair pass stores the Raman lines in column order (large grids)
   bool chain = false;        // the step close also issues the next step's stage-0 head
-  double* qdense = nullptr;  // [P][M][M] (or parity-compact) dense coupling blocks for the register gathers
+  // coupling blocks of the register gathers: the products' steps (FP64 column-stage step), or the slots'
+  // [P][M][M] (mixed column-stage step: parity-compact where they have the structure)
+  double* qdense = nullptr;
+  std::vector<uint32_t> step_table;  // the vector gather's steps, whose order the coupling blocks follow
+  bool loaded = false;       // every fiber's data is on the device
+  bool need_im = false;      // the column-stage step runs the Im products (a fiber's couplings need them)
+  uint32_t plan_id = 0;      // counts changes of the kernels' plan: graphs captured before are stale
   // work arrays of the step in the work precision (the FP64 buffers above in FP64 mode)
   bool mixed = false;
   size_t wbytes = 16;        // bytes per complex work value
@@ -151,6 +161,7 @@ struct mmp_group {
   std::vector<mmp_solver*> members;
   std::vector<hipStream_t> branches;   // distinct member streams other than ctx->stream
   std::vector<hipEvent_t> events;      // fork, then one join per branch, then one per branch for advance
+  std::vector<uint32_t> plan_ids;      // the members' plans that the graphs hold
   hipGraph_t graph = nullptr, graph1 = nullptr;
   hipGraphExec_t exec = nullptr, exec1 = nullptr;
 };
@@ -294,7 +305,7 @@ mmp_status enqueue_step_w(mmp_solver* s) {
   const double cb = sizeof(cw);  // bytes per complex work value
   const double cs = 16.0;        // bytes per complex FP64 state value
   const double MN = (double)P.M * P.N;
-  const double LN = (double)s->n_lines * P.N;
+  const double LN = (double)(s->use_fused ? s->fused.n_lines : s->n_lines) * P.N;
   const double invN = 1.0 / P.N;
   for (int i = 0; i <= P.rk.s; i++) {
     if (i > 0 || !s->chain) MMP_TRY(enqueue_head_w<W>(s, i));
@@ -302,15 +313,18 @@ mmp_status enqueue_step_w(mmp_solver* s) {
     const int F = (int)s->F;
     if (s->use_fused) {
       MMP_TRY(run_kernel(s, "col_fields_pairs", cb * (2 * MN + LN) * F, [&] {
-        return launch_colstage_fields_pairs<W>(g, s->tw, ybuf, U, conv, s->n_lines, s->pairs, invN, s->batch, F,
-                                               s->pair_columns, s->pair_groups, s->conv_cols, st);
+        return launch_colstage_fields_pairs<W>(g, s->tw, ybuf, U, conv, s->fused.line_prod, s->fused.n_lines, invN,
+                                               s->batch, F, s->pair_columns, std::min(s->pair_groups, s->fused.n_lines),
+                                               s->conv_cols, st);
       }));
       MMP_TRY(run_kernel(s, "row_raman", cb * (2 * LN + P.N) * F, [&] {
-        return launch_row_raman_cols<W>(g, s->tw, conv, convt, s->n_lines, hspec, s->batch, F, s->conv_cols, st);
+        return launch_row_raman_cols<W>(g, s->tw, conv, convt, s->fused.n_lines, hspec, s->batch, F, s->conv_cols, st);
       }));
       MMP_TRY(run_kernel(s, "col_raman_gather", cb * (2 * MN + LN) * F, [&] {
-        return launch_colstage_raman_gather<W>(g, s->tw, U, convt, ybuf, s->gather, s->fused, qdense, invN, s->batch,
-                                               F, st);
+        if constexpr (std::is_same<W, double>::value)
+          return launch_colstage_products(g, s->tw, U, convt, ybuf, s->fused, qdense, invN, s->batch, F, st);
+        else
+          return launch_colstage_raman_gather(g, s->tw, U, convt, ybuf, s->slots, qdense, invN, s->batch, F, st);
       }));
       continue;
     }
@@ -489,6 +503,14 @@ void release(mmp_solver* s) {
 // mixed-precision stage heads form E_u from Im L and the fiber's z where they use it.
 bool lawson_tables(bool mixed) { return !mixed; }
 
+// Coupling coefficients of one fiber: of the FP64 column-stage gather's products, or of the slots.
+size_t coupling_block_size(const Problem& P, bool fused) {
+  if (fused && !P.mixed) return (size_t)P.M * P.product_steps() * 16;
+  return (size_t)P.P * P.M * (fused && P.parity ? (P.M + 1) / 2 : P.M);
+}
+// Step descriptors of the products' gather, read 64 at a time.
+size_t step_table_size(const Problem& P) { return (P.product_steps() / 64 + 2) * 64; }
+
 // Device bytes create_impl allocates for F fibers of problem P (kept in step with its dalloc calls).
 size_t planned_device_bytes(const Problem& P, const mmp_options& opt, size_t F) {
   auto c = [](size_t n) { return n ? n : (size_t)1; };
@@ -507,12 +529,12 @@ size_t planned_device_bytes(const Problem& P, const mmp_options& opt, size_t F) 
     if (P.raman) b += 8 * (size_t)P.N * F;
   }
   if (P.fused_chunks > 0 && !(opt.flags & MMP_FLAG_SEPARATE_COLUMNS)) {
-    b += 4 * (2 * (P.line_a.size() + 1) + c(P.P));  // chunk bounds sized for the finest plan, slot metadata
+    // chunk bounds sized for the finest plan, the lines' products, the steps or the slots
+    b += 4 * (L + 1) + 8 * c(L) + 4 * (mixed ? L + 1 + c(P.P) : step_table_size(P));
     if (P.raman) b += (mixed ? 8 : 16) * c(L) * P.N * F;  // the Raman lines in column order
   }
   const bool fused = P.fused_chunks > 0 && !(opt.flags & MMP_FLAG_SEPARATE_COLUMNS);
-  const size_t block = (fused && P.parity) ? (size_t)P.M * ((P.M + 1) / 2) : (size_t)P.M * P.M;
-  if (fused || dense_gather_chunk((int)P.M) > 0) b += (mixed ? 4 : 8) * (size_t)P.P * block * F;
+  if (fused || dense_gather_chunk((int)P.M) > 0) b += (mixed ? 4 : 8) * coupling_block_size(P, fused) * F;
   return b;
 }
 
@@ -578,6 +600,89 @@ std::vector<double> dense_blocks(const Problem& P, bool compact) {
   return qc;
 }
 
+// Uploads fiber f's coupling blocks for the step's present plan (host copies: a synchronisation
+// follows before they go).
+mmp_status upload_couplings(mmp_solver* s, uint32_t f, const Problem& Pf) {
+  if (!s->qdense_w) return MMP_OK;
+  std::vector<double> qd;
+  std::vector<float> qd32;
+  const Batch& b = s->batch;
+  if (s->use_fused && !s->mixed) qd = product_blocks(Pf, product_coefficients(Pf), s->step_table);
+  else qd = dense_blocks(Pf, s->slots.parity != 0);
+  if (s->mixed) {
+    qd32.assign(qd.begin(), qd.end());
+    MMP_TRY(upload(s, static_cast<float*>(const_cast<void*>(s->qdense_w)) + f * b.sq, qd32.data(), qd32.size() * 4));
+  } else {
+    MMP_TRY(upload(s, s->qdense + f * b.sq, qd.data(), qd.size() * 8));
+  }
+  HIP_TRY(hipStreamSynchronize(s->ctx->stream), "hipStreamSynchronize");
+  return MMP_OK;
+}
+
+// The Raman lines and their chunks (at most max_lines each) of the column-stage step. FP64: the lines of
+// the Re products, or of all products where s->need_im, and the products' steps; mixed: the slots'.
+mmp_status install_lines(mmp_solver* s, int max_lines) {
+  Problem& P = s->P;
+  if (!plan_colstage_chunks(P, max_lines, s->need_im)) return fail(MMP_ERR_INVALID_ARGUMENT, "no chunk plan for these limits");
+  const uint32_t* d_line = s->mixed ? s->slots.chunk_line : s->fused.chunk_line;
+  MMP_TRY(upload(s, const_cast<uint32_t*>(d_line), P.fused_line.data(), P.fused_line.size() * 4));
+  HIP_TRY(hipStreamSynchronize(s->ctx->stream), "hipStreamSynchronize");  // P.fused_line is the staging copy
+  s->chunk_lines = max_lines;
+  if (s->mixed) {
+    SlotArgs& sa = s->slots;
+    MMP_TRY(upload(s, const_cast<uint32_t*>(sa.chunk_slot), P.fused_slot.data(), P.fused_slot.size() * 4));
+    HIP_TRY(hipStreamSynchronize(s->ctx->stream), "hipStreamSynchronize");
+    sa.n_chunks = P.fused_chunks;
+    sa.max_chunk_lines = P.fused_max_lines;
+    sa.max_chunk_slots = P.fused_max_slots;
+    sa.first_lines = (int)P.fused_line[1];
+    sa.first_slots = (int)P.fused_slot[1];
+    return MMP_OK;
+  }
+  ProductArgs& fa = s->fused;
+  fa.n_chunks = P.fused_chunks;
+  fa.max_chunk_lines = P.fused_max_lines;
+  fa.first_lines = (int)P.fused_line[1];
+  fa.n_lines = (int)P.active_lines(s->need_im);
+  fa.n_products = (int)P.active_products(s->need_im);
+  fa.stride = (int)P.product_steps();
+  std::vector<uint32_t> table = product_step_table(P, s->need_im);
+  fa.n_steps = (int)table.size();
+  fa.odd_step = 0;
+  while (fa.odd_step < fa.n_steps && !(table[fa.odd_step] >> 28 & 1u)) fa.odd_step++;
+  const bool changed = table != s->step_table;
+  s->step_table = table;
+  table.resize(step_table_size(P), 0u);
+  MMP_TRY(upload(s, const_cast<uint32_t*>(fa.steps), table.data(), table.size() * 4));
+  HIP_TRY(hipStreamSynchronize(s->ctx->stream), "hipStreamSynchronize");
+  // the coupling blocks follow the steps' order
+  if (changed && s->loaded)
+    for (uint32_t f = 0; f < s->F; f++) MMP_TRY(upload_couplings(s, f, s->fib[f]));
+  return MMP_OK;
+}
+
+// FP64: columns per gather workgroup for the solver's grid.
+int gather_cols(const mmp_solver* s) {
+  const int M = (int)s->P.M;
+  const long columns = (long)s->g.N2 * s->F;
+  for (int cols : {4, 2})
+    if (columns >= 1024 * cols && colstage_cols_ok(M, cols) &&
+        colstage_products_lds_bytes(M, cols, s->fused.max_chunk_lines, s->fused.stride) <= kColStageLds)
+      return cols;
+  return 1;
+}
+
+// FP64: wavefronts of the gather's workgroup. On grids that leave a CU one or two workgroups the vector
+// form takes eight (12 at 5 and 6 modes where the Im products double the sums): a wavefront per
+// mode, up to 4 modes (12: 6) one per mode and parity class. Larger grids hide the sums' latency with
+// other workgroups.
+int gather_waves(const mmp_solver* s) {
+  const int M = (int)s->P.M;
+  if (s->fused.cols > 1 || (long)s->g.N2 * s->F > 512) return 4;
+  if ((M == 5 || M == 6) && s->need_im && s->fused.parity && s->fused.n_chunks == 1) return 12;
+  return 8;
+}
+
 // Uploads fiber f's own data (operators, couplings, Raman spectrum, initial state, scalars),
 // resets its z and Lawson tables, then frees the large host arrays of its problem.
 mmp_status load_fiber(mmp_solver* s, uint32_t f, Problem& Pf) {
@@ -590,17 +695,7 @@ mmp_status load_fiber(mmp_solver* s, uint32_t f, Problem& Pf) {
     MMP_TRY(upload(s, s->etab0 + f * b.se, Pf.etab0.data(), Pf.etab0.size() * sizeof(double)));
     MMP_TRY(upload(s, s->etab + f * b.se, Pf.etab0.data(), Pf.etab0.size() * sizeof(double)));
   }
-  std::vector<double> qd;
-  std::vector<float> qd32;
-  if (s->qdense_w) {
-    qd = dense_blocks(Pf, s->fused.parity != 0);
-    if (s->mixed) {
-      qd32.assign(qd.begin(), qd.end());
-      MMP_TRY(upload(s, static_cast<float*>(const_cast<void*>(s->qdense_w)) + f * b.sq, qd32.data(), qd32.size() * 4));
-    } else {
-      MMP_TRY(upload(s, s->qdense + f * b.sq, qd.data(), qd.size() * 8));
-    }
-  }
+  MMP_TRY(upload_couplings(s, f, Pf));
   const FiberParams fp{Pf.delta_z, Pf.sign_gamma, Pf.delta_t, Pf.kv, Pf.kr, 1u, 0u};
   MMP_TRY(upload(s, s->d_fp + f, &fp, sizeof fp));
   // b_{i-1} h and a_ij h of every head, multiplied in FP64 on the host as the single solver does
@@ -705,8 +800,8 @@ mmp_status create_impl(mmp_ctx* ctx, uint32_t n_fibers, const mmp_params* params
   s->batch.se = s->ntab * MN;
   s->batch.ss = (size_t)P.rk.s * MN;
   const bool compact = s->use_fused && P.parity;
-  s->batch.sq = (size_t)P.P * P.M * (compact ? (P.M + 1) / 2 : P.M);
-  s->fused.parity = compact ? 1 : 0;
+  s->slots.parity = compact && s->mixed ? 1 : 0;
+  s->batch.sq = coupling_block_size(P, s->use_fused);
   s->batch.sh = P.N;
   // device buffers: per-fiber arrays are [F][...]; ybuf and U are also the FP64 scratch of
   // getResult, set_state and energy (their first M x NT values)
@@ -840,48 +935,80 @@ mmp_status create_impl(mmp_ctx* ctx, uint32_t n_fibers, const mmp_params* params
   s->batch.fp = s->d_fp;
   s->batch.coef = s->d_coef;
   s->batch.st = s->st;
-  std::vector<uint32_t> slot_meta(P.P);
+  std::vector<uint2> line_prod(s->mixed ? P.line_a.size() : (P.n_products() + 1) / 2);
+  std::vector<uint32_t> slot_meta(s->mixed ? P.P : 0);
   if (s->use_fused) {
-    uint32_t *d_cl, *d_cs, *d_meta;
-    const size_t max_chunks = P.line_a.size() + 1;  // room for the finest chunking the tuner may pick
-    A(dalloc(s, &d_cl, max_chunks));
-    A(dalloc(s, &d_cs, max_chunks));
-    A(dalloc(s, &d_meta, P1));
+    uint32_t* d_cl;
+    uint2* d_lp;
+    A(dalloc(s, &d_cl, L1 + 1));  // room for the finest chunking the tuner may pick
+    A(dalloc(s, &d_lp, L1));
     if (st != MMP_OK) return cleanup(st);
-    for (uint32_t j = 0; j < P.P; j++)
-      slot_meta[j] = P.slot_a[j] | (P.slot_b[j] << 8) | (P.slot_kind[j] << 16) | ((uint32_t)P.slot_parity[j] << 18) |
-                     (P.slot_line[j] << 19);
-    A(upload(s, d_cl, P.fused_line.data(), P.fused_line.size() * 4));
-    A(upload(s, d_cs, P.fused_slot.data(), P.fused_slot.size() * 4));
-    A(upload(s, d_meta, slot_meta.data(), P.P * 4));
-    // eight gather wavefronts from 4 to 6 modes (two per SIMD hide the slot loop's LDS latency);
-    // below 4 modes a column has at most 6 Raman lines and 9 slots, which four wavefronts cover
-    // (measured, 29 fibers of 3 modes at NT = 16384: 71 us with eight, 38 us with four)
-    s->fused = FusedArgs{d_cl,   d_cs, d_meta, P.fused_chunks, P.fused_max_lines, P.fused_max_slots, compact ? 1 : 0,
-                         P.M >= 4 && P.M <= 6 ? 8 : 4};
-    s->chunk_lines = colstage_lines_per_chunk((int)P.M);
-    colstage_pairs_plan((int)P.M, s->g.N2, s->n_lines, (int)s->F, s->mixed, s->pair_columns, s->pair_groups);
-    // grids of 8 or more workgroups per CU
-    s->fused.hi_occupancy = colstage_hi_occupancy_ok((int)P.M, s->mixed, compact) && (long)s->g.N2 * s->F >= 2048;
-    // the coupling sums on the matrix cores (FP32) by default at 4 to 10 and 13 to 16 modes,
-    // whatever the number of fibers (a batch runs the arithmetic of its fibers alone). Measured on
-    // one MI355X, gather per launch against the vector gather: 7-8 modes 1.03-1.23x (one 32-row
-    // tile, three workgroups per CU); 4-6 modes 1.06-1.31x on grids of 2048 workgroups and more,
-    // 0.84-0.90x on small ones (against the eight-wavefront vector gather); 9-10 modes 1.04-1.19x
-    // on the grids of one fiber or a few, 0.84-0.92x on large batches, where two tiles hold the
-    // matrix-core gather to two workgroups per CU against three for the vector gather (the tuner
-    // picks per batch); 11-12 modes 0.89-1.05x; 13-16 modes 1.03-1.25x on every grid (three or
-    // four tiles, the wavefront pairs splitting them).
-    {
-      const int M = (int)P.M;
+    auto product = [](uint32_t a, uint32_t b, uint32_t im) { return a | (b << 8) | (im << 16); };
+    const uint32_t absent = 1u << 17;
+    for (uint32_t l = 0; l < line_prod.size(); l++) {
+      if (s->mixed) {  // a cross pair's line, or two self pairs'
+        const uint32_t a = P.line_a[l], b = P.line_b[l];
+        line_prod[l] = P.line_self[l] ? make_uint2(product(a, a, 0), b != 0xffffffffu ? product(b, b, 0) : absent)
+                                      : make_uint2(product(a, b, 0), product(a, b, 1));
+      } else {
+        auto at = [&](uint32_t x) {
+          return x < P.n_products() ? product(P.prod_a[x], P.prod_b[x], P.prod_im[x]) : absent;
+        };
+        line_prod[l] = make_uint2(at(2 * l), at(2 * l + 1));
+      }
+    }
+    A(upload(s, d_lp, line_prod.data(), line_prod.size() * sizeof(uint2)));
+    s->fused.line_prod = d_lp;
+    s->fused.n_lines = (int)line_prod.size();
+    const int M = (int)P.M;
+    if (s->mixed) {
+      uint32_t *d_cs, *d_meta;
+      A(dalloc(s, &d_cs, L1 + 1));
+      A(dalloc(s, &d_meta, P1));
+      if (st != MMP_OK) return cleanup(st);
+      for (uint32_t j = 0; j < P.P; j++)
+        slot_meta[j] = P.slot_a[j] | (P.slot_b[j] << 8) | (P.slot_kind[j] << 16) | ((uint32_t)P.slot_parity[j] << 18) |
+                       (P.slot_line[j] << 19);
+      A(upload(s, d_meta, slot_meta.data(), P.P * 4));
+      s->slots.chunk_line = d_cl;
+      s->slots.chunk_slot = d_cs;
+      s->slots.slot_meta = d_meta;
+      if (st == MMP_OK) A(install_lines(s, colstage_lines_per_chunk(M)));
+      // eight gather wavefronts from 4 to 6 modes (two per SIMD hide the slot loop's LDS latency);
+      // below 4 modes a column has at most 6 Raman lines and 9 slots, which four wavefronts cover
+      // (measured, 29 fibers of 3 modes at NT = 16384: 71 us with eight, 38 us with four)
+      s->slots.waves = M >= 4 && M <= 6 ? 8 : 4;
+      // grids of 8 or more workgroups per CU
+      s->slots.hi_occupancy = colstage_hi_occupancy_ok(M, true, compact) && (long)s->g.N2 * s->F >= 2048;
+      // the coupling sums on the matrix cores (FP32) by default at 4 to 10 and 13 to 16 modes,
+      // whatever the number of fibers (a batch runs the arithmetic of its fibers alone). Measured on
+      // one MI355X, gather per launch against the vector gather: 7-8 modes 1.03-1.23x (one 32-row
+      // tile, three workgroups per CU); 4-6 modes 1.06-1.31x on grids of 2048 workgroups and more,
+      // 0.84-0.90x on small ones (against the eight-wavefront vector gather); 9-10 modes 1.04-1.19x
+      // on the grids of one fiber or a few, 0.84-0.92x on large batches, where two tiles hold the
+      // matrix-core gather to two workgroups per CU against three for the vector gather (the tuner
+      // picks per batch); 11-12 modes 0.89-1.05x; 13-16 modes 1.03-1.25x on every grid (three or
+      // four tiles, the wavefront pairs splitting them).
       const bool want = (opt.flags & MMP_FLAG_MATRIX_CORES) || (M >= 4 && M <= 10) || M >= 13;
-      s->fused.matrix_cores =
-          !(opt.flags & MMP_FLAG_NO_MATRIX_CORES) && want && colstage_matrix_cores_ok(M, s->mixed, compact) ? 1 : 0;
+      s->slots.matrix_cores =
+          !(opt.flags & MMP_FLAG_NO_MATRIX_CORES) && want && colstage_matrix_cores_ok(M, true, compact) ? 1 : 0;
+      if (s->slots.matrix_cores) {
+        s->slots.waves = 4;
+        s->slots.hi_occupancy = 0;
+      }
+    } else {
+      uint32_t* d_steps;
+      A(dalloc(s, &d_steps, step_table_size(P)));
+      if (st != MMP_OK) return cleanup(st);
+      s->fused.chunk_line = d_cl;
+      s->fused.steps = d_steps;
+      s->fused.parity = compact ? 1 : 0;
+      for (const Problem& Pf : s->fib) s->need_im = s->need_im || Pf.need_im;
+      if (st == MMP_OK) A(install_lines(s, colstage_lines_per_chunk(M)));
+      s->fused.cols = gather_cols(s);
+      s->fused.waves = gather_waves(s);
     }
-    if (s->fused.matrix_cores) {
-      s->fused.waves = 4;
-      s->fused.hi_occupancy = 0;
-    }
+    colstage_pairs_plan(M, s->g.N2, s->n_lines, (int)s->F, s->mixed, s->pair_columns, s->pair_groups);
     // lines in column order before the Raman row pass too: its LDS staging costs latency that
     // only large grids hide (measured: batched M = 10, NT = 16384 x 36 fibers row pass 140 ->
     // 111 us; one grin6 fiber 7.0 -> 7.6 us)
@@ -946,6 +1073,7 @@ mmp_status create_impl(mmp_ctx* ctx, uint32_t n_fibers, const mmp_params* params
     if (e != hipSuccess) A(hip_fail(e, "hipStreamSynchronize"));
   }
   for (uint32_t f = 0; f < F && st == MMP_OK; f++) A(load_fiber(s, f, s->fib[f]));
+  s->loaded = st == MMP_OK;
   if (st == MMP_OK && (opt.flags & MMP_FLAG_AUTOTUNE) && s->use_fused) A(autotune(s));
   if (st == MMP_OK) A(build_graph(s));
   if (st != MMP_OK) return cleanup(st);
@@ -959,25 +1087,37 @@ mmp_status create_impl(mmp_ctx* ctx, uint32_t n_fibers, const mmp_params* params
 // Raman lines travel in column order into their row pass. Only the gather variants change the
 // order of a sum (over the pair slots); the other choices leave every result bit-identical.
 struct ColPlan {
-  int waves, lines, hi, columns, groups, conv_cols, mf;
+  int waves, lines, hi, cols, columns, groups, conv_cols, mf;  // hi, mf: mixed precision; cols: FP64
   bool operator==(const ColPlan& o) const {
-    return waves == o.waves && lines == o.lines && hi == o.hi && columns == o.columns && groups == o.groups &&
-           conv_cols == o.conv_cols && mf == o.mf;
+    return waves == o.waves && lines == o.lines && hi == o.hi && cols == o.cols && columns == o.columns &&
+           groups == o.groups && conv_cols == o.conv_cols && mf == o.mf;
   }
 };
 
 ColPlan current_plan(const mmp_solver* s) {
-  return ColPlan{s->fused.waves, s->chunk_lines, s->fused.hi_occupancy, s->pair_columns, s->pair_groups,
-                 s->conv_cols, s->fused.matrix_cores};
+  if (s->mixed)
+    return ColPlan{s->slots.waves, s->chunk_lines, s->slots.hi_occupancy, 1, s->pair_columns, s->pair_groups,
+                   s->conv_cols, s->slots.matrix_cores};
+  return ColPlan{s->fused.waves, s->chunk_lines, 0, s->fused.cols, s->pair_columns, s->pair_groups, s->conv_cols, 0};
 }
 
 bool plan_valid(const mmp_solver* s, const ColPlan& c) {
   const int M = (int)s->P.M;
-  if (c.waves != 4 && !(c.waves == 8 && colstage_wide_ok(M, s->mixed))) return false;
-  if (c.hi && !(c.waves == 4 && colstage_hi_occupancy_ok(M, s->mixed, s->fused.parity != 0))) return false;
-  const bool mf_ok = colstage_matrix_cores_ok(M, s->mixed, s->fused.parity != 0);
-  if (c.mf && (c.waves != 4 || c.hi || (s->opt.flags & MMP_FLAG_NO_MATRIX_CORES) || !mf_ok)) return false;
-  if (!c.mf && mf_ok && (s->opt.flags & MMP_FLAG_MATRIX_CORES)) return false;
+  if (s->mixed) {
+    if (c.cols != 1 || (c.waves != 4 && !(c.waves == 8 && colstage_wide_ok(M)))) return false;
+    if (c.hi && !(c.waves == 4 && colstage_hi_occupancy_ok(M, true, s->slots.parity != 0))) return false;
+    const bool mf_ok = colstage_matrix_cores_ok(M, true, s->slots.parity != 0);
+    if (c.mf && (c.waves != 4 || c.hi || (s->opt.flags & MMP_FLAG_NO_MATRIX_CORES) || !mf_ok)) return false;
+    if (!c.mf && mf_ok && (s->opt.flags & MMP_FLAG_MATRIX_CORES)) return false;
+  } else {
+    // (a 12-wavefront plan is a default only; it needs its one chunk)
+    if (c.hi || c.mf) return false;
+    if (c.waves != 4 && !((c.waves == 8 || (c.waves == 12 && c == current_plan(s))) && c.cols == 1)) return false;
+    if (!colstage_cols_ok(M, c.cols) || s->g.N2 % c.cols ||
+        colstage_products_lds_bytes(M, c.cols, std::min(c.lines, s->fused.n_lines), s->fused.stride) > kColStageLds)
+      return false;
+    if (c.waves == 8 && M <= 4 && s->fused.parity && c.lines < s->fused.n_lines) return false;  // one chunk
+  }
   if (c.columns != 1 && c.columns != 2 && c.columns != 4) return false;
   if (s->g.N2 % c.columns || colstage_pairs_lds_bytes(M, c.columns, s->mixed) > kColStagePairsLds) return false;
   if (c.groups < 1 || c.groups > s->n_lines || (c.groups & (c.groups - 1))) return false;
@@ -988,21 +1128,19 @@ bool plan_valid(const mmp_solver* s, const ColPlan& c) {
 mmp_status apply_colstage_plan(mmp_solver* s, const ColPlan& c) {
   if (!s->use_fused) return fail(MMP_ERR_UNSUPPORTED, "no column-stage kernels in this solver");
   if (!plan_valid(s, c)) return fail(MMP_ERR_INVALID_ARGUMENT, "no such column-stage variant for this problem");
-  Problem& P = s->P;
-  if (!plan_colstage_chunks(P, c.lines)) return fail(MMP_ERR_INVALID_ARGUMENT, "no chunk plan for these limits");
-  MMP_TRY(upload(s, const_cast<uint32_t*>(s->fused.chunk_line), P.fused_line.data(), P.fused_line.size() * 4));
-  MMP_TRY(upload(s, const_cast<uint32_t*>(s->fused.chunk_slot), P.fused_slot.data(), P.fused_slot.size() * 4));
-  HIP_TRY(hipStreamSynchronize(s->ctx->stream), "hipStreamSynchronize");  // host staging copies
-  s->fused.n_chunks = P.fused_chunks;
-  s->fused.max_chunk_lines = P.fused_max_lines;
-  s->fused.max_chunk_slots = P.fused_max_slots;
-  s->fused.waves = c.waves;
-  s->fused.hi_occupancy = c.hi;
-  s->fused.matrix_cores = c.mf;
-  s->chunk_lines = c.lines;
+  MMP_TRY(install_lines(s, c.lines));
+  if (s->mixed) {
+    s->slots.waves = c.waves;
+    s->slots.hi_occupancy = c.hi;
+    s->slots.matrix_cores = c.mf;
+  } else {
+    s->fused.waves = c.waves;
+    s->fused.cols = c.cols;
+  }
   s->pair_columns = c.columns;
   s->pair_groups = c.groups;
   s->conv_cols = c.conv_cols;
+  s->plan_id++;
   drop_graph(s);
   return MMP_OK;
 }
@@ -1059,7 +1197,7 @@ mmp_status tune_passes(mmp_solver* s, hipEvent_t e0, hipEvent_t e1, ColPlan& bes
   for (int lines : {colstage_lines_per_chunk(M), 24, 16}) {
     if (lines > colstage_lines_per_chunk(M)) continue;
     Problem probe = P;
-    if (!plan_colstage_chunks(probe, lines)) continue;
+    if (!plan_colstage_chunks(probe, lines, s->need_im)) continue;
     if (std::find(seen.begin(), seen.end(), probe.fused_line) != seen.end()) continue;
     seen.push_back(probe.fused_line);
     lines_opts.push_back(lines);
@@ -1067,12 +1205,13 @@ mmp_status tune_passes(mmp_solver* s, hipEvent_t e0, hipEvent_t e1, ColPlan& bes
   const ColPlan base1 = best;
   for (int waves : {4, 8})
     for (int lines : lines_opts)
-      for (int hi : {0, 1})
-        for (int mf : {0, 1}) {
+      for (int v : {0, 1, 2}) {  // mixed: matrix cores, three workgroups per CU; FP64: two, four columns
+          const int mf = s->mixed && v == 1, hi = s->mixed && v == 2, cols = !s->mixed && v ? 2 * v : 1;
           ColPlan c = base1;
           c.waves = waves;
           c.lines = lines;
           c.hi = hi;
+          c.cols = cols;
           c.mf = mf;
           MMP_TRY(consider(c));
         }
@@ -1094,8 +1233,8 @@ mmp_status tune_passes(mmp_solver* s, hipEvent_t e0, hipEvent_t e1, ColPlan& bes
 
 mmp_status autotune(mmp_solver* s) {
   const Problem& P = s->P;
-  const TuneKey key{{P.M, P.N, (uint32_t)P.rk.s, P.P, (uint32_t)s->n_lines, (uint32_t)P.parity, s->mixed ? 1u : 0u,
-                     s->F}};
+  const TuneKey key{{P.M, P.N, (uint32_t)P.rk.s, P.P, (uint32_t)s->fused.n_lines, (uint32_t)P.parity,
+                     s->mixed ? 1u : 0u, s->F}};
   {
     std::lock_guard<std::mutex> lock(g_tune_mutex);
     auto it = g_tune_cache.find(key);
@@ -1218,8 +1357,8 @@ mmp_status capture_group(mmp_group* g, int steps, hipGraph_t* graph_out, hipGrap
   return MMP_OK;
 }
 
-void group_release(mmp_group* g) {
-  if (!g) return;
+// Waits for the group's stream (a replay may be in flight) and destroys its graphs.
+void drop_group_graphs(mmp_group* g) {
   if (g->ctx) {
     hipSetDevice(g->ctx->device);
     hipStreamSynchronize(g->ctx->stream);
@@ -1228,6 +1367,22 @@ void group_release(mmp_group* g) {
   if (g->graph) hipGraphDestroy(g->graph);
   if (g->exec1) hipGraphExecDestroy(g->exec1);
   if (g->graph1) hipGraphDestroy(g->graph1);
+  g->exec = g->exec1 = nullptr;
+  g->graph = g->graph1 = nullptr;
+}
+
+// The group's graphs over the members' present plans.
+mmp_status capture_group_graphs(mmp_group* g) {
+  MMP_TRY(capture_group(g, kGraphSteps, &g->graph, &g->exec));
+  MMP_TRY(capture_group(g, 1, &g->graph1, &g->exec1));
+  g->plan_ids.clear();
+  for (const mmp_solver* s : g->members) g->plan_ids.push_back(s->plan_id);
+  return MMP_OK;
+}
+
+void group_release(mmp_group* g) {
+  if (!g) return;
+  drop_group_graphs(g);
   for (hipEvent_t e : g->events) hipEventDestroy(e);
   delete g;
 }
@@ -1378,8 +1533,7 @@ mmp_status mmp_group_create(mmp_ctx* ctx, uint32_t n, mmp_solver* const* solvers
       if (e != hipSuccess) st = hip_fail(e, "hipEventCreate");
       else g->events.push_back(ev);
     }
-    if (st == MMP_OK) st = capture_group(g, kGraphSteps, &g->graph, &g->exec);
-    if (st == MMP_OK) st = capture_group(g, 1, &g->graph1, &g->exec1);
+    if (st == MMP_OK) st = capture_group_graphs(g);
     if (st != MMP_OK) {
       group_release(g);
       return st;
@@ -1395,6 +1549,14 @@ mmp_status mmp_group_advance(mmp_group* g, uint32_t n) {
   if (!g) return fail(MMP_ERR_INVALID_ARGUMENT, "group is NULL");
   HIP_TRY(hipSetDevice(g->ctx->device), "hipSetDevice");
   if (n == 0) return MMP_OK;
+  // a member whose plan changed since the capture (a loaded fiber that needs the Im products); after
+  // a capture that failed there are no graphs, and the next call tries again
+  bool stale = !g->exec || !g->exec1;
+  for (size_t i = 0; i < g->members.size(); i++) stale = stale || g->plan_ids[i] != g->members[i]->plan_id;
+  if (stale) {
+    drop_group_graphs(g);
+    MMP_TRY(capture_group_graphs(g));
+  }
   for (mmp_solver* s : g->members)
     if (s->chain) MMP_TRY(enqueue_head(s, 0));  // stage 0 of each member's first step, on its stream
   hipStream_t st = g->ctx->stream;
@@ -1558,6 +1720,15 @@ mmp_status mmp_fiber_load(mmp_solver* s, uint32_t f, const mmp_params* params) {
                                             "and pair structure");
     MMP_TRY(set_device(s));
     HIP_TRY(hipStreamSynchronize(s->ctx->stream), "hipStreamSynchronize");  // queued steps read the old fiber
+    if (s->use_fused && !s->mixed && Pf.need_im && !s->need_im) {
+      // the first fiber whose couplings need the Im products: the step takes their lines too (the other
+      // fibers' Im coefficients are zero, and their Re products' arithmetic stays the same)
+      s->need_im = true;
+      MMP_TRY(install_lines(s, s->chunk_lines));
+      s->plan_id++;
+      drop_graph(s);
+      MMP_TRY(build_graph(s));
+    }
     MMP_TRY(load_fiber(s, f, Pf));
     s->fib[f] = std::move(Pf);
     s->time_window[f] = params->time_window;
@@ -1653,15 +1824,16 @@ mmp_status mmp_fiber_info(mmp_solver* s, uint32_t f, mmp_info* o) {
   o->device_bytes = s->device_bytes;
   o->n_fibers = s->F;
   o->live = s->live[f];
-  o->gather_waves = s->use_fused ? (uint32_t)s->fused.waves : 0u;
+  const int waves = s->mixed ? s->slots.waves : s->fused.waves;
+  o->gather_waves = s->use_fused ? (uint32_t)waves : 0u;
   o->chunk_lines = s->use_fused ? (uint32_t)s->chunk_lines : 0u;
   o->tuned = s->tuned ? 1u : 0u;
   o->pair_columns = s->use_fused ? (uint32_t)s->pair_columns : 0u;
   o->pair_groups = s->use_fused ? (uint32_t)s->pair_groups : 0u;
   o->gather_hi_occupancy =
-      s->use_fused && s->fused.waves == 4 && s->fused.hi_occupancy && !s->fused.matrix_cores ? 1u : 0u;
-  o->gather_matrix_cores = s->use_fused && s->fused.waves == 4 && s->fused.matrix_cores ? 1u : 0u;
-  o->gather_chunks = s->use_fused ? (uint32_t)s->fused.n_chunks : 0u;
+      s->use_fused && s->slots.waves == 4 && s->slots.hi_occupancy && !s->slots.matrix_cores ? 1u : 0u;
+  o->gather_matrix_cores = s->use_fused && s->slots.waves == 4 && s->slots.matrix_cores ? 1u : 0u;
+  o->gather_chunks = s->use_fused ? (uint32_t)(s->mixed ? s->slots.n_chunks : s->fused.n_chunks) : 0u;
   o->halted = s->halted[f];
   return MMP_OK;
 }
