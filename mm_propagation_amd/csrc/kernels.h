@@ -159,12 +159,6 @@ struct GatherArgs {
 // LDS plan of the gather for M modes and P slots: capacity and slots per chunk (0 if none fits).
 void gather_plan(int M, int P, int& cap, int& chunk);
 
-struct PairLineArgs {
-  const uint32_t* line_a;  // [n_lines]
-  const uint32_t* line_b;  // [n_lines]; for self lines the second mode or 0xffffffff
-  const uint32_t* line_self;  // [n_lines] 1 = packed self pairs, 0 = cross pair a, b
-};
-
 // Column-stage kernels (one workgroup per column, Raman on, N1 = 64, M <= 16). A Raman line carries
 // two real products as its real and imaginary parts, each Re or Im of U_a conj(U_b); lines are
 // processed in chunks, chunk c covers lines [chunk_line[c], chunk_line[c+1]).
@@ -178,6 +172,7 @@ struct ProductArgs {
   int first_lines;             // chunk_line[1]
   int n_lines;                 // lines in use (those of the Re products, or of all)
   int n_products;              // products in use
+  int seg_b[4], seg_e[4];      // the segments' products (setup.h)
   const uint32_t* steps;       // first product | segment << 28 | another step of the chunk follows << 30 | last
                                // of its segment in the chunk << 31 of each step, padded to a multiple
                                // of 64 + 64
@@ -248,7 +243,7 @@ hipError_t launch_col_forward_real(const Geometry& g, const Twiddles& tw, const 
                                    hipStream_t s);
 template <class W>
 hipError_t launch_col_pairs_forward(const Geometry& g, const Twiddles& tw, const cpx<W>* U, cpx<W>* out, int lines,
-                                    const PairLineArgs& pl, hipStream_t s);
+                                    const uint2* line_prod, hipStream_t s);
 hipError_t launch_row_forward(const Geometry& g, const Twiddles& tw, cd* data, int lines, hipStream_t s);
 hipError_t launch_row_inverse_phase(const Geometry& g, const Twiddles& tw, const cd* in, cd* out,
                                     const double* imL, const StepState* st, int use_phase, hipStream_t s);
@@ -264,6 +259,12 @@ hipError_t launch_row_raman_cols(const Geometry& g, const Twiddles& tw, const cp
 template <class W>
 hipError_t launch_gather(const Geometry& g, const cpx<W>* U, const cpx<W>* VR, cpx<W>* sigma, const GatherArgs& a,
                          hipStream_t s);
+// The separate passes' FP64 gather on the real products: modes it takes, and the Raman lines of one
+// LDS chunk at most. raman: VR holds the lines' convolutions (row order).
+bool gather_products_ok(int M, bool parity);
+int gather_products_lines(int M, bool parity);
+hipError_t launch_gather_products(const Geometry& g, const cd* U, const cd* VR, cd* sigma, const ProductArgs& fa,
+                                  const double* Qp, const Batch& b, int raman, hipStream_t s);
 // C1 takes `columns` (1, 2 or 4) neighbouring columns per workgroup and deals each column
 // block's Raman lines to `groups` workgroups; the LDS it then needs is
 // colstage_pairs_lds_bytes, at most kColStagePairsLds. Results do not depend on either.
@@ -280,7 +281,7 @@ hipError_t launch_colstage_products(const Geometry& g, const Twiddles& tw, const
 hipError_t launch_colstage_raman_gather(const Geometry& g, const Twiddles& tw, const cf* U, const cf* conv, cf* yout,
                                         const SlotArgs& fa, const float* Qd, double scale, const Batch& b, int F,
                                         hipStream_t s);
-// Dense-block gather (M <= 16): Qd is [P][M][M] with Qd[s][p][k] = sum of Q/max|Q| over the
+// Dense-block gather (FP32, M <= 16): Qd is [P][M][M] with Qd[s][p][k] = sum of Q/max|Q| over the
 // nonzeros (k, slot s) of Q^(p). dense_gather_chunk(M) is 0 when M is out of range.
 int dense_gather_chunk(int M);
 template <class W>

@@ -371,12 +371,12 @@ __global__ void __launch_bounds__(256) k_col_forward_real(Geometry g, const cd* 
   }
 }
 
-// pair products of the time-domain fields U, then forward column DFT
+// pair products of the time-domain fields U (two real products a line), then forward column DFT
 template <int L, int CB, class W>
 __global__ void __launch_bounds__(256) k_col_pairs_forward(Geometry g, const cpx<W>* __restrict__ coltw,
                                                            const cpx<W>* __restrict__ fourtw,
                                                            const cpx<W>* __restrict__ U, cpx<W>* __restrict__ out,
-                                                           int lines, PairLineArgs pl) {
+                                                           int lines, const uint2* __restrict__ line_prod) {
   using C = ColCfg<L, CB>;
   using cw = cpx<W>;
   __shared__ cw smem[C::G * C::SLOTS * CB];
@@ -385,7 +385,13 @@ __global__ void __launch_bounds__(256) k_col_pairs_forward(Geometry g, const cpx
   const int n2 = ix.cb * CB + ix.c;
   const bool valid = q < lines;
   const int qq = valid ? q : 0;
-  const uint32_t la = pl.line_a[qq], lb = pl.line_b[qq], self = pl.line_self[qq];
+  const uint2 d = line_prod[qq];
+  const cw* const a0 = U + (size_t)(d.x & 255u) * g.N;
+  const cw* const b0 = U + (size_t)((d.x >> 8) & 255u) * g.N;
+  const cw* const a1 = U + (size_t)(d.y & 255u) * g.N;
+  const cw* const b1 = U + (size_t)((d.y >> 8) & 255u) * g.N;
+  const bool im0 = (d.x >> 16) & 1u, im1 = (d.y >> 16) & 1u, has1 = !((d.y >> 17) & 1u);
+  const bool same = !((d.x ^ d.y) & 0xffffu);  // both parts of one pair's product
   cw* sm = smem + ix.gl * C::SLOTS * CB + ix.c;
   LineTw<L, W> lt;
   load_line_tw<L>(lt, coltw, ix.t);
@@ -396,16 +402,10 @@ __global__ void __launch_bounds__(256) k_col_pairs_forward(Geometry g, const cpx
     const size_t tt = (size_t)n1 * g.N2 + n2;
     cw x = {0, 0};
     if (valid) {
-      const cw ua = U[(size_t)la * g.N + tt];
-      if (self) {
-        x.re = ua.re * ua.re + ua.im * ua.im;
-        if (lb != 0xffffffffu) {
-          const cw ub = U[(size_t)lb * g.N + tt];
-          x.im = ub.re * ub.re + ub.im * ub.im;
-        }
-      } else {
-        x = cmulc(ua, U[(size_t)lb * g.N + tt]);
-      }
+      const cw x0 = cmulc(a0[tt], b0[tt]);
+      cw x1 = x0;
+      if (has1 && !same) x1 = cmulc(a1[tt], b1[tt]);
+      x = {im0 ? x0.im : x0.re, has1 ? (im1 ? x1.im : x1.re) : (W)0};
     }
     v[i] = x;
     w4[i] = fourtw[n2 * n1];
@@ -1342,6 +1342,136 @@ __global__ void __launch_bounds__(NW * 64) k_colstage_products(
 }
 
 // ---------------------------------------------------------------------------
+// The separate column passes' gather in FP64, on the same real products: a workgroup takes a tile of
+// 64 samples (lane = sample) and a group of modes, a wavefront per mode; the chunk's X rows are mixed by
+// whole wavefronts, then each wavefront sums its mode, segment by segment (the steps of a segment take
+// consecutive products, so no step table is read).
+// ---------------------------------------------------------------------------
+// More groups of modes give more wavefronts, and each group mixes the tile's X rows again: groups of at most
+// eight. LDS holds the field rows and as many lines' X rows as 64 KB take; a chunk's Raman rows are requested
+// before the sums of the chunk before. Bound by latency (a chain of steps whose coefficients come from
+// the L2). Whole step on one MI355X against the sparse sum (one slot entry after the other, up to 20 modes 708 us a
+// launch, now 25) or the dense slot blocks: 20 modes, NT = 4096 2995 -> 251 us; 6 modes, NT = 16384
+// without Raman 93.0 -> 78.7 us; 2 modes, NT = 1024 113.0 -> 107.6 us. Of it at 20 modes: step table as in
+// C2 336 us, steps by segment 272, loads kept in place 260, Raman rows ahead 251.
+constexpr int kProductsTS = 64, kProductsMaxWaves = 8;
+// (16 coefficients of a product and mode fill the register; field rows beyond 32 leave the chunks few lines)
+bool gather_products_ok(int M, bool parity) { return M >= 1 && M <= 32 && (parity ? (M + 1) / 2 : M) <= 16; }
+static int products_field_rows(int M, bool parity) { return parity ? M + (M & 1) : M; }
+int gather_products_lines(int M, bool parity) {
+  return ((int)(kColStageLds / (kProductsTS * sizeof(cd))) - products_field_rows(M, parity)) & ~1;
+}
+
+// One segment's part of a chunk for mode p: B[kk] = sum over the products [x, x + G ns) of this lane's sample
+// (xs: that of product x, rows of TS) and the coefficients from step `step` on, PD steps ahead in PD fixed
+// registers; the steps past the last one read any valid place.
+template <int QROW, int PD, int TS>
+__device__ __forceinline__ void segment_products(double (&B)[QROW], const double* __restrict__ q, int step, int last_step,
+                                                 const double* xs, int ns, int lane) {
+  constexpr int QP = coef_pad(QROW), G = 16 / QP;
+  double cq[PD], xv[PD][G];
+  auto load = [&](int s, int u) {
+    const int sq = step + s < last_step ? step + s : last_step, sx = s < ns ? s : ns - 1;
+    cq[u] = (q + (size_t)sq * 16)[lane & 15];
+#pragma unroll
+    for (int i = 0; i < G; i++) xv[u][i] = xs[(sx * G + i) * TS];
+  };
+#pragma unroll
+  for (int u = 0; u < PD; u++) load(u, u);
+#pragma unroll
+  for (int kk = 0; kk < QROW; kk++) B[kk] = 0.;
+  int s = 0;
+#pragma unroll 1
+  for (; s + PD <= ns; s += PD) {
+#pragma unroll
+    for (int u = 0; u < PD; u++) {
+      group_fmac<QROW, QP>(B, cq[u], xv[u]);
+      load(s + PD + u, u);
+      __builtin_amdgcn_sched_barrier(0);  // (else all PD loads end up behind the last step, each round a latency)
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < PD - 1; u++)
+    if (s + u < ns) group_fmac<QROW, QP>(B, cq[u], xv[u]);
+}
+
+template <int QROW, bool PAR>
+__global__ void __launch_bounds__(kProductsMaxWaves * 64) k_gather_products(
+    Geometry g, const cd* __restrict__ U, const cd* __restrict__ VR, cd* __restrict__ sigma, ProductArgs fa,
+    const double* __restrict__ Qp, Batch b, int raman, int field_rows) {
+  constexpr int TS = kProductsTS, PD = 8, R = 8, G = 16 / coef_pad(QROW);
+  extern __shared__ __align__(16) unsigned char gp_lds[];
+  cd* const Ush = reinterpret_cast<cd*>(gp_lds);                       // [field_rows][TS], zeros beyond M
+  double* const Xsh = reinterpret_cast<double*>(Ush + field_rows * TS);  // [2 lines of a chunk][TS]
+  const int M = g.M;
+  const int t0 = blockIdx.x * TS;
+  const int tid = threadIdx.x, lane = tid % TS, waves = blockDim.x / TS;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / TS);
+  const int p = blockIdx.y * waves + wave;  // this wavefront's mode
+  const double kv = b.fp[0].kv, kr = raman ? b.fp[0].kr : 0.;
+  const double* const q = Qp + (size_t)(p < M ? p : 0) * fa.stride * 16;
+  // a chunk's first Raman rows of this wavefront are requested before the sums of the chunk before
+  cd vr[R];
+  uint2 d[R];
+  auto request = [&](int l, int l1) {
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+      const int r = l + i * waves < l1 ? l + i * waves : l1 - 1;
+      d[i] = fa.line_prod[r];
+      vr[i] = raman ? VR[(size_t)r * g.N + t0 + lane] : cd{0, 0};
+    }
+  };
+  request(wave, (int)fa.chunk_line[1]);
+#pragma unroll 4
+  for (int r = wave; r < field_rows; r += waves)
+    Ush[r * TS + lane] = r < M ? U[(size_t)r * g.N + t0 + lane] : cd{0, 0};
+  cd acc = {0, 0}, acc2 = {0, 0};  // sums of the even and of the odd parity class
+  int step = 0;
+  for (int ch = 0; ch < fa.n_chunks; ch++) {
+    const int l0 = (int)fa.chunk_line[ch], l1 = (int)fa.chunk_line[ch + 1];
+    __syncthreads();  // the fields' rows / X rows of the previous chunk consumed
+    // (a step of four products may read the row after the chunk's last one, times zero)
+    const int lend = l0 + (l1 - l0 + 1) / 2 * 2;
+#pragma unroll 1
+    for (int l = l0 + wave; l < lend; l += R * waves) {
+      if (l > l0 + wave) request(l, l1);
+#pragma unroll
+      for (int i = 0; i < R; i++) {
+        if (l + i * waves >= lend) break;
+        const cd V0 = cmulc(Ush[(d[i].x & 255u) * TS + lane], Ush[((d[i].x >> 8) & 255u) * TS + lane]);
+        const cd V1 = cmulc(Ush[(d[i].y & 255u) * TS + lane], Ush[((d[i].y >> 8) & 255u) * TS + lane]);
+        double* x0 = Xsh + (l + i * waves - l0) * 2 * TS + lane;
+        x0[0] = kv * ((d[i].x >> 16) & 1u ? V0.im : V0.re) + kr * vr[i].re;
+        x0[TS] = kv * ((d[i].y >> 16) & 1u ? V1.im : V1.re) + kr * vr[i].im;
+      }
+    }
+    if (ch + 1 < fa.n_chunks) request(l1 + wave, (int)fa.chunk_line[ch + 2]);
+    __syncthreads();
+    if (p < M) {
+      const int xc0 = 2 * l0, xc1 = 2 * l1 < fa.n_products ? 2 * l1 : fa.n_products;  // products of the chunk
+#pragma unroll
+      for (int j = 0; j < (PAR ? 4 : 2); j++) {  // segments in the order of their steps
+        const int sg = PAR ? (j == 1 ? 2 : (j == 2 ? 1 : j)) : 2 * j;
+        const int xb = fa.seg_b[sg] > xc0 ? fa.seg_b[sg] : xc0, xe = fa.seg_e[sg] < xc1 ? fa.seg_e[sg] : xc1;
+        if (xb >= xe) continue;
+        const int x = xb / G * G, ns = (xe - x + G - 1) / G;
+        double B[QROW];
+        segment_products<QROW, PD, TS>(B, q, step, fa.stride - 1, Xsh + (x - xc0) * TS + lane, ns, lane);
+        step += ns;
+        const cd* const Uc = Ush + (PAR ? (p + sg) & 1 : 0) * TS + lane;
+        cd sum = {0, 0};
+#pragma unroll
+        for (int kk = 0; kk < QROW; kk++) sum = cadd(sum, cscale(Uc[(PAR ? 2 * kk : kk) * TS], B[kk]));
+        if (sg >= 2) sum = {-sum.im, sum.re};
+        cd& a = sg & 1 ? acc2 : acc;
+        a = cadd(a, sum);
+      }
+    }
+  }
+  if (p < M) sigma[(size_t)p * g.N + t0 + lane] = PAR ? cadd(acc, acc2) : acc;
+}
+
+// ---------------------------------------------------------------------------
 // C2 in FP32 (mixed precision): complex slots X_s and complex Raman lines
 // ---------------------------------------------------------------------------
 // 4-wavefront FP32 gathers of 7 to 10 modes also come in a variant held to 168 VGPRs, so
@@ -1998,13 +2128,13 @@ hipError_t launch_col_forward_real(const Geometry& g, const Twiddles& tw, const 
 
 template <int L, class W>
 static hipError_t col_pairs_forward_impl(const Geometry& g, const Twiddles& tw, const cpx<W>* U, cpx<W>* out,
-                                         int lines, const PairLineArgs& pl, hipStream_t s) {
-  MMP_COL_LAUNCH(k_col_pairs_forward, lines, g, TwOf<W>::col(tw), TwOf<W>::four(tw), U, out, lines, pl)
+                                         int lines, const uint2* line_prod, hipStream_t s) {
+  MMP_COL_LAUNCH(k_col_pairs_forward, lines, g, TwOf<W>::col(tw), TwOf<W>::four(tw), U, out, lines, line_prod)
 }
 template <class W>
 hipError_t launch_col_pairs_forward(const Geometry& g, const Twiddles& tw, const cpx<W>* U, cpx<W>* out, int lines,
-                                    const PairLineArgs& pl, hipStream_t s) {
-  MMP_DISPATCH_COL_LW(g.N1, col_pairs_forward_impl, W, g, tw, U, out, lines, pl, s);
+                                    const uint2* line_prod, hipStream_t s) {
+  MMP_DISPATCH_COL_LW(g.N1, col_pairs_forward_impl, W, g, tw, U, out, lines, line_prod, s);
 }
 
 template <int L>
@@ -2076,6 +2206,37 @@ hipError_t launch_gather(const Geometry& g, const cpx<W>* U, const cpx<W>* VR, c
   else if (a.cap == 8192) MMP_LAUNCH((k_gather<8192, W>), grid, block, 0, s, g, U, VR, sigma, a);
   else return hipErrorInvalidValue;
   return hipGetLastError();
+}
+
+template <int QROW, bool PAR>
+static hipError_t gather_products_impl(const Geometry& g, const cd* U, const cd* VR, cd* sigma, const ProductArgs& fa,
+                                       const double* Qp, const Batch& b, int raman, hipStream_t s) {
+  const int rows = products_field_rows(g.M, PAR);
+  const size_t lds = (size_t)(rows + (fa.max_chunk_lines + 1) / 2 * 2) * kProductsTS * sizeof(cd);
+  if (lds > kColStageLds) return hipErrorInvalidValue;
+  const int groups = (g.M + kProductsMaxWaves - 1) / kProductsMaxWaves;
+  int waves = (g.M + groups - 1) / groups;
+  if (waves < 4) waves = 4;  // (the X rows are mixed by all)
+  MMP_LAUNCH((k_gather_products<QROW, PAR>), dim3(g.N / kProductsTS, groups), dim3(waves * 64), lds, s, g, U, VR, sigma, fa,
+             Qp, b, raman, rows);
+  return hipGetLastError();
+}
+#define MMP_GATHER_PRODUCTS_CASE(QV)                                                                    \
+  case QV:                                                                                              \
+    return fa.parity ? gather_products_impl<QV, true>(g, U, VR, sigma, fa, Qp, b, raman, s)             \
+                     : gather_products_impl<QV, false>(g, U, VR, sigma, fa, Qp, b, raman, s);
+hipError_t launch_gather_products(const Geometry& g, const cd* U, const cd* VR, cd* sigma, const ProductArgs& fa,
+                                  const double* Qp, const Batch& b, int raman, hipStream_t s) {
+  if (g.N % kProductsTS || !gather_products_ok(g.M, fa.parity) || fa.n_chunks < 1 || fa.max_chunk_lines < 1 ||
+      fa.n_products > 2 * fa.n_lines || fa.n_steps < 1 || fa.n_steps > fa.stride || (raman && !VR))
+    return hipErrorInvalidValue;
+  switch (fa.parity ? (g.M + 1) / 2 : g.M) {
+    MMP_GATHER_PRODUCTS_CASE(1) MMP_GATHER_PRODUCTS_CASE(2) MMP_GATHER_PRODUCTS_CASE(3) MMP_GATHER_PRODUCTS_CASE(4)
+    MMP_GATHER_PRODUCTS_CASE(5) MMP_GATHER_PRODUCTS_CASE(6) MMP_GATHER_PRODUCTS_CASE(7) MMP_GATHER_PRODUCTS_CASE(8)
+    MMP_GATHER_PRODUCTS_CASE(9) MMP_GATHER_PRODUCTS_CASE(10) MMP_GATHER_PRODUCTS_CASE(11) MMP_GATHER_PRODUCTS_CASE(12)
+    MMP_GATHER_PRODUCTS_CASE(13) MMP_GATHER_PRODUCTS_CASE(14) MMP_GATHER_PRODUCTS_CASE(15) MMP_GATHER_PRODUCTS_CASE(16)
+    default: return hipErrorInvalidValue;
+  }
 }
 
 size_t colstage_pairs_lds_bytes(int M, int columns, bool mixed) {
@@ -2296,19 +2457,19 @@ hipError_t launch_photon_number(const Geometry& g, const cd* spectra, double* ou
   template hipError_t launch_col_forward<W>(const Geometry&, const Twiddles&, const cpx<W>*, cpx<W>*, int,         \
                                             hipStream_t);                                                         \
   template hipError_t launch_col_pairs_forward<W>(const Geometry&, const Twiddles&, const cpx<W>*, cpx<W>*, int,   \
-                                                  const PairLineArgs&, hipStream_t);                              \
+                                                  const uint2*, hipStream_t);                                     \
   template hipError_t launch_row_raman<W>(const Geometry&, const Twiddles&, cpx<W>*, int, const cpx<W>*,           \
                                           const Batch&, int, hipStream_t);                                         \
   template hipError_t launch_gather<W>(const Geometry&, const cpx<W>*, const cpx<W>*, cpx<W>*, const GatherArgs&,  \
                                        hipStream_t);                                                              \
-  template hipError_t launch_gather_dense<W>(const Geometry&, const cpx<W>*, const cpx<W>*, cpx<W>*,               \
-                                             const GatherArgs&, const W*, hipStream_t);                            \
   template hipError_t launch_row_raman_cols<W>(const Geometry&, const Twiddles&, const cpx<W>*, cpx<W>*, int,         \
                                                const cpx<W>*, const Batch&, int, int, hipStream_t);                 \
   template hipError_t launch_colstage_fields_pairs<W>(const Geometry&, const Twiddles&, const cpx<W>*, cpx<W>*,     \
                                                       cpx<W>*, const uint2*, int, double, const Batch&, int, int,  \
                                                       int, int, hipStream_t);
 MMP_INSTANTIATE_W(double)
+template hipError_t launch_gather_dense<float>(const Geometry&, const cf*, const cf*, cf*, const GatherArgs&, const float*,
+                                               hipStream_t);
 MMP_INSTANTIATE_W(float)
 
 }  // namespace mmp

@@ -583,6 +583,17 @@ static bool plan_slot_chunks(Problem& P, int max_lines) {
   return false;
 }
 
+void plan_product_chunks(Problem& P, int max_lines, bool im) {
+  const int nl = (int)P.active_lines(im);
+  P.fused_line.assign(1, 0u);
+  P.fused_max_lines = 0;
+  for (int l = 0; l < nl; l += max_lines) {
+    const int lines = std::min(max_lines, nl - l);
+    P.fused_line.push_back((uint32_t)(l + lines));
+    P.fused_max_lines = std::max(P.fused_max_lines, lines);
+  }
+  P.fused_chunks = (int)P.fused_line.size() - 1;
+}
 
 // Column-stage kernels (Raman on, N1 = 64, M <= 16): Raman lines are processed in chunks of at
 // most max_lines (their LDS rows); chunk c covers lines [fused_line[c], fused_line[c+1]). The
@@ -596,15 +607,8 @@ bool plan_colstage_chunks(Problem& P, int max_lines, bool im) {
   P.fused_slot.clear();
   if (!P.raman || P.N1 != 64 || (int)P.M > colstage_max_modes()) return false;
   if (P.mixed) return plan_slot_chunks(P, max_lines);
-  const int nl = (int)P.active_lines(im);
-  if (nl < 1) return false;
-  P.fused_line.push_back(0);
-  for (int l = 0; l < nl; l += max_lines) {
-    const int lines = std::min(max_lines, nl - l);
-    P.fused_line.push_back((uint32_t)(l + lines));
-    P.fused_max_lines = std::max(P.fused_max_lines, lines);
-  }
-  P.fused_chunks = (int)P.fused_line.size() - 1;
+  if (P.active_lines(im) < 1) return false;
+  plan_product_chunks(P, max_lines, im);
   return true;
 }
 

@@ -103,6 +103,10 @@ bool split_length(uint32_t nt, uint32_t& n1, uint32_t& n2);
 // all products. Mixed precision: over line_a/b/self, within the LDS limits on slots and coefficients.
 bool plan_colstage_chunks(Problem& P, int max_lines, bool im);
 
+// The FP64 gathers' chunks (at most max_lines lines each) over the lines of the Re products or (im) of
+// all products: fills P.fused_*.
+void plan_product_chunks(Problem& P, int max_lines, bool im);
+
 // Coupling coefficients of the real products: Re products Q1 + Q2, Im products Q1 - Q2, as [p][x][k].
 std::vector<double> product_coefficients(const Problem& P);
 // Index k of coefficient kk of mode p in segment sg (>= P.M: none).

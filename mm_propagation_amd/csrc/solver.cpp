@@ -105,24 +105,24 @@ struct mmp_solver {
   int n_lines = 0;
   std::vector<HeadArgs> heads;  // s + 1 entries
   GatherArgs gather{};
-  PairLineArgs pairs{};
-  // column-stage step: the FP64 products' arguments (n_lines, line_prod also serve the pair pass in mixed
-  // precision), the mixed-precision slots'
+  // the FP64 gathers' products (n_lines and line_prod also serve the pair passes of the other gathers),
+  // and the slots of the mixed-precision column-stage step
   ProductArgs fused{};
   SlotArgs slots{};
   bool use_fused = false;
+  bool products = false;     // the gather sums the real products (FP64; beyond its sizes the sparse slots)
   int chunk_lines = 0;       // column-stage gather: Raman lines per LDS chunk at most
   bool tuned = false;        // MMP_FLAG_AUTOTUNE chose fused.waves and chunk_lines
   int pair_columns = 1;      // column-stage pair pass: columns per workgroup and line groups
   int pair_groups = 1;
   int conv_cols = 0;         // the pair pass stores the Raman lines in column order (large grids)
   bool chain = false;        // the step close also issues the next step's stage-0 head
-  // coupling blocks of the register gathers: the products' steps (FP64 column-stage step), or the slots'
-  // [P][M][M] (mixed column-stage step: parity-compact where they have the structure)
+  // coupling blocks of the register gathers: the products' steps (FP64), or the slots' [P][M][M] (mixed
+  // column-stage step: parity-compact where they have the structure)
   double* qdense = nullptr;
   std::vector<uint32_t> step_table;  // the vector gather's steps, whose order the coupling blocks follow
   bool loaded = false;       // every fiber's data is on the device
-  bool need_im = false;      // the column-stage step runs the Im products (a fiber's couplings need them)
+  bool need_im = false;      // the step runs the Im products (a fiber's couplings need them)
   uint32_t plan_id = 0;      // counts changes of the kernels' plan: graphs captured before are stale
   // work arrays of the step in the work precision (the FP64 buffers above in FP64 mode)
   bool mixed = false;
@@ -305,7 +305,7 @@ mmp_status enqueue_step_w(mmp_solver* s) {
   const double cb = sizeof(cw);  // bytes per complex work value
   const double cs = 16.0;        // bytes per complex FP64 state value
   const double MN = (double)P.M * P.N;
-  const double LN = (double)(s->use_fused ? s->fused.n_lines : s->n_lines) * P.N;
+  const double LN = (double)s->fused.n_lines * P.N;
   const double invN = 1.0 / P.N;
   for (int i = 0; i <= P.rk.s; i++) {
     if (i > 0 || !s->chain) MMP_TRY(enqueue_head_w<W>(s, i));
@@ -332,17 +332,21 @@ mmp_status enqueue_step_w(mmp_solver* s) {
                        [&] { return launch_col_inverse<W>(g, s->tw, ybuf, U, P.M, invN, 1.0, st); }));
     if (P.raman) {
       MMP_TRY(run_kernel(s, "col_pairs_forward", cb * (MN + LN), [&] {
-        return launch_col_pairs_forward<W>(g, s->tw, U, conv, s->n_lines, s->pairs, st);
+        return launch_col_pairs_forward<W>(g, s->tw, U, conv, s->fused.n_lines, s->fused.line_prod, st);
       }));
       MMP_TRY(run_kernel(s, "row_raman", cb * (2 * LN + P.N),
-                         [&] { return launch_row_raman<W>(g, s->tw, conv, s->n_lines, hspec, s->batch, 1, st); }));
+                         [&] { return launch_row_raman<W>(g, s->tw, conv, s->fused.n_lines, hspec, s->batch, 1, st); }));
       MMP_TRY(run_kernel(s, "col_inverse_raman", 2 * cb * LN, [&] {
-        return launch_col_inverse<W>(g, s->tw, conv, conv, s->n_lines, invN, 1.0, st);
+        return launch_col_inverse<W>(g, s->tw, conv, conv, s->fused.n_lines, invN, 1.0, st);
       }));
     }
     MMP_TRY(run_kernel(s, "gather_kerr_raman", cb * (2 * MN + LN), [&] {
-      return qdense ? launch_gather_dense<W>(g, U, conv, ybuf, s->gather, qdense, st)
-                    : launch_gather<W>(g, U, conv, ybuf, s->gather, st);
+      if constexpr (std::is_same<W, double>::value) {
+        if (s->products) return launch_gather_products(g, U, conv, ybuf, s->fused, qdense, s->batch, P.raman, st);
+      } else {
+        if (qdense) return launch_gather_dense<W>(g, U, conv, ybuf, s->gather, qdense, st);
+      }
+      return launch_gather<W>(g, U, conv, ybuf, s->gather, st);
     }));
     MMP_TRY(run_kernel(s, "col_forward_sigma", 2 * cb * MN,
                        [&] { return launch_col_forward<W>(g, s->tw, ybuf, ybuf, P.M, st); }));
@@ -503,11 +507,24 @@ void release(mmp_solver* s) {
 // mixed-precision stage heads form E_u from Im L and the fiber's z where they use it.
 bool lawson_tables(bool mixed) { return !mixed; }
 
-// Coupling coefficients of one fiber: of the FP64 column-stage gather's products, or of the slots.
+// FP64 gathers sum the real products: the column-stage one always, the separate one up to 16
+// coefficients per product and mode (32 modes with the parity structure).
+bool sums_products(const Problem& P, bool fused) {
+  return !P.mixed && (fused || (P.n_products() > 0 && gather_products_ok((int)P.M, P.parity)));
+}
+// Dense coupling blocks exist (else the sparse gather's lists serve).
+bool coupling_blocks(const Problem& P, bool fused) {
+  return fused || sums_products(P, fused) || (P.mixed && dense_gather_chunk((int)P.M) > 0);
+}
+
+// Coupling coefficients of one fiber: of the FP64 gathers' products, or of the slots.
 size_t coupling_block_size(const Problem& P, bool fused) {
-  if (fused && !P.mixed) return (size_t)P.M * P.product_steps() * 16;
+  if (sums_products(P, fused)) return (size_t)P.M * P.product_steps() * 16;
   return (size_t)P.P * P.M * (fused && P.parity ? (P.M + 1) / 2 : P.M);
 }
+// Line descriptors: of the Raman lines, where the gather sums the products of these (two a line, Raman on
+// or off).
+size_t product_lines(const Problem& P, bool products) { return products ? (P.n_products() + 1) / 2 : P.line_a.size(); }
 // Step descriptors of the products' gather, read 64 at a time.
 size_t step_table_size(const Problem& P) { return (P.product_steps() / 64 + 2) * 64; }
 
@@ -523,18 +540,18 @@ size_t planned_device_bytes(const Problem& P, const mmp_options& opt, size_t F) 
   if (lawson_tables(mixed)) b += 16 * MN * F * (2 * P.c_unique.size() + 1);
   if (any_stash) b += 16 * (size_t)P.rk.s * MN * F;
   if (P.raman) b += (mixed ? 8 : 16) * c(L) * P.N * F + 16 * (size_t)P.N * F + 8 * (size_t)P.N;
-  b += 4 * c(P.coff.size()) + 4 * c(P.nnz) + 8 * c(P.nnz) + 4 * 4 * c(P.P) + 4 * 3 * c(L);
+  const bool fused = P.fused_chunks > 0 && !(opt.flags & MMP_FLAG_SEPARATE_COLUMNS), products = sums_products(P, fused);
+  const size_t LP = product_lines(P, products);
+  b += 8 * c(LP);
+  if (!products) b += 4 * c(P.coff.size()) + 4 * c(P.nnz) + 8 * c(P.nnz) + 4 * 4 * c(P.P);  // the sparse gather's lists
   if (mixed) {
     b += 8 * (2 * MN) * F + 8 * (P.N2 + P.N1 + P.N) + 4 * c(P.nnz);
     if (P.raman) b += 8 * (size_t)P.N * F;
   }
-  if (P.fused_chunks > 0 && !(opt.flags & MMP_FLAG_SEPARATE_COLUMNS)) {
-    // chunk bounds sized for the finest plan, the lines' products, the steps or the slots
-    b += 4 * (L + 1) + 8 * c(L) + 4 * (mixed ? L + 1 + c(P.P) : step_table_size(P));
-    if (P.raman) b += (mixed ? 8 : 16) * c(L) * P.N * F;  // the Raman lines in column order
-  }
-  const bool fused = P.fused_chunks > 0 && !(opt.flags & MMP_FLAG_SEPARATE_COLUMNS);
-  if (fused || dense_gather_chunk((int)P.M) > 0) b += (mixed ? 4 : 8) * coupling_block_size(P, fused) * F;
+  // chunk bounds sized for the finest plan, the steps or the slots
+  if (fused || products) b += 4 * (c(LP) + 1) + 4 * (mixed ? c(L) + 1 + c(P.P) : step_table_size(P));
+  if (fused && P.raman) b += (mixed ? 8 : 16) * c(L) * P.N * F;  // the Raman lines in column order
+  if (coupling_blocks(P, fused)) b += (mixed ? 4 : 8) * coupling_block_size(P, fused) * F;
   return b;
 }
 
@@ -607,7 +624,7 @@ mmp_status upload_couplings(mmp_solver* s, uint32_t f, const Problem& Pf) {
   std::vector<double> qd;
   std::vector<float> qd32;
   const Batch& b = s->batch;
-  if (s->use_fused && !s->mixed) qd = product_blocks(Pf, product_coefficients(Pf), s->step_table);
+  if (s->products) qd = product_blocks(Pf, product_coefficients(Pf), s->step_table);
   else qd = dense_blocks(Pf, s->slots.parity != 0);
   if (s->mixed) {
     qd32.assign(qd.begin(), qd.end());
@@ -619,11 +636,13 @@ mmp_status upload_couplings(mmp_solver* s, uint32_t f, const Problem& Pf) {
   return MMP_OK;
 }
 
-// The Raman lines and their chunks (at most max_lines each) of the column-stage step. FP64: the lines of
-// the Re products, or of all products where s->need_im, and the products' steps; mixed: the slots'.
+// The Raman lines and their chunks (at most max_lines each) of the gather. FP64: the lines of the Re
+// products, or of all products where s->need_im, and the products' steps; mixed: the slots'.
 mmp_status install_lines(mmp_solver* s, int max_lines) {
   Problem& P = s->P;
-  if (!plan_colstage_chunks(P, max_lines, s->need_im)) return fail(MMP_ERR_INVALID_ARGUMENT, "no chunk plan for these limits");
+  if (!s->use_fused) plan_product_chunks(P, max_lines, s->need_im);
+  else if (!plan_colstage_chunks(P, max_lines, s->need_im))
+    return fail(MMP_ERR_INVALID_ARGUMENT, "no chunk plan for these limits");
   const uint32_t* d_line = s->mixed ? s->slots.chunk_line : s->fused.chunk_line;
   MMP_TRY(upload(s, const_cast<uint32_t*>(d_line), P.fused_line.data(), P.fused_line.size() * 4));
   HIP_TRY(hipStreamSynchronize(s->ctx->stream), "hipStreamSynchronize");  // P.fused_line is the staging copy
@@ -646,6 +665,10 @@ mmp_status install_lines(mmp_solver* s, int max_lines) {
   fa.n_lines = (int)P.active_lines(s->need_im);
   fa.n_products = (int)P.active_products(s->need_im);
   fa.stride = (int)P.product_steps();
+  for (int sg = 0; sg < 4; sg++) {
+    fa.seg_b[sg] = (int)P.seg_b[sg];
+    fa.seg_e[sg] = (int)P.seg_e[sg];
+  }
   std::vector<uint32_t> table = product_step_table(P, s->need_im);
   fa.n_steps = (int)table.size();
   fa.odd_step = 0;
@@ -793,13 +816,13 @@ mmp_status create_impl(mmp_ctx* ctx, uint32_t n_fibers, const mmp_params* params
   const size_t conv_n = (size_t)(s->n_lines ? s->n_lines : 1) * P.N;
   bool any_stash = false;
   for (int j = 0; j < P.rk.s; j++) any_stash = any_stash || P.stash_needed[j];
-  // dense blocks: the column-stage gather always takes them, the separate gather up to its own limit
-  const bool dense = s->use_fused || dense_gather_chunk((int)P.M) > 0;
+  const bool dense = coupling_blocks(P, s->use_fused);
   s->batch.sf = MN;
   s->batch.sl = conv_n;
   s->batch.se = s->ntab * MN;
   s->batch.ss = (size_t)P.rk.s * MN;
-  const bool compact = s->use_fused && P.parity;
+  s->products = sums_products(P, s->use_fused);
+  const bool compact = (s->use_fused || s->products) && P.parity;
   s->slots.parity = compact && s->mixed ? 1 : 0;
   s->batch.sq = coupling_block_size(P, s->use_fused);
   s->batch.sh = P.N;
@@ -876,19 +899,18 @@ mmp_status create_impl(mmp_ctx* ctx, uint32_t n_fibers, const mmp_params* params
       s->qdense_w = s->qdense;
     }
   }
-  uint32_t *d_coff, *d_k, *d_sa, *d_sb, *d_sl, *d_sk, *d_la, *d_lb, *d_ls;
-  double* d_q;
-  const size_t nnz1 = P.nnz ? P.nnz : 1, P1 = P.P ? P.P : 1, L1 = s->n_lines ? s->n_lines : 1;
-  A(dalloc(s, &d_coff, P.coff.size()));
-  A(dalloc(s, &d_k, nnz1));
-  A(dalloc(s, &d_q, nnz1));
-  A(dalloc(s, &d_sa, P1));
-  A(dalloc(s, &d_sb, P1));
-  A(dalloc(s, &d_sl, P1));
-  A(dalloc(s, &d_sk, P1));
-  A(dalloc(s, &d_la, L1));
-  A(dalloc(s, &d_lb, L1));
-  A(dalloc(s, &d_ls, L1));
+  uint32_t *d_coff = nullptr, *d_k = nullptr, *d_sa = nullptr, *d_sb = nullptr, *d_sl = nullptr, *d_sk = nullptr;
+  double* d_q = nullptr;
+  const size_t nnz1 = P.nnz ? P.nnz : 1, P1 = P.P ? P.P : 1, LP = product_lines(P, s->products), L1 = LP ? LP : 1;
+  if (!s->products) {  // the sparse gather's lists
+    A(dalloc(s, &d_coff, P.coff.size()));
+    A(dalloc(s, &d_k, nnz1));
+    A(dalloc(s, &d_q, nnz1));
+    A(dalloc(s, &d_sa, P1));
+    A(dalloc(s, &d_sb, P1));
+    A(dalloc(s, &d_sl, P1));
+    A(dalloc(s, &d_sk, P1));
+  }
   if (st != MMP_OK) return cleanup(st);
   // batch-wide tables (host copies stay alive until the stream synchronisation below)
   std::vector<uint32_t> kslot(P.nnz);
@@ -903,22 +925,17 @@ mmp_status create_impl(mmp_ctx* ctx, uint32_t n_fibers, const mmp_params* params
     A(upload(s, coltw32, tc32.data(), tc32.size() * 4));
     A(upload(s, fourtw32, t432.data(), t432.size() * 4));
   }
-  A(upload(s, d_coff, P.coff.data(), P.coff.size() * 4));
-  if (P.nnz) {
+  if (!s->products) A(upload(s, d_coff, P.coff.data(), P.coff.size() * 4));
+  if (P.nnz && !s->products) {
     for (uint32_t e = 0; e < P.nnz; e++) kslot[e] = P.k[e] | (P.slot[e] << 8);
     A(upload(s, d_k, kslot.data(), P.nnz * 4));
     A(upload(s, d_q, P.q.data(), P.nnz * 8));
   }
-  if (P.P) {
+  if (P.P && !s->products) {
     A(upload(s, d_sa, P.slot_a.data(), P.P * 4));
     A(upload(s, d_sb, P.slot_b.data(), P.P * 4));
     A(upload(s, d_sl, P.slot_line.data(), P.P * 4));
     A(upload(s, d_sk, P.slot_kind.data(), P.P * 4));
-  }
-  if (s->n_lines) {
-    A(upload(s, d_la, P.line_a.data(), s->n_lines * 4));
-    A(upload(s, d_lb, P.line_b.data(), s->n_lines * 4));
-    A(upload(s, d_ls, P.line_self.data(), s->n_lines * 4));
   }
   std::vector<float> q32(P.q.begin(), P.q.end());
   float* d_q32 = nullptr;
@@ -931,36 +948,37 @@ mmp_status create_impl(mmp_ctx* ctx, uint32_t n_fibers, const mmp_params* params
   s->q_w = s->mixed ? (const void*)d_q32 : (const void*)d_q;
   s->gather = GatherArgs{d_coff, d_k, s->q_w, d_sa, d_sb, d_sl, d_sk, (int)P.P, P.gather_chunk,
                          P.gather_chunks, P.gather_cap, P.raman, P.kv, P.kr};
-  s->pairs = PairLineArgs{d_la, d_lb, d_ls};
   s->batch.fp = s->d_fp;
   s->batch.coef = s->d_coef;
   s->batch.st = s->st;
-  std::vector<uint2> line_prod(s->mixed ? P.line_a.size() : (P.n_products() + 1) / 2);
+  // the two products of every line
+  std::vector<uint2> line_prod(LP);
   std::vector<uint32_t> slot_meta(s->mixed ? P.P : 0);
-  if (s->use_fused) {
-    uint32_t* d_cl;
-    uint2* d_lp;
-    A(dalloc(s, &d_cl, L1 + 1));  // room for the finest chunking the tuner may pick
-    A(dalloc(s, &d_lp, L1));
-    if (st != MMP_OK) return cleanup(st);
-    auto product = [](uint32_t a, uint32_t b, uint32_t im) { return a | (b << 8) | (im << 16); };
-    const uint32_t absent = 1u << 17;
-    for (uint32_t l = 0; l < line_prod.size(); l++) {
-      if (s->mixed) {  // a cross pair's line, or two self pairs'
-        const uint32_t a = P.line_a[l], b = P.line_b[l];
-        line_prod[l] = P.line_self[l] ? make_uint2(product(a, a, 0), b != 0xffffffffu ? product(b, b, 0) : absent)
-                                      : make_uint2(product(a, b, 0), product(a, b, 1));
-      } else {
-        auto at = [&](uint32_t x) {
-          return x < P.n_products() ? product(P.prod_a[x], P.prod_b[x], P.prod_im[x]) : absent;
-        };
-        line_prod[l] = make_uint2(at(2 * l), at(2 * l + 1));
-      }
+  uint2* d_lp;
+  A(dalloc(s, &d_lp, L1));
+  if (st != MMP_OK) return cleanup(st);
+  auto product = [](uint32_t a, uint32_t b, uint32_t im) { return a | (b << 8) | (im << 16); };
+  const uint32_t absent = 1u << 17;
+  for (uint32_t l = 0; l < LP; l++) {
+    if (!s->products) {  // a cross pair's line, or two self pairs'
+      const uint32_t a = P.line_a[l], b = P.line_b[l];
+      line_prod[l] = P.line_self[l] ? make_uint2(product(a, a, 0), b != 0xffffffffu ? product(b, b, 0) : absent)
+                                    : make_uint2(product(a, b, 0), product(a, b, 1));
+    } else {
+      auto at = [&](uint32_t x) {
+        return x < P.n_products() ? product(P.prod_a[x], P.prod_b[x], P.prod_im[x]) : absent;
+      };
+      line_prod[l] = make_uint2(at(2 * l), at(2 * l + 1));
     }
-    A(upload(s, d_lp, line_prod.data(), line_prod.size() * sizeof(uint2)));
-    s->fused.line_prod = d_lp;
-    s->fused.n_lines = (int)line_prod.size();
-    const int M = (int)P.M;
+  }
+  if (LP) A(upload(s, d_lp, line_prod.data(), LP * sizeof(uint2)));
+  s->fused.line_prod = d_lp;
+  s->fused.n_lines = (int)LP;
+  const int M = (int)P.M;
+  if (s->use_fused || s->products) {
+    uint32_t* d_cl;
+    A(dalloc(s, &d_cl, L1 + 1));  // room for the finest chunking the tuner may pick
+    if (st != MMP_OK) return cleanup(st);
     if (s->mixed) {
       uint32_t *d_cs, *d_meta;
       A(dalloc(s, &d_cs, L1 + 1));
@@ -1004,11 +1022,11 @@ mmp_status create_impl(mmp_ctx* ctx, uint32_t n_fibers, const mmp_params* params
       s->fused.steps = d_steps;
       s->fused.parity = compact ? 1 : 0;
       for (const Problem& Pf : s->fib) s->need_im = s->need_im || Pf.need_im;
-      if (st == MMP_OK) A(install_lines(s, colstage_lines_per_chunk(M)));
-      s->fused.cols = gather_cols(s);
-      s->fused.waves = gather_waves(s);
+      if (st == MMP_OK) A(install_lines(s, s->use_fused ? colstage_lines_per_chunk(M) : gather_products_lines(M, P.parity)));
+      s->fused.cols = s->use_fused ? gather_cols(s) : 1;
+      s->fused.waves = s->use_fused ? gather_waves(s) : 0;
     }
-    colstage_pairs_plan(M, s->g.N2, s->n_lines, (int)s->F, s->mixed, s->pair_columns, s->pair_groups);
+    if (s->use_fused) colstage_pairs_plan(M, s->g.N2, s->n_lines, (int)s->F, s->mixed, s->pair_columns, s->pair_groups);
     // lines in column order before the Raman row pass too: its LDS staging costs latency that
     // only large grids hide (measured: batched M = 10, NT = 16384 x 36 fibers row pass 140 ->
     // 111 us; one grin6 fiber 7.0 -> 7.6 us)
@@ -1720,7 +1738,7 @@ mmp_status mmp_fiber_load(mmp_solver* s, uint32_t f, const mmp_params* params) {
                                             "and pair structure");
     MMP_TRY(set_device(s));
     HIP_TRY(hipStreamSynchronize(s->ctx->stream), "hipStreamSynchronize");  // queued steps read the old fiber
-    if (s->use_fused && !s->mixed && Pf.need_im && !s->need_im) {
+    if (s->products && Pf.need_im && !s->need_im) {
       // the first fiber whose couplings need the Im products: the step takes their lines too (the other
       // fibers' Im coefficients are zero, and their Re products' arithmetic stays the same)
       s->need_im = true;

@@ -12,7 +12,8 @@ import oracle_binding as ob
 from gpu_util import note, require_device
 from mm_propagation_amd import _capi, configs
 from mm_propagation_amd.batch import MultimodePropagationBatch, SolverGroup
-from mm_propagation_amd.solver import Context, MultimodePropagationGPU_RamanON
+from mm_propagation_amd.problem import NonZeroValue
+from mm_propagation_amd.solver import Context, MultimodePropagationGPU_RamanOFF, MultimodePropagationGPU_RamanON
 
 pytestmark = pytest.mark.gpu
 
@@ -81,3 +82,39 @@ def test_a_general_fiber_joins_a_symmetric_batch(M, precision):
     g.close()
     b.close()
     other.close()
+
+
+def odd_coupling(sp):
+    """One more nonzero, at odd k + l - m - p: the couplings have no parity structure left."""
+    out = copy.deepcopy(sp)
+    q = out.coupling_coefficients[0]
+    q.addNonZeroValue(NonZeroValue((0, 1, 0), 0.3 * q.getNonZeroValue(0).value))
+    return out
+
+
+@pytest.mark.parametrize("raman", [True, False])
+@pytest.mark.parametrize("M,nt,coupling", [(1, 256, "symmetric"), (2, 1024, "k_le_l"), (4, 512, "odd"), (5, 1024, "unsymmetric"),
+                                           (8, 2048, "symmetric"), (9, 1024, "unsymmetric"), (16, 256, "odd"),
+                                           (17, 1024, "symmetric"), (17, 256, "odd"), (20, 512, "unsymmetric"),
+                                           (32, 256, "symmetric"), (33, 256, "symmetric")])
+def test_separate_gather_against_oracle(M, nt, coupling, raman):
+    """The separate passes' gather at its smallest and largest tables: one chunk and several, one to
+    four groups of modes, 4, 2 and 1 products a step; beyond 16 coefficients per product and mode the sparse
+    gather serves (odd couplings of 17 modes, 33 modes)."""
+    require_device()
+    sp = configs.grin_fiber(M=M, nt=nt, symmetric=coupling != "k_le_l", power_range=(1.0, 100.0), seed=5)
+    if coupling == "unsymmetric":
+        sp = unsymmetric(sp)
+    if coupling == "odd":
+        sp = odd_coupling(sp)
+    note(f"case separate gather M={M} nt={nt} {coupling} raman={raman}")
+    cls = MultimodePropagationGPU_RamanON if raman else MultimodePropagationGPU_RamanOFF
+    s = cls(sp, pair_decode=1)
+    s.computeLawsonRK(3)
+    got = s.getResult()
+    s.close()
+    o = ob.Oracle(sp, raman=raman, pair_decode=1, n_threads=16)
+    o.compute_lawson_rk(3)
+    err = configs.rel_l2_per_mode(got, o.get_result())
+    o.close()
+    assert np.all(err <= 1e-12), err
