@@ -1743,6 +1743,10 @@ mmp_status mmp_fiber_load(mmp_solver* s, uint32_t f, const mmp_params* params) {
       // fibers' Im coefficients are zero, and their Re products' arithmetic stays the same)
       s->need_im = true;
       MMP_TRY(install_lines(s, s->chunk_lines));
+      if (s->use_fused && !plan_valid(s, current_plan(s))) {  // more lines than the workgroup's LDS holds at these columns
+        s->fused.cols = gather_cols(s);
+        s->fused.waves = gather_waves(s);
+      }
       s->plan_id++;
       drop_graph(s);
       MMP_TRY(build_graph(s));

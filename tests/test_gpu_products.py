@@ -118,3 +118,22 @@ def test_separate_gather_against_oracle(M, nt, coupling, raman):
     err = configs.rel_l2_per_mode(got, o.get_result())
     o.close()
     assert np.all(err <= 1e-12), err
+
+
+def test_a_general_fiber_joins_a_large_symmetric_batch():
+    """At 6 modes and 2048 columns the gather takes two columns per workgroup on the 11 lines of
+    symmetric couplings; all 18 lines pass its LDS, so the load changes the workgroups too."""
+    require_device()
+    sps = [configs.grin_fiber(M=6, nt=4096, fiber_length=0.5 + 0.01 * i, seed=20 + i, symmetric=True) for i in range(32)]
+    general = unsymmetric(configs.grin_fiber(M=6, nt=4096, fiber_length=0.9, seed=61, symmetric=True))
+    note("case general fiber into a large symmetric batch")
+    b = MultimodePropagationBatch(sps, pair_decode=1)
+    b.advance(3)
+    b.load(31, general)
+    b.advance(3)
+    for f, sp, steps in ((0, sps[0], 6), (30, sps[30], 6), (31, general, 3)):
+        s = MultimodePropagationGPU_RamanON(sp, pair_decode=1)
+        s.computeLawsonRK(steps)
+        assert np.array_equal(b.result(f), s.getResult()), f
+        s.close()
+    b.close()
