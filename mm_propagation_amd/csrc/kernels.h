@@ -273,7 +273,8 @@ template <class W>
 hipError_t launch_colstage_fields_pairs(const Geometry& g, const Twiddles& tw, const cpx<W>* yin, cpx<W>* U,
                                         cpx<W>* conv, const uint2* line_prod, int n_lines, double scale,
                                         const Batch& b, int F, int columns, int groups, int conv_cols, hipStream_t s);
-// Qp: the products' coupling blocks [p][step][16] (product_blocks).
+// Qp: the products' coupling blocks [p][step][16] (product_blocks). Without Raman conv is null and U holds
+// the stage head's rows (row order; yout may be the same array): the whole column side of the stage.
 hipError_t launch_colstage_products(const Geometry& g, const Twiddles& tw, const cd* U, const cd* conv, cd* yout,
                                     const ProductArgs& fa, const double* Qp, double scale, const Batch& b, int F,
                                     hipStream_t s);

@@ -1143,11 +1143,14 @@ __device__ __forceinline__ void product_sums(const ProductArgs& fa, const W* Qsh
 // instead of 11 at 6 modes and 4 to 5 times the coupling sums. Whole step on one MI355X, before and after: 6 modes,
 // NT = 16384, RK4 111.5 -> 101.7 us; 2 modes, NT = 4096 71.1 -> 68.3 us; 5 modes without the
 // symmetric couplings (all products), NT = 8192, sixth order 164.6 -> 165.2 us (the one form kept).
-template <int M, int NW, int COLS, class W, bool PAR>
+// Without Raman (RAMAN = false) the whole column side of a stage is this one kernel: it takes the fields
+// themselves from `U` (row order; the same array as yout: a workgroup reads and writes its own columns only),
+// transforms them in their LDS rows, and the products have no line: 8 launches of 5-8 us an RK4 step in place
+// of 16, 6 modes, NT = 16384 78.7 -> 50.6 us per step. Bound by latency and its column access.
+template <int M, int NW, int COLS, class W, bool PAR, bool RAMAN>
 __global__ void __launch_bounds__(NW * 64) k_colstage_products(
-    Geometry g, const cpx<W>* __restrict__ coltw, const cpx<W>* __restrict__ fourtw, const cpx<W>* __restrict__ U,
-    const cpx<W>* __restrict__ conv, cpx<W>* __restrict__ yout, ProductArgs fa, const W* __restrict__ Qp, double scale,
-    Batch b) {
+    Geometry g, const cpx<W>* __restrict__ coltw, const cpx<W>* __restrict__ fourtw, const cpx<W>* U,
+    const cpx<W>* __restrict__ conv, cpx<W>* yout, ProductArgs fa, const W* __restrict__ Qp, double scale, Batch b) {
   using cw = cpx<W>;
   using C2 = C2Cfg<M, COLS, W, PAR>;
   const int fib = blockIdx.y;
@@ -1182,19 +1185,21 @@ __global__ void __launch_bounds__(NW * 64) k_colstage_products(
   cw v[8], uin[UIN], w4[8];
   LineTw<L, W> lt;
   int l0 = 0, l1 = fa.first_lines;
-  if (wave * JW < l1) {
-    const int q = jl < l1 ? jl : l1 - 1;  // lanes without a line read the last one's
-    const size_t base = (size_t)q * g.N + (size_t)n2 * L;
+  if (wave * JW < (RAMAN ? l1 : M)) {
+    const int last = (RAMAN ? l1 : M) - 1, q = jl < last ? jl : last;  // lanes without a line read the last one's
+    const size_t base = (size_t)q * g.N + (RAMAN ? (size_t)n2 * L : (size_t)n2);
 #pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = conv[base + t + i * T];
+    for (int i = 0; i < 8; i++) v[i] = RAMAN ? conv[base + t + i * T] : U[base + (size_t)(t + i * T) * g.N2];
   }
+  if constexpr (RAMAN) {
 #pragma unroll
-  for (int r = 0; r < UIN; r++) {
-    const int e = tid + r * NT;
-    if (wave * 64 + r * NT < M * COLS * L)  // (whole wavefronts)
-      uin[r] = U[(size_t)(e / (COLS * L)) * g.N + (size_t)n20 * L + e % (COLS * L)];
+    for (int r = 0; r < UIN; r++) {
+      const int e = tid + r * NT;
+      if (wave * 64 + r * NT < M * COLS * L)  // (whole wavefronts)
+        uin[r] = U[(size_t)(e / (COLS * L)) * g.N + (size_t)n20 * L + e % (COLS * L)];
+    }
   }
-  if (wave * JW < (l1 > M ? l1 : M)) {
+  if (wave * JW < (RAMAN && l1 > M ? l1 : M)) {
     load_line_tw<L>(lt, coltw, t);
 #pragma unroll
     for (int i = 0; i < 8; i++) w4[i] = fourtw[n2 * (t + i * T)];
@@ -1237,15 +1242,25 @@ __global__ void __launch_bounds__(NW * 64) k_colstage_products(
       }
     }
   }
+  if constexpr (RAMAN) {
 #pragma unroll
-  for (int r = 0; r < UIN; r++) {
-    const int e = tid + r * NT;
-    if (wave * 64 + r * NT < M * COLS * L) Ush[(e / L) * RS + e % L] = uin[r];
+    for (int r = 0; r < UIN; r++) {
+      const int e = tid + r * NT;
+      if (wave * 64 + r * NT < M * COLS * L) Ush[(e / L) * RS + e % L] = uin[r];
+    }
+    // the field row after the last one, which the coupling rows of an odd number of modes read with
+    // zero coefficients
+    constexpr int UZ = M % 2 && PAR ? M + 1 : M;
+    for (int e = M * COLS * L + tid; e < UZ * COLS * L; e += NT) Ush[(e / L) * RS + e % L] = cw{0, 0};
+  } else if (wave * JW < M) {
+    // the fields; the lanes beyond the last one leave zero rows (whole wavefronts: up to UR rows)
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] = cmulc(v[i], w4[i]);
+    cw* row = Ush + (jl * COLS + c) * RS;
+    line_fft<L, 1, 1, 1, W, true>(v, row, lt, t);
+#pragma unroll
+    for (int i = 0; i < 8; i++) row[t + i * T] = jl < M ? cscale(v[i], (W)scale) : cw{0, 0};
   }
-  // the field row after the last one, which the coupling rows of an odd number of modes read with
-  // zero coefficients
-  constexpr int UZ = M % 2 && PAR ? M + 1 : M;
-  for (int e = M * COLS * L + tid; e < UZ * COLS * L; e += NT) Ush[(e / L) * RS + e % L] = cw{0, 0};
   if constexpr (QL) {
 #pragma unroll
     for (int r = 0; r < QIN; r++)
@@ -1271,9 +1286,11 @@ __global__ void __launch_bounds__(NW * 64) k_colstage_products(
       }
     }
     // lane i: the products of the wavefront's i-th (line, column) row to mix
-    const int rows = (l1 - l0) * COLS;
-    const uint2 dl = fa.line_prod[l0 + (wave + NW * lane < rows ? (wave + NW * lane) / COLS : 0)];
-    for (int r0 = l0; r0 < l1; r0 += JL) {
+    // (without lines: to an even number, as a step of four products may read the row after the last one,
+    // times zero; the lines' rows fill up whole wavefronts)
+    const int rows = (RAMAN ? l1 - l0 : (l1 - l0 + 1) / 2 * 2) * COLS, nrow = (l1 - l0) * COLS;
+    const uint2 dl = fa.line_prod[l0 + (wave + NW * lane < nrow ? (wave + NW * lane) / COLS : 0)];
+    for (int r0 = l0; RAMAN && r0 < l1; r0 += JL) {
       if (r0 + wave * JW >= l1) break;  // no line of this wavefront in the round
       const int q = r0 + jl;
       const bool valid = q < l1;
@@ -1299,9 +1316,14 @@ __global__ void __launch_bounds__(NW * 64) k_colstage_products(
       const cw V0 = cmulc(uc[(d0 & 255u) * COLS * RS], uc[((d0 >> 8) & 255u) * COLS * RS]);
       const cw V1 = cmulc(uc[(d1 & 255u) * COLS * RS], uc[((d1 >> 8) & 255u) * COLS * RS]);
       W* x0 = Xsh + r * 2 * RS + lane;
-      const cw vr = Rsh[r * RS + lane];
-      x0[0] = kv * ((d0 >> 16) & 1u ? V0.im : V0.re) + kr * (vr.re * sc);
-      x0[RS] = kv * ((d1 >> 16) & 1u ? V1.im : V1.re) + kr * (vr.im * sc);
+      if constexpr (RAMAN) {
+        const cw vr = Rsh[r * RS + lane];
+        x0[0] = kv * ((d0 >> 16) & 1u ? V0.im : V0.re) + kr * (vr.re * sc);
+        x0[RS] = kv * ((d1 >> 16) & 1u ? V1.im : V1.re) + kr * (vr.im * sc);
+      } else {
+        x0[0] = kv * ((d0 >> 16) & 1u ? V0.im : V0.re);
+        x0[RS] = kv * ((d1 >> 16) & 1u ? V1.im : V1.re);
+      }
     }
     if constexpr (!QL) {
 #pragma unroll
@@ -2280,39 +2302,45 @@ hipError_t launch_colstage_fields_pairs(const Geometry& g, const Twiddles& tw, c
 }
 
 // C2 in FP64, on the real products
-template <int M, int NW, int COLS, bool PAR>
+template <int M, int NW, int COLS, bool PAR, bool RAMAN>
 static hipError_t c2_launch(const Geometry& g, const Twiddles& tw, const cd* U, const cd* conv, cd* yout,
                             const ProductArgs& fa, const double* Qp, double scale, const Batch& b, int F, hipStream_t s) {
   const size_t lds = colstage_products_lds_bytes(M, COLS, fa.max_chunk_lines, fa.stride);
   if (g.N2 % COLS || lds > kColStageLds) return hipErrorInvalidValue;
-  MMP_LAUNCH((k_colstage_products<M, NW, COLS, double, PAR>), dim3(g.N2 / COLS, F), dim3(NW * 64), lds, s, g, tw.coltw,
+  MMP_LAUNCH((k_colstage_products<M, NW, COLS, double, PAR, RAMAN>), dim3(g.N2 / COLS, F), dim3(NW * 64), lds, s, g, tw.coltw,
              tw.fourtw, U, conv, yout, fa, Qp, scale, b);
   return hipGetLastError();
 }
-template <int M, bool PAR>
+template <int M, bool PAR, bool RAMAN>
 static hipError_t c2_variant(const Geometry& g, const Twiddles& tw, const cd* U, const cd* conv, cd* yout,
                              const ProductArgs& fa, const double* Qp, double scale, const Batch& b, int F, hipStream_t s) {
-  if constexpr (M <= kColStageMaxM4) {
-    if (fa.cols == 4) return c2_launch<M, 4, 4, PAR>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
+  if constexpr (RAMAN && M <= kColStageMaxM4) {  // (without Raman one fiber's columns, at most 1024)
+    if (fa.cols == 4) return c2_launch<M, 4, 4, PAR, RAMAN>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
   }
-  if constexpr (M <= kColStageMaxM2) {
-    if (fa.cols == 2) return c2_launch<M, 4, 2, PAR>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
+  if constexpr (RAMAN && M <= kColStageMaxM2) {
+    if (fa.cols == 2) return c2_launch<M, 4, 2, PAR, RAMAN>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
   }
   if (fa.cols != 1) return hipErrorInvalidValue;
   if constexpr (PAR && (M == 5 || M == 6)) {
     if (fa.waves == 12) {
       if (fa.n_chunks != 1) return hipErrorInvalidValue;
-      return c2_launch<M, 12, 1, PAR>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
+      return c2_launch<M, 12, 1, PAR, RAMAN>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
     }
   }
   if (fa.waves == 8 && M <= 4 && PAR && fa.n_chunks != 1) return hipErrorInvalidValue;
-  if (fa.waves == 8) return c2_launch<M, 8, 1, PAR>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
-  return c2_launch<M, 4, 1, PAR>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
+  if (fa.waves == 8) return c2_launch<M, 8, 1, PAR, RAMAN>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
+  return c2_launch<M, 4, 1, PAR, RAMAN>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
 }
-#define MMP_PRODUCTS_CASE(MV)                                                                  \
-  case MV:                                                                                      \
-    return fa.parity ? c2_variant<MV, true>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s)       \
-                     : c2_variant<MV, false>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
+template <int M>
+static hipError_t c2_form(const Geometry& g, const Twiddles& tw, const cd* U, const cd* conv, cd* yout, const ProductArgs& fa,
+                          const double* Qp, double scale, const Batch& b, int F, hipStream_t s) {
+  if (conv) return fa.parity ? c2_variant<M, true, true>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s)
+                             : c2_variant<M, false, true>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
+  return fa.parity ? c2_variant<M, true, false>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s)
+                   : c2_variant<M, false, false>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
+}
+#define MMP_PRODUCTS_CASE(MV) \
+  case MV: return c2_form<MV>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
 hipError_t launch_colstage_products(const Geometry& g, const Twiddles& tw, const cd* U, const cd* conv, cd* yout,
                                     const ProductArgs& fa, const double* Qp, double scale, const Batch& b, int F,
                                     hipStream_t s) {

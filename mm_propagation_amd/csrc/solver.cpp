@@ -110,6 +110,7 @@ struct mmp_solver {
   ProductArgs fused{};
   SlotArgs slots{};
   bool use_fused = false;
+  bool kerr_cols = false;    // FP64 without Raman: one column kernel per stage (one fiber)
   bool products = false;     // the gather sums the real products (FP64; beyond its sizes the sparse slots)
   int chunk_lines = 0;       // column-stage gather: Raman lines per LDS chunk at most
   bool tuned = false;        // MMP_FLAG_AUTOTUNE chose fused.waves and chunk_lines
@@ -328,6 +329,13 @@ mmp_status enqueue_step_w(mmp_solver* s) {
       }));
       continue;
     }
+    if constexpr (std::is_same<W, double>::value)
+      if (s->kerr_cols) {
+        MMP_TRY(run_kernel(s, "col_kerr_gather", 2 * cb * MN, [&] {
+          return launch_colstage_products(g, s->tw, ybuf, nullptr, ybuf, s->fused, qdense, invN, s->batch, 1, st);
+        }));
+        continue;
+      }
     MMP_TRY(run_kernel(s, "col_inverse_fields", 2 * cb * MN,
                        [&] { return launch_col_inverse<W>(g, s->tw, ybuf, U, P.M, invN, 1.0, st); }));
     if (P.raman) {
@@ -555,6 +563,15 @@ size_t planned_device_bytes(const Problem& P, const mmp_options& opt, size_t F) 
   return b;
 }
 
+// FP64: wavefronts of the column-stage gather's workgroup. On grids that leave a CU one or two workgroups
+// it takes eight (12 at 5 and 6 modes where the Im products double the sums, `both`): a wavefront per
+// mode, up to 4 modes (12: 6) one per mode and parity class. Larger grids hide the sums' latency with
+// other workgroups.
+int products_waves(int M, long columns, bool both) {
+  if (columns > 512) return 4;
+  return (M == 5 || M == 6) && both ? 12 : 8;
+}
+
 void fill_info(const Problem& P, const mmp_options& opt, mmp_info* o) {
   std::memset(o, 0, sizeof *o);
   o->n_modes = P.M;
@@ -579,7 +596,9 @@ void fill_info(const Problem& P, const mmp_options& opt, mmp_info* o) {
   o->n_fibers = 1;
   o->live = 1;
   const bool fused = P.fused_chunks > 0 && !(opt.flags & MMP_FLAG_SEPARATE_COLUMNS);
-  o->gather_waves = fused ? (P.M <= 6 ? 8u : 4u) : 0u;  // the defaults, before any tuning
+  // the defaults, before any tuning
+  const bool both = P.need_im && P.parity && P.fused_chunks == 1;
+  o->gather_waves = !fused ? 0u : (P.mixed ? (P.M <= 6 ? 8u : 4u) : (uint32_t)products_waves((int)P.M, (long)P.N2, both));
   o->chunk_lines = fused ? (uint32_t)colstage_lines_per_chunk((int)P.M) : 0u;
   if (fused) {  // a solver of one fiber (a batch may choose differently; results do not depend on it)
     int columns = 1, groups = 1;
@@ -695,15 +714,9 @@ int gather_cols(const mmp_solver* s) {
   return 1;
 }
 
-// FP64: wavefronts of the gather's workgroup. On grids that leave a CU one or two workgroups the vector
-// form takes eight (12 at 5 and 6 modes where the Im products double the sums): a wavefront per
-// mode, up to 4 modes (12: 6) one per mode and parity class. Larger grids hide the sums' latency with
-// other workgroups.
 int gather_waves(const mmp_solver* s) {
-  const int M = (int)s->P.M;
-  if (s->fused.cols > 1 || (long)s->g.N2 * s->F > 512) return 4;
-  if ((M == 5 || M == 6) && s->need_im && s->fused.parity && s->fused.n_chunks == 1) return 12;
-  return 8;
+  if (s->fused.cols > 1) return 4;
+  return products_waves((int)s->P.M, (long)s->g.N2 * s->F, s->need_im && s->fused.parity && s->fused.n_chunks == 1);
 }
 
 // Uploads fiber f's own data (operators, couplings, Raman spectrum, initial state, scalars),
@@ -822,6 +835,10 @@ mmp_status create_impl(mmp_ctx* ctx, uint32_t n_fibers, const mmp_params* params
   s->batch.se = s->ntab * MN;
   s->batch.ss = (size_t)P.rk.s * MN;
   s->products = sums_products(P, s->use_fused);
+  // Raman off: the column-stage gather takes the fields from the heads and returns sigma in one kernel; the
+  // three separate passes measured 78.7 against 50.6 us per step at 6 modes, NT = 16384
+  s->kerr_cols = s->products && !P.raman && P.N1 == 64 && (int)P.M <= colstage_max_modes() &&
+                 !(opt.flags & MMP_FLAG_SEPARATE_COLUMNS);
   const bool compact = (s->use_fused || s->products) && P.parity;
   s->slots.parity = compact && s->mixed ? 1 : 0;
   s->batch.sq = coupling_block_size(P, s->use_fused);
@@ -1022,9 +1039,10 @@ mmp_status create_impl(mmp_ctx* ctx, uint32_t n_fibers, const mmp_params* params
       s->fused.steps = d_steps;
       s->fused.parity = compact ? 1 : 0;
       for (const Problem& Pf : s->fib) s->need_im = s->need_im || Pf.need_im;
-      if (st == MMP_OK) A(install_lines(s, s->use_fused ? colstage_lines_per_chunk(M) : gather_products_lines(M, P.parity)));
-      s->fused.cols = s->use_fused ? gather_cols(s) : 1;
-      s->fused.waves = s->use_fused ? gather_waves(s) : 0;
+      if (st == MMP_OK) A(install_lines(s, s->use_fused || s->kerr_cols ? colstage_lines_per_chunk(M)
+                                                                    : gather_products_lines(M, P.parity)));
+      s->fused.cols = gather_cols(s);
+      s->fused.waves = gather_waves(s);
     }
     if (s->use_fused) colstage_pairs_plan(M, s->g.N2, s->n_lines, (int)s->F, s->mixed, s->pair_columns, s->pair_groups);
     // lines in column order before the Raman row pass too: its LDS staging costs latency that
@@ -1743,7 +1761,7 @@ mmp_status mmp_fiber_load(mmp_solver* s, uint32_t f, const mmp_params* params) {
       // fibers' Im coefficients are zero, and their Re products' arithmetic stays the same)
       s->need_im = true;
       MMP_TRY(install_lines(s, s->chunk_lines));
-      if (s->use_fused && !plan_valid(s, current_plan(s))) {  // more lines than the workgroup's LDS holds at these columns
+      if (s->kerr_cols || (s->use_fused && !plan_valid(s, current_plan(s)))) {  // more lines than the workgroup's LDS holds at these columns
         s->fused.cols = gather_cols(s);
         s->fused.waves = gather_waves(s);
       }

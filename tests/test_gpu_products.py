@@ -137,3 +137,30 @@ def test_a_general_fiber_joins_a_large_symmetric_batch():
         assert np.array_equal(b.result(f), s.getResult()), f
         s.close()
     b.close()
+
+
+@pytest.mark.parametrize("M,nt,coupling", [(1, 4096, "symmetric"), (2, 8192, "k_le_l"), (3, 4096, "unsymmetric"), (4, 4096, "odd"),
+                                           (5, 4096, "unsymmetric"), (6, 65536, "symmetric"), (7, 4096, "mirror"),
+                                           (9, 4096, "unsymmetric"), (10, 4096, "odd"), (16, 4096, "unsymmetric")])
+def test_kerr_column_kernel_against_oracle(M, nt, coupling):
+    """Without Raman the whole column side of a stage is one kernel: odd and even modes (the zero field
+    row), one product to 256, coefficients in LDS and read ahead, one chunk and several; and the separate
+    passes on the same fiber."""
+    require_device()
+    sp = configs.grin_fiber(M=M, nt=nt, symmetric=coupling in ("symmetric", "unsymmetric", "odd"), mirror=coupling == "mirror",
+                            power_range=(1.0, 100.0), seed=9)
+    if coupling == "unsymmetric":
+        sp = unsymmetric(sp)
+    if coupling == "odd":
+        sp = odd_coupling(sp)
+    note(f"case kerr columns M={M} nt={nt} {coupling}")
+    o = ob.Oracle(sp, raman=False, pair_decode=1, n_threads=16)
+    o.compute_lawson_rk(3)
+    want = o.get_result()
+    o.close()
+    for flags in (0, _capi.MMP_FLAG_SEPARATE_COLUMNS):
+        s = MultimodePropagationGPU_RamanOFF(sp, pair_decode=1, flags=flags)
+        s.computeLawsonRK(3)
+        err = configs.rel_l2_per_mode(s.getResult(), want)
+        s.close()
+        assert np.all(err <= 1e-12), (flags, err)
