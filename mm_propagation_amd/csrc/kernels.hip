@@ -630,9 +630,9 @@ __global__ void __launch_bounds__((RamanColsCfg<L, W>::THREADS)) k_row_raman_col
 // Kerr + Raman gather over a tile of 64 consecutive samples:
 //   X_slot = kv * U_a conj(U_b) + kr * VR_slot        (slot mix, into LDS)
 //   sigma_p = sum over the nonzeros (k, slot, q) of Q^(p):  q * X_slot * U_k
-// One wavefront per mode p (lanes = samples), so the nonzero loop and its
-// metadata loads are uniform; nonzeros are sorted by slot so consecutive ones
-// reuse X. Slots are staged through LDS in chunks when M + P exceeds the tile.
+// One wavefront per mode p (lanes = samples; wavefronts of blockIdx.y's groups take turns where the
+// modes are more), so the nonzero loop and its metadata loads are uniform; nonzeros are sorted by slot
+// so consecutive ones reuse X. Slots are staged through LDS in chunks when M + P exceeds the tile.
 // ---------------------------------------------------------------------------
 // sum += q_e * X[slot_e - s0] * U[k_e] over the nonzeros [e0, e1) for this lane's sample.
 // e0, e1 and s0 are wave-uniform. Xs and Us point at the lane's sample in LDS rows of
@@ -760,7 +760,7 @@ __global__ void __launch_bounds__(512) k_gather(Geometry g, const cpx<W>* __rest
   cw* Xsh = sh + M * TS;   // [chunk][TS]
   const int t0 = blockIdx.x * TS;
   const int tid = threadIdx.x, nthr = blockDim.x;
-  const int lane = tid % TS, nwaves = nthr / TS;
+  const int lane = tid % TS, nwaves = nthr / TS, ny = gridDim.y;
   const int wave = __builtin_amdgcn_readfirstlane(tid / TS);  // wave-uniform for the compiler
 #pragma unroll 4
   for (int e = tid; e < M * TS; e += nthr) Ush[e] = U[(size_t)(e / TS) * g.N + t0 + e % TS];
@@ -775,7 +775,7 @@ __global__ void __launch_bounds__(512) k_gather(Geometry g, const cpx<W>* __rest
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < kGatherMaxPW; r++) {
-      const int p = wave + r * nwaves;
+      const int p = wave + (r * ny + blockIdx.y) * nwaves;
       if (p >= M) break;
       const uint32_t* co = a.coff + (size_t)p * (a.n_chunks + 1) + c;
       acc[r] = gather_sum(acc[r], a.kslot, qv, co[0], co[1], s0, Xsh + lane, Ush + lane, TS, lane);
@@ -783,7 +783,7 @@ __global__ void __launch_bounds__(512) k_gather(Geometry g, const cpx<W>* __rest
   }
 #pragma unroll
   for (int r = 0; r < kGatherMaxPW; r++) {
-    const int p = wave + r * nwaves;
+    const int p = wave + (r * ny + blockIdx.y) * nwaves;
     if (p >= M) break;
     sigma[(size_t)p * g.N + t0 + lane] = acc[r];
   }
@@ -2223,7 +2223,16 @@ hipError_t launch_gather(const Geometry& g, const cpx<W>* U, const cpx<W>* VR, c
   if (g.N % kGatherTS) return hipErrorInvalidValue;
   int waves = g.M < 8 ? g.M : 8;
   if ((g.M + waves - 1) / waves > kGatherMaxPW) return hipErrorInvalidValue;
-  dim3 grid(g.N / kGatherTS), block(kGatherTS * waves);
+  // A wavefront sums its modes one after the other, so small grids deal the modes to groups of workgroups,
+  // up to one mode a wavefront, while tiles x groups stay within 512 (two workgroups a CU). Beyond that
+  // each group's own slot mix costs more than it gives. Mixed steps on one MI355X, us with one group and
+  // with the rule's: 20 modes, NT = 1024 (16 tiles) 2307 -> 1174, NT = 4096 2392 -> 1223; 32 modes, NT = 4096
+  // 15423 -> 4310; 14 modes, NT = 1024 835 -> 527; 18 modes, NT = 16384 (256 tiles) 2002 -> 1644 with two, 1873
+  // with three; 20 modes, NT = 65536 (1024 tiles) 8222, two groups 8546.
+  const int tiles = g.N / kGatherTS;
+  int groups = (g.M + waves - 1) / waves;
+  while (groups > 1 && tiles * groups > 512) groups--;
+  dim3 grid(g.N / kGatherTS, groups), block(kGatherTS * waves);
   if (a.cap == 4096) MMP_LAUNCH((k_gather<4096, W>), grid, block, 0, s, g, U, VR, sigma, a);
   else if (a.cap == 8192) MMP_LAUNCH((k_gather<8192, W>), grid, block, 0, s, g, U, VR, sigma, a);
   else return hipErrorInvalidValue;
