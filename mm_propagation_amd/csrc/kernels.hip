@@ -1605,7 +1605,8 @@ __global__ void __launch_bounds__(NW * 64, HI ? 3 : (MF ? (MfmaRows<M, PAR>::RT 
     qin[r] = e < (s1 - s0) * MM ? Qd[(size_t)s0 * MM + e] : (W)0;
   }
   if (tid < s1 - s0) min_ = fa.slot_meta[s0 + tid];
-  if (wave * (64 / T) < (l1 > M ? l1 : M)) {
+  // (a later chunk may hold more lines than the first one: its limit is on slots, one or two a line)
+  if (wave * (64 / T) < (fa.max_chunk_lines > M ? fa.max_chunk_lines : M)) {
     load_line_tw<L>(lt, coltw, t);
 #pragma unroll
     for (int i = 0; i < 8; i++) w4[i] = fourtw[n2 * (t + i * T)];
