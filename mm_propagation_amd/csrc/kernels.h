@@ -219,7 +219,7 @@ int colstage_lines_per_chunk(int M);  // Raman lines of one LDS chunk at most
 int colstage_slots_per_chunk();
 int colstage_coefficients_per_chunk(int M, bool mixed);
 constexpr size_t kColStageLds = 65536;      // dynamic LDS of one gather workgroup at most
-size_t colstage_products_lds_bytes(int M, int cols, int lines, int steps);
+size_t colstage_products_lds_bytes(int M, int cols, int lines, int steps, bool parity);
 constexpr size_t kColStagePairsLds = 65536;
 size_t colstage_pairs_lds_bytes(int M, int columns, bool mixed);
 // C1 layout for F fibers: four columns per workgroup where the LDS allows (else two, else

@@ -1007,6 +1007,10 @@ constexpr int steps_cap(int M, bool parity) {
   const int G = 16 / coef_pad(parity ? (M + 1) / 2 : M);
   return (M * M + G - 1) / G + 3;
 }
+// sigma in rows of its own (one barrier less) where one column's LDS has room for them beside the lines of
+// all products: up to 6 modes with the parity structure, up to 5 without (6 modes: 18 lines in 24 rows and 19
+// steps would take 65,792 bytes; sigma in the lines' rows leaves 51,968)
+constexpr bool own_sigma(int M, int cols, bool parity) { return cols == 1 && M <= (parity ? 6 : 5); }
 template <int M, int COLS, class W, bool PAR>
 struct C2Cfg {
   static constexpr int UR = (M + 7) / 8 * 8;
@@ -1015,15 +1019,14 @@ struct C2Cfg {
     const int jw = 8 / COLS, rows = (lines + jw - 1) / jw * jw, sig = 2 * M;
     return (size_t)(UR + (OWN ? rows + sig : (rows > sig ? rows : sig))) * COLS * kColStageRS * sizeof(cpx<W>);
   }
-  // sigma in rows of its own (one barrier less) where one column's LDS leaves room for them
-  static constexpr bool OWN = COLS == 1 && M <= 6;
+  static constexpr bool OWN = own_sigma(M, COLS, PAR);
   // vector form with two wavefronts per mode and column, one for each parity class
   template <int NW>
   static constexpr bool cs() { return PAR && M <= 6 && NW / COLS >= 2 * M; }
 };
-size_t colstage_products_lds_bytes(int M, int cols, int lines, int steps) {
+size_t colstage_products_lds_bytes(int M, int cols, int lines, int steps, bool parity) {
   const int jw = 8 / cols, rows = (lines + jw - 1) / jw * jw, sig = 2 * M;
-  const bool own = cols == 1 && M <= 6;
+  const bool own = own_sigma(M, cols, parity);
   return (size_t)((M + 7) / 8 * 8 + (own ? rows + sig : (rows > sig ? rows : sig))) * cols * kColStageRS * sizeof(cd) +
          (M <= 6 ? ((size_t)M * steps + 4) * 16 * sizeof(double) : 0);  // (+ 4: steps read ahead)
 }
@@ -2315,7 +2318,7 @@ hipError_t launch_colstage_fields_pairs(const Geometry& g, const Twiddles& tw, c
 template <int M, int NW, int COLS, bool PAR, bool RAMAN>
 static hipError_t c2_launch(const Geometry& g, const Twiddles& tw, const cd* U, const cd* conv, cd* yout,
                             const ProductArgs& fa, const double* Qp, double scale, const Batch& b, int F, hipStream_t s) {
-  const size_t lds = colstage_products_lds_bytes(M, COLS, fa.max_chunk_lines, fa.stride);
+  const size_t lds = colstage_products_lds_bytes(M, COLS, fa.max_chunk_lines, fa.stride, PAR);
   if (g.N2 % COLS || lds > kColStageLds) return hipErrorInvalidValue;
   MMP_LAUNCH((k_colstage_products<M, NW, COLS, double, PAR, RAMAN>), dim3(g.N2 / COLS, F), dim3(NW * 64), lds, s, g, tw.coltw,
              tw.fourtw, U, conv, yout, fa, Qp, scale, b);

@@ -535,7 +535,7 @@ mmp_status prepare_problem(const mmp_params* in, const mmp_options& opt, Problem
   }
   P.kv = P.raman ? 1 - P.fR : 1.;
   P.kr = P.raman ? P.fR * P.T0 : 0.;
-  plan_colstage_chunks(P, colstage_lines_per_chunk((int)M), P.need_im);
+  plan_colstage_chunks(P, colstage_chunk_lines(P, P.need_im), P.need_im);
   // a stage result N_j needs a stash slot when a stage i > j + 1 reads it
   P.stash_needed.assign(P.rk.s, 0);
   for (int i = 0; i < P.rk.s; i++)
@@ -593,6 +593,14 @@ void plan_product_chunks(Problem& P, int max_lines, bool im) {
     P.fused_max_lines = std::max(P.fused_max_lines, lines);
   }
   P.fused_chunks = (int)P.fused_line.size() - 1;
+}
+
+int colstage_chunk_lines(const Problem& P, bool im) {
+  if ((int)P.M > colstage_max_modes()) return 0;
+  const int lines = colstage_lines_per_chunk((int)P.M), n = (int)P.active_lines(im);
+  if (P.mixed) return lines;
+  return colstage_products_lds_bytes((int)P.M, 1, std::min(lines, n), (int)P.product_steps(), P.parity) <= kColStageLds ? lines
+                                                                                                                : 0;
 }
 
 // Column-stage kernels (Raman on, N1 = 64, M <= 16): Raman lines are processed in chunks of at

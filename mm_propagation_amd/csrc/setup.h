@@ -98,6 +98,10 @@ mmp_status prepare_problem(const mmp_params* in, const mmp_options& opt, Problem
 // rows would exceed 1024 samples; false if NT is unsupported.
 bool split_length(uint32_t nt, uint32_t& n1, uint32_t& n2);
 
+// Raman lines per LDS chunk of the column-stage kernels by default; 0 where the kernels do not take the problem
+// (FP64: the lines of the Re products or (im) of all, sigma and the coefficients in one column's workgroup).
+int colstage_chunk_lines(const Problem& P, bool im);
+
 // Chunks of Raman lines (at most max_lines each) for the column-stage kernels: fills P.fused_*; false
 // (and no chunks) when those kernels do not apply. FP64: over the lines of the Re products or (im) of
 // all products. Mixed precision: over line_a/b/self, within the LDS limits on slots and coefficients.

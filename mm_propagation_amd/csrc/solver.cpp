@@ -599,7 +599,7 @@ void fill_info(const Problem& P, const mmp_options& opt, mmp_info* o) {
   // the defaults, before any tuning
   const bool both = P.need_im && P.parity && P.fused_chunks == 1;
   o->gather_waves = !fused ? 0u : (P.mixed ? (P.M <= 6 ? 8u : 4u) : (uint32_t)products_waves((int)P.M, (long)P.N2, both));
-  o->chunk_lines = fused ? (uint32_t)colstage_lines_per_chunk((int)P.M) : 0u;
+  o->chunk_lines = fused ? (uint32_t)colstage_chunk_lines(P, P.need_im) : 0u;
   if (fused) {  // a solver of one fiber (a batch may choose differently; results do not depend on it)
     int columns = 1, groups = 1;
     colstage_pairs_plan((int)P.M, (int)P.N2, (int)P.line_a.size(), 1, opt.precision == MMP_PRECISION_MIXED, columns,
@@ -709,7 +709,8 @@ int gather_cols(const mmp_solver* s) {
   const long columns = (long)s->g.N2 * s->F;
   for (int cols : {4, 2})
     if (columns >= 1024 * cols && colstage_cols_ok(M, cols) &&
-        colstage_products_lds_bytes(M, cols, s->fused.max_chunk_lines, s->fused.stride) <= kColStageLds)
+        colstage_products_lds_bytes(M, cols, s->fused.max_chunk_lines, s->fused.stride, s->P.parity) <=
+            kColStageLds)
       return cols;
   return 1;
 }
@@ -835,10 +836,11 @@ mmp_status create_impl(mmp_ctx* ctx, uint32_t n_fibers, const mmp_params* params
   s->batch.se = s->ntab * MN;
   s->batch.ss = (size_t)P.rk.s * MN;
   s->products = sums_products(P, s->use_fused);
+  for (const Problem& Pf : s->fib) s->need_im = s->need_im || (s->products && Pf.need_im);
+  const int chunk_lines = colstage_chunk_lines(P, s->need_im);  // (0 beyond the column-stage kernels' sizes)
   // Raman off: the column-stage gather takes the fields from the heads and returns sigma in one kernel; the
   // three separate passes measured 78.7 against 50.6 us per step at 6 modes, NT = 16384
-  s->kerr_cols = s->products && !P.raman && P.N1 == 64 && (int)P.M <= colstage_max_modes() &&
-                 !(opt.flags & MMP_FLAG_SEPARATE_COLUMNS);
+  s->kerr_cols = s->products && !P.raman && P.N1 == 64 && chunk_lines > 0 && !(opt.flags & MMP_FLAG_SEPARATE_COLUMNS);
   const bool compact = (s->use_fused || s->products) && P.parity;
   s->slots.parity = compact && s->mixed ? 1 : 0;
   s->batch.sq = coupling_block_size(P, s->use_fused);
@@ -1008,7 +1010,7 @@ mmp_status create_impl(mmp_ctx* ctx, uint32_t n_fibers, const mmp_params* params
       s->slots.chunk_line = d_cl;
       s->slots.chunk_slot = d_cs;
       s->slots.slot_meta = d_meta;
-      if (st == MMP_OK) A(install_lines(s, colstage_lines_per_chunk(M)));
+      if (st == MMP_OK) A(install_lines(s, chunk_lines));
       // eight gather wavefronts from 4 to 6 modes (two per SIMD hide the slot loop's LDS latency);
       // below 4 modes a column has at most 6 Raman lines and 9 slots, which four wavefronts cover
       // (measured, 29 fibers of 3 modes at NT = 16384: 71 us with eight, 38 us with four)
@@ -1038,9 +1040,8 @@ mmp_status create_impl(mmp_ctx* ctx, uint32_t n_fibers, const mmp_params* params
       s->fused.chunk_line = d_cl;
       s->fused.steps = d_steps;
       s->fused.parity = compact ? 1 : 0;
-      for (const Problem& Pf : s->fib) s->need_im = s->need_im || Pf.need_im;
-      if (st == MMP_OK) A(install_lines(s, s->use_fused || s->kerr_cols ? colstage_lines_per_chunk(M)
-                                                                    : gather_products_lines(M, P.parity)));
+      if (st == MMP_OK)
+        A(install_lines(s, s->use_fused || s->kerr_cols ? chunk_lines : gather_products_lines(M, P.parity)));
       s->fused.cols = gather_cols(s);
       s->fused.waves = gather_waves(s);
     }
@@ -1150,7 +1151,8 @@ bool plan_valid(const mmp_solver* s, const ColPlan& c) {
     if (c.hi || c.mf) return false;
     if (c.waves != 4 && !((c.waves == 8 || (c.waves == 12 && c == current_plan(s))) && c.cols == 1)) return false;
     if (!colstage_cols_ok(M, c.cols) || s->g.N2 % c.cols ||
-        colstage_products_lds_bytes(M, c.cols, std::min(c.lines, s->fused.n_lines), s->fused.stride) > kColStageLds)
+        colstage_products_lds_bytes(M, c.cols, std::min(c.lines, s->fused.n_lines), s->fused.stride, s->P.parity) >
+            kColStageLds)
       return false;
     if (c.waves == 8 && M <= 4 && s->fused.parity && c.lines < s->fused.n_lines) return false;  // one chunk
   }
@@ -1759,8 +1761,11 @@ mmp_status mmp_fiber_load(mmp_solver* s, uint32_t f, const mmp_params* params) {
     if (s->products && Pf.need_im && !s->need_im) {
       // the first fiber whose couplings need the Im products: the step takes their lines too (the other
       // fibers' Im coefficients are zero, and their Re products' arithmetic stays the same)
+      int lines = s->chunk_lines;
+      if (s->use_fused || s->kerr_cols) lines = std::min(lines, colstage_chunk_lines(s->P, true));
+      if (lines < 1) return fail(MMP_ERR_UNSUPPORTED, "the fiber's couplings do not fit the batch's kernels");
       s->need_im = true;
-      MMP_TRY(install_lines(s, s->chunk_lines));
+      MMP_TRY(install_lines(s, lines));
       if (s->kerr_cols || (s->use_fused && !plan_valid(s, current_plan(s)))) {  // more lines than the workgroup's LDS holds at these columns
         s->fused.cols = gather_cols(s);
         s->fused.waves = gather_waves(s);

@@ -8,8 +8,9 @@ import pytest
 import oracle_binding as ob
 from gpu_util import note, require_device
 from mm_propagation_amd import _capi, configs
+from mm_propagation_amd.batch import MultimodePropagationBatch
 from mm_propagation_amd.problem import Sparse3DArray
-from mm_propagation_amd.solver import MultimodePropagationGPU_RamanON
+from mm_propagation_amd.solver import MultimodePropagationGPU_RamanOFF, MultimodePropagationGPU_RamanON
 
 pytestmark = pytest.mark.gpu
 
@@ -42,6 +43,18 @@ def partial_pairs(sp, both):
     return with_lists(sp, entries)
 
 
+def full(sp, symmetric, seed=11):
+    """Every (k, l, m): no parity structure; symmetric: equal values at (l, m) and (m, l)."""
+    out = with_lists(sp, lambda p: [(k, l, m) for k in range(sp.n_modes) for l in range(sp.n_modes) for m in range(sp.n_modes)])
+    rng = np.random.default_rng(seed)
+    for q in out.coupling_coefficients:
+        values = configs.SR * rng.uniform(-0.5, 1.0, (sp.n_modes,) * 3)
+        for i, e in enumerate(q):
+            k, l, m = e.index
+            q.resetValue(i, values[(k, min(l, m), max(l, m)) if symmetric else (k, l, m)])
+    return out
+
+
 def check(solver, sp, steps, decode, bar):
     solver.computeLawsonRK(steps)
     got = solver.getResult()
@@ -64,3 +77,39 @@ def test_later_chunks_with_more_lines_than_the_first(M, both, flags):
     assert s.info()["gather_chunks"] > 1
     check(s, sp, 5, 1, 1e-6)
     s.close()
+
+
+@pytest.mark.parametrize("raman", [True, False])
+@pytest.mark.parametrize("M", [5, 6, 7])
+def test_full_lists_without_parity_structure(M, raman):
+    """At 6 modes all 36 products' 18 lines, 19 steps of coefficients and sigma in rows of its own pass the 64 KB
+    of the FP64 column gather's workgroup."""
+    require_device()
+    sp = full(configs.grin_fiber(M=M, nt=4096, power_range=(1.0, 100.0), seed=3), symmetric=False)
+    cls = MultimodePropagationGPU_RamanON if raman else MultimodePropagationGPU_RamanOFF
+    for decode in (0, 1):
+        note(f"case full list M={M} raman={raman} decode={decode}")
+        s = cls(sp, pair_decode=decode)
+        check(s, sp, 5, decode, 1e-12)
+        s.close()
+
+
+@pytest.mark.parametrize("fibers", [3, 32])
+def test_a_general_fiber_joins_a_symmetric_batch_without_parity_structure(fibers):
+    """6 modes: 11 lines before the load and 18 after; every fiber equals itself alone bit for bit (32 fibers:
+    2048 columns, two a workgroup before)."""
+    require_device()
+    base = [configs.grin_fiber(M=6, nt=4096, fiber_length=0.5 + 0.01 * i, seed=20 + i, power_range=(1.0, 100.0)) for i in range(3)]
+    sps = [full(sp, symmetric=True, seed=i) for i, sp in enumerate(base)]
+    general = full(base[0], symmetric=False, seed=9)
+    note(f"case general fiber into a symmetric batch without parity, {fibers} fibers")
+    b = MultimodePropagationBatch([sps[i % 3] for i in range(fibers)])
+    b.advance(3)
+    b.load(1, general)
+    b.advance(3)
+    for f, sp, steps in ((0, sps[0], 6), (2, sps[2], 6), (1, general, 3)):
+        s = MultimodePropagationGPU_RamanON(sp)
+        s.computeLawsonRK(steps)
+        assert np.array_equal(b.result(f), s.getResult()), f
+        s.close()
+    b.close()

@@ -133,3 +133,32 @@ def test_mixed_precision_plan_holds_no_lawson_tables():
     fp64 = plan.plan(sp, pair_decode=1)["device_bytes"]
     mixed = plan.plan(sp, pair_decode=1, precision=MIXED)["device_bytes"]
     assert fp64 - mixed >= 7 * 16 * M * nt
+
+
+@pytest.mark.parametrize("decode", [0, 1])
+@pytest.mark.parametrize("kind", ["parity", "general", "none"])
+@pytest.mark.parametrize("M", range(1, 17))
+def test_column_gather_fits_its_workgroup(M, kind, decode):
+    """The FP64 column gather's workgroup holds, in 64 KB of LDS, rows of 72 complex values (1152 bytes):
+    the fields' in eights, a chunk's lines in eights and two sigma rows a mode (up to 6 modes, without parity
+    structure up to 5; beyond, sigma takes the lines' rows), and up to 6 modes 16 coefficients a mode and step with 4 steps spare. Steps: 16 /
+    (M or, with parity, ceil(M/2), padded to 4, 8 or 16) products each, at most 3 more where segments share one,
+    over M(M+1)/2 products (parity: couplings symmetric in the pair) or M^2."""
+    sp = configs.grin_fiber(M=M, nt=4096, symmetric=kind == "parity")
+    if kind == "none":
+        for p, q in enumerate(sp.coupling_coefficients):
+            for k in range(M):
+                for l in range(M):
+                    for m in range(M):
+                        q.addNonZeroValue(configs.NonZeroValue((k, l, m), configs.SR * (1 + p + k + 2 * l + 3 * m)))
+    lines = plan.plan(sp, pair_decode=decode)["chunk_lines"]
+    products = M * (M + 1) // 2 if kind == "parity" and decode == 1 else M * M
+    assert lines >= 8
+    rows = (min(lines, (products + 1) // 2) + 7) // 8 * 8
+    row = M if kind == "none" else (M + 1) // 2
+    steps = -(-M * M // (16 // (4 if row <= 4 else 8 if row <= 8 else 16))) + (1 if kind == "none" else 3)
+    lds = ((M + 7) // 8 * 8 + (rows + 2 * M if M <= (5 if kind == "none" else 6) else max(rows, 2 * M))) * 1152
+    if M <= 6:
+        lds += (M * steps + 4) * 128
+    assert lds <= 65536, (lines, lds)
+    assert lines == (16 if M <= 4 else 24 if M <= 6 else 40)
