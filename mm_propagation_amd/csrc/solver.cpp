@@ -1147,14 +1147,16 @@ bool plan_valid(const mmp_solver* s, const ColPlan& c) {
     if (c.mf && (c.waves != 4 || c.hi || (s->opt.flags & MMP_FLAG_NO_MATRIX_CORES) || !mf_ok)) return false;
     if (!c.mf && mf_ok && (s->opt.flags & MMP_FLAG_MATRIX_CORES)) return false;
   } else {
-    // (a 12-wavefront plan is a default only; it needs its one chunk)
     if (c.hi || c.mf) return false;
-    if (c.waves != 4 && !((c.waves == 8 || (c.waves == 12 && c == current_plan(s))) && c.cols == 1)) return false;
+    // (12 wavefronts: the instances of 5 and 6 modes with parity structure)
+    const bool twelve = c.waves == 12 && (M == 5 || M == 6) && s->fused.parity;
+    if (c.waves != 4 && !((c.waves == 8 || twelve) && c.cols == 1)) return false;
     if (!colstage_cols_ok(M, c.cols) || s->g.N2 % c.cols ||
         colstage_products_lds_bytes(M, c.cols, std::min(c.lines, s->fused.n_lines), s->fused.stride, s->P.parity) >
             kColStageLds)
       return false;
-    if (c.waves == 8 && M <= 4 && s->fused.parity && c.lines < s->fused.n_lines) return false;  // one chunk
+    // a wavefront per mode and parity class takes its lines in one chunk
+    if (s->fused.parity && c.waves >= 2 * M && c.lines < s->fused.n_lines) return false;
   }
   if (c.columns != 1 && c.columns != 2 && c.columns != 4) return false;
   if (s->g.N2 % c.columns || colstage_pairs_lds_bytes(M, c.columns, s->mixed) > kColStagePairsLds) return false;

@@ -86,3 +86,27 @@ def test_tuning_leaves_no_fiber_parked():
     b.computeLawsonRK(8)
     assert b.info(1)["halted"] == 1 and b.info(0)["halted"] == 0
     b.close()
+
+
+@pytest.mark.parametrize("M", [5, 6])
+def test_general_couplings_tune_from_twelve_wavefronts(M):
+    """5 and 6 modes with parity structure whose couplings need all products start from 12 gather wavefronts;
+    that plan stays a valid choice once the tuner has installed others, and for a later solver."""
+    require_device()
+    sp = configs.grin_fiber(M=M, nt=4096, power_range=(1.0, 100.0), seed=17)
+    plain = MultimodePropagationGPU_RamanON(sp, pair_decode=1)
+    assert plain.info()["gather_waves"] == 12
+    plain.close()
+    results = []
+    for k in range(2):
+        note(f"case autotune general couplings M={M}, solver {k}")
+        s = MultimodePropagationGPU_RamanON(sp, pair_decode=1, flags=_capi.MMP_FLAG_AUTOTUNE)
+        assert s.info()["tuned"] == 1 and s.info()["gather_waves"] in (4, 8, 12)
+        s.computeLawsonRK(10)
+        results.append(s.getResult())
+        s.close()
+    assert np.array_equal(results[0], results[1])
+    o = ob.Oracle(sp, pair_decode=1)
+    o.compute_lawson_rk(10)
+    assert np.all(configs.rel_l2_per_mode(results[0], o.get_result()) <= 1e-12)
+    o.close()
