@@ -1193,13 +1193,13 @@ mmp_status advance_impl(mmp_solver* s, uint32_t n);
 // pass's columns per workgroup and line groups, then the line order into the Raman row pass.
 // Every candidate runs one warm-up graph and two
 // timed graphs of steps on this solver's own fibers (HIP events); the fastest is kept and
-// remembered per structure (modes, samples, stages, slots, lines, parity, precision, fibers) for
-// later solvers of the process. The fibers' spectra are saved first and restored after; z, steps,
+// remembered per structure (modes, samples, stages, slots, lines, parity, precision, fibers, the FP64
+// gather's steps: its LDS grows with them, and the matrix-core flags) for later solvers of the process. The fibers' spectra are saved first and restored after; z, steps,
 // Lawson tables and any fiber the device parked during the runs are reset, so the solver ends as
 // created.
 struct TuneKey {
-  uint32_t v[8];
-  bool operator<(const TuneKey& o) const { return std::lexicographical_compare(v, v + 8, o.v, o.v + 8); }
+  uint32_t v[10];
+  bool operator<(const TuneKey& o) const { return std::lexicographical_compare(v, v + 10, o.v, o.v + 10); }
 };
 std::mutex g_tune_mutex;
 std::map<TuneKey, ColPlan> g_tune_cache;
@@ -1274,11 +1274,12 @@ mmp_status tune_passes(mmp_solver* s, hipEvent_t e0, hipEvent_t e1, ColPlan& bes
 mmp_status autotune(mmp_solver* s) {
   const Problem& P = s->P;
   const TuneKey key{{P.M, P.N, (uint32_t)P.rk.s, P.P, (uint32_t)s->fused.n_lines, (uint32_t)P.parity,
-                     s->mixed ? 1u : 0u, s->F}};
+                     s->mixed ? 1u : 0u, s->F, (uint32_t)s->fused.stride,
+                     s->opt.flags & (MMP_FLAG_MATRIX_CORES | MMP_FLAG_NO_MATRIX_CORES)}};
   {
     std::lock_guard<std::mutex> lock(g_tune_mutex);
     auto it = g_tune_cache.find(key);
-    if (it != g_tune_cache.end()) {
+    if (it != g_tune_cache.end() && plan_valid(s, it->second)) {
       MMP_TRY(apply_colstage_plan(s, it->second));
       s->tuned = true;
       return MMP_OK;

@@ -110,3 +110,26 @@ def test_general_couplings_tune_from_twelve_wavefronts(M):
     o.compute_lawson_rk(10)
     assert np.all(configs.rel_l2_per_mode(results[0], o.get_result()) <= 1e-12)
     o.close()
+
+
+@pytest.mark.parametrize("precision", [_capi.MMP_PRECISION_FP64, _capi.MMP_PRECISION_MIXED])
+def test_a_choice_serves_only_solvers_it_fits(precision):
+    """6 modes, 2048 columns, the same slots and lines: with the reference decode the FP64 coefficients take 16
+    steps instead of 12, and two columns of 16 lines (65,024 bytes of LDS with 12) no longer fit; and a mixed
+    solver without matrix cores after one that may have chosen them."""
+    require_device()
+    fib = [configs.grin_fiber(M=6, nt=8192, seed=40 + i, power_range=(1.0, 100.0)) for i in range(2)]
+    note(f"case autotune choices precision={precision}")
+    for decode, flags in ((1, 0), (0, 0), (1, _capi.MMP_FLAG_NO_MATRIX_CORES), (1, 0)):
+        t = MultimodePropagationBatch([fib[f % 2] for f in range(16)], pair_decode=decode, precision=precision,
+                                      flags=flags | _capi.MMP_FLAG_AUTOTUNE)
+        assert t.info(0)["tuned"] == 1
+        assert not (flags and t.info(0)["gather_matrix_cores"])
+        u = MultimodePropagationBatch([fib[f % 2] for f in range(2)], pair_decode=decode, precision=precision, flags=flags)
+        t.computeLawsonRK(4)
+        u.computeLawsonRK(4)
+        tol = 1e-12 if precision == _capi.MMP_PRECISION_FP64 else 1e-6
+        for f in range(2):
+            assert np.all(configs.rel_l2_per_mode(t.result(14 + f), u.result(f)) <= tol)
+        t.close()
+        u.close()
