@@ -1748,6 +1748,23 @@ mmp_status mmp_fiber_set_state(mmp_solver* s, uint32_t f, const double* psi) {
   return MMP_OK;
 }
 
+// Makes the solver of one fiber anew for another one, in its place: its graphs, and a group's that hold it, are
+// stale; the profile's totals stay. On a failure the solver stays as it was.
+static mmp_status remake_solver(mmp_solver* s, const mmp_params* params) {
+  MMP_TRY(drain_profile(s));
+  mmp_solver* fresh = nullptr;
+  const mmp_options opt = s->opt;
+  MMP_TRY(create_impl(s->ctx, 1, params, &opt, &fresh));
+  fresh->plan_id = s->plan_id + 1;
+  fresh->kernel_names.swap(s->kernel_names);
+  fresh->kernel_bytes.swap(s->kernel_bytes);
+  fresh->kernel_ms.swap(s->kernel_ms);
+  fresh->kernel_count.swap(s->kernel_count);
+  std::swap(*s, *fresh);
+  release(fresh);
+  return MMP_OK;
+}
+
 mmp_status mmp_fiber_load(mmp_solver* s, uint32_t f, const mmp_params* params) {
   MMP_TRY(check_fiber(s, f));
   if (!params) return fail(MMP_ERR_INVALID_ARGUMENT, "params is required");
@@ -1761,6 +1778,8 @@ mmp_status mmp_fiber_load(mmp_solver* s, uint32_t f, const mmp_params* params) {
                                             "and pair structure");
     MMP_TRY(set_device(s));
     HIP_TRY(hipStreamSynchronize(s->ctx->stream), "hipStreamSynchronize");  // queued steps read the old fiber
+    // the slots' gathers of the separate passes hold their fiber's lists and mix: made anew
+    if (!s->use_fused && !s->products) return remake_solver(s, params);
     if (s->products && Pf.need_im && !s->need_im) {
       // the first fiber whose couplings need the Im products: the step takes their lines too (the other
       // fibers' Im coefficients are zero, and their Re products' arithmetic stays the same)

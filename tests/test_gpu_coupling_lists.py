@@ -8,9 +8,9 @@ import pytest
 import oracle_binding as ob
 from gpu_util import note, require_device
 from mm_propagation_amd import _capi, configs
-from mm_propagation_amd.batch import MultimodePropagationBatch
+from mm_propagation_amd.batch import MultimodePropagationBatch, SolverGroup
 from mm_propagation_amd.problem import Sparse3DArray
-from mm_propagation_amd.solver import MultimodePropagationGPU_RamanOFF, MultimodePropagationGPU_RamanON
+from mm_propagation_amd.solver import Context, MultimodePropagationGPU_RamanOFF, MultimodePropagationGPU_RamanON
 
 pytestmark = pytest.mark.gpu
 
@@ -113,3 +113,53 @@ def test_a_general_fiber_joins_a_symmetric_batch_without_parity_structure(fibers
         assert np.array_equal(b.result(f), s.getResult()), f
         s.close()
     b.close()
+
+
+def one_k_per_pair(sp):
+    """Every pair (l, m), one coupling each, with the parity structure."""
+    M = sp.n_modes
+    return with_lists(sp, lambda p: [((p + l + m) % 2, l, m) for l in range(M) for m in range(M)])
+
+
+def every_k(sp):
+    """The same pairs in the same order with all their couplings of the parity structure."""
+    M = sp.n_modes
+    return with_lists(sp, lambda p: [(k, l, m) for l in range(M) for m in range(M) for k in range((p + l + m) % 2, M, 2)])
+
+
+def other_fiber(sp, lists):
+    """Another length, pulse width, Raman share, field and couplings; the same structure."""
+    out = lists(configs.grin_fiber(M=sp.n_modes, nt=sp.nt, fiber_length=0.7, t0=0.15, seed=8, power_range=(1.0, 100.0)))
+    out.raman_proportion = 0.25
+    return out
+
+
+@pytest.mark.parametrize("M,nt,precision,raman", [(2, 1024, MIXED, True), (5, 1024, MIXED, False), (13, 512, MIXED, True),
+                                                  (20, 256, MIXED, False), (20, 512, FP64, True), (33, 256, FP64, True),
+                                                  (16, 4096, FP64, False)])
+def test_a_loaded_fiber_brings_its_couplings(M, nt, precision, raman):
+    """A solver of one fiber on the separate passes: the fiber loaded into it, with fewer, more and other couplings,
+    equals itself alone bit for bit, also stepped by a group that was there before."""
+    require_device()
+    base = configs.grin_fiber(M=M, nt=nt, power_range=(1.0, 100.0), seed=4)
+    first, few, many = every_k(base), other_fiber(base, one_k_per_pair), other_fiber(base, every_k)
+    ctx = Context(0)
+    b = MultimodePropagationBatch([first], raman=raman, precision=precision, ctx=ctx)
+    other = MultimodePropagationBatch([first], raman=raman, precision=precision, ctx=Context(0))
+    g = SolverGroup([b, other], ctx)
+    g.advance(3)
+    steps = 0
+    for sp in (few, many, few):
+        note(f"case load M={M} nt={nt} precision={precision} raman={raman}")
+        b.load(0, sp)
+        g.advance(4)
+        steps += 4
+        alone = MultimodePropagationBatch([sp], raman=raman, precision=precision)
+        alone.advance(4)
+        assert np.array_equal(b.result(0), alone.result(0))
+        alone.close()
+    untouched = MultimodePropagationBatch([first], raman=raman, precision=precision)
+    untouched.advance(3 + steps)
+    assert np.array_equal(other.result(0), untouched.result(0))
+    for x in (g, b, other, untouched):
+        x.close()
