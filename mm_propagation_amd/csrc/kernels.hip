@@ -2228,16 +2228,17 @@ hipError_t launch_gather(const Geometry& g, const cpx<W>* U, const cpx<W>* VR, c
   int waves = g.M < 8 ? g.M : 8;
   if ((g.M + waves - 1) / waves > kGatherMaxPW) return hipErrorInvalidValue;
   // A wavefront sums its modes one after the other, so small grids deal the modes to groups of workgroups,
-  // up to one mode a wavefront, while all of them run at once: 256 CUs with the workgroups their LDS
-  // holds, one at 128 KB (FP64 beyond 64 slots and modes), else two. Beyond that each group's own slot mix
-  // costs more than it gives. Steps on one MI355X, us with one group and with the rule's. Mixed: 20 modes, NT =
-  // 1024 (16 tiles) 2307 -> 1174, NT = 4096 2392 -> 1223; 32 modes, NT = 4096 15423 -> 4310; 14 modes, NT = 1024
-  // 835 -> 527; 18 modes, NT = 16384 (256 tiles) 2002 -> 1644 with two, 1873 with three; 20 modes, NT = 65536 (1024
-  // tiles) 8222, two groups 8546; a tenth of the list or less gains too (20 modes, NT = 16384 590 -> 494) or
-  // stays. FP64, 20 modes without parity structure, a tenth of the list: NT = 4096 679 -> 353 (three groups of
-  // 64 tiles), NT = 8192 693 -> 516 with two (598 with three), NT = 16384 748 with one, 854 with two.
+  // up to one mode a wavefront, while tiles x groups stay within 512 in FP32 (two workgroups a CU) and 256 in FP64
+  // (one: up to 128 KB of LDS each). Beyond that each group's own slot mix, and its reading of every field, cost
+  // more than it gives. Steps on one MI355X, us with one group and with the rule's. Mixed: 20 modes, NT = 1024 (16
+  // tiles) 2307 -> 1174, NT = 4096 2392 -> 1223; 32 modes, NT = 4096 15423 -> 4310; 14 modes, NT = 1024 835 -> 527;
+  // 18 modes, NT = 16384 (256 tiles) 2002 -> 1644 with two, 1873 with three; 20 modes, NT = 65536 (1024 tiles)
+  // 8222, two groups 8546; a tenth of the list or less gains too (20 modes, NT = 16384 590 -> 494) or stays. FP64,
+  // 20 modes without parity structure, a tenth of the list: NT = 4096 679 -> 353 (three groups of 64 tiles), NT =
+  // 8192 693 -> 516 with two (598 with three), NT = 16384 748 with one, 854 with two; self pairs alone, NT = 16384
+  // 133 with one, 145 with two.
   const int tiles = g.N / kGatherTS;
-  const int resident = (size_t)a.cap * sizeof(cpx<W>) > 81920 ? 256 : 512;
+  const int resident = sizeof(W) == 8 ? 256 : 512;
   int groups = (g.M + waves - 1) / waves;
   while (groups > 1 && tiles * groups > resident) groups--;
   dim3 grid(g.N / kGatherTS, groups), block(kGatherTS * waves);

@@ -247,6 +247,32 @@ std::vector<double> product_blocks(const Problem& P, const std::vector<double>& 
   return out;
 }
 
+// Whether the gather sums the real products: in FP64 the column stage with Raman always; the separate passes, and
+// without Raman the column kernel in their place, up to 16 coefficients per product and mode (32 modes with the
+// parity structure) unless the list is far from full. The products cost all their coefficients
+// whatever the list holds; the sparse gather its longest list's nonzeros and a mix of every slot; and
+// with Raman both a line for two products or slots (half as many where couplings are symmetric and only the Re
+// products run). Counted in FMAs of a sample: a nonzero 12 (20 up to 64 workgroups of 64 samples, where the
+// sums are a latency), a slot's mix 32, a Raman line's half 256; against the column kernel, which is worse beyond
+// 12 modes than its passes saved, a nonzero 6 and a mix 64. Fitted on 520 lists of 13 to 32 modes at NT = 1024 to
+// 65536: within 1 % of the better one in the mean, 1.2x at worst. One MI355X, us per step, sparse and products: 32
+// modes, NT = 16384, one nonzero a slot, no Raman 367 and 3067; 20 modes, NT = 4096, 3 % of a symmetric
+// list, no Raman 171 and 145; full lists 2995 and 254. Up to 12 modes the products won on every
+// list tried.
+static bool choose_products(const Problem& P, const mmp_options& opt) {
+  const bool separate = opt.flags & MMP_FLAG_SEPARATE_COLUMNS;
+  if (P.mixed) return false;
+  if (P.fused_chunks > 0 && !separate) return true;
+  if (P.n_products() < 1 || !gather_products_ok((int)P.M, P.parity)) return false;
+  if (P.M <= 12) return true;
+  const bool columns = !P.raman && P.N1 == 64 && (int)P.M <= colstage_max_modes() && !separate;
+  double longest = 0.;
+  for (uint32_t p = 0; p < P.M; p++) longest = std::max(longest, (double)(P.off[p + 1] - P.off[p]));
+  const double line = P.raman ? 256. : 0., nonzero = columns ? 6. : (P.N <= 4096 ? 20. : 12.), mix = columns ? 64. : 32.;
+  return P.active_products(P.need_im) * (P.M * (double)colstage_coef_pad((int)P.M, P.parity) + line) <=
+         nonzero * P.M * longest + (mix + line) * P.P;
+}
+
 mmp_status prepare_problem(const mmp_params* in, const mmp_options& opt, Problem& P, std::string& err) {
   if (!in) { err = "params is NULL"; return MMP_ERR_INVALID_ARGUMENT; }
   const uint32_t M = in->n_modes, nt = in->nt, nb = in->n_beta;
@@ -536,6 +562,7 @@ mmp_status prepare_problem(const mmp_params* in, const mmp_options& opt, Problem
   P.kv = P.raman ? 1 - P.fR : 1.;
   P.kr = P.raman ? P.fR * P.T0 : 0.;
   plan_colstage_chunks(P, colstage_chunk_lines(P, P.need_im), P.need_im);
+  P.products = choose_products(P, opt);
   // a stage result N_j needs a stash slot when a stage i > j + 1 reads it
   P.stash_needed.assign(P.rk.s, 0);
   for (int i = 0; i < P.rk.s; i++)

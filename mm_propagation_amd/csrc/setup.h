@@ -72,6 +72,7 @@ struct Problem {
   uint32_t seg_b[4] = {0, 0, 0, 0}, seg_e[4] = {0, 0, 0, 0};
   uint32_t seg_products() const { return seg_e[0] - seg_b[0] + seg_e[1] - seg_b[1] + seg_e[2] - seg_b[2] + seg_e[3] - seg_b[3]; }
   bool need_im = false;                             // some Q1 - Q2 is not zero
+  bool products = false;                            // the gather sums the real products (choose_products)
   // chunks of Raman lines (0 chunks: the column-stage kernels do not apply) and the largest chunk
   int fused_chunks = 0, fused_max_lines = 0;
   std::vector<uint32_t> fused_line;                 // [fused_chunks + 1]

@@ -515,19 +515,14 @@ void release(mmp_solver* s) {
 // mixed-precision stage heads form E_u from Im L and the fiber's z where they use it.
 bool lawson_tables(bool mixed) { return !mixed; }
 
-// FP64 gathers sum the real products: the column-stage one always, the separate one up to 16
-// coefficients per product and mode (32 modes with the parity structure).
-bool sums_products(const Problem& P, bool fused) {
-  return !P.mixed && (fused || (P.n_products() > 0 && gather_products_ok((int)P.M, P.parity)));
-}
 // Dense coupling blocks exist (else the sparse gather's lists serve).
 bool coupling_blocks(const Problem& P, bool fused) {
-  return fused || sums_products(P, fused) || (P.mixed && dense_gather_chunk((int)P.M) > 0);
+  return fused || P.products || (P.mixed && dense_gather_chunk((int)P.M) > 0);
 }
 
 // Coupling coefficients of one fiber: of the FP64 gathers' products, or of the slots.
 size_t coupling_block_size(const Problem& P, bool fused) {
-  if (sums_products(P, fused)) return (size_t)P.M * P.product_steps() * 16;
+  if (P.products) return (size_t)P.M * P.product_steps() * 16;
   return (size_t)P.P * P.M * (fused && P.parity ? (P.M + 1) / 2 : P.M);
 }
 // Line descriptors: of the Raman lines, where the gather sums the products of these (two a line, Raman on
@@ -548,7 +543,7 @@ size_t planned_device_bytes(const Problem& P, const mmp_options& opt, size_t F) 
   if (lawson_tables(mixed)) b += 16 * MN * F * (2 * P.c_unique.size() + 1);
   if (any_stash) b += 16 * (size_t)P.rk.s * MN * F;
   if (P.raman) b += (mixed ? 8 : 16) * c(L) * P.N * F + 16 * (size_t)P.N * F + 8 * (size_t)P.N;
-  const bool fused = P.fused_chunks > 0 && !(opt.flags & MMP_FLAG_SEPARATE_COLUMNS), products = sums_products(P, fused);
+  const bool fused = P.fused_chunks > 0 && !(opt.flags & MMP_FLAG_SEPARATE_COLUMNS), products = P.products;
   const size_t LP = product_lines(P, products);
   b += 8 * c(LP);
   if (!products) b += 4 * c(P.coff.size()) + 4 * c(P.nnz) + 8 * c(P.nnz) + 4 * 4 * c(P.P);  // the sparse gather's lists
@@ -835,7 +830,7 @@ mmp_status create_impl(mmp_ctx* ctx, uint32_t n_fibers, const mmp_params* params
   s->batch.sl = conv_n;
   s->batch.se = s->ntab * MN;
   s->batch.ss = (size_t)P.rk.s * MN;
-  s->products = sums_products(P, s->use_fused);
+  s->products = P.products;
   for (const Problem& Pf : s->fib) s->need_im = s->need_im || (s->products && Pf.need_im);
   const int chunk_lines = colstage_chunk_lines(P, s->need_im);  // (0 beyond the column-stage kernels' sizes)
   // Raman off: the column-stage gather takes the fields from the heads and returns sigma in one kernel; the
@@ -1778,8 +1773,9 @@ mmp_status mmp_fiber_load(mmp_solver* s, uint32_t f, const mmp_params* params) {
                                             "and pair structure");
     MMP_TRY(set_device(s));
     HIP_TRY(hipStreamSynchronize(s->ctx->stream), "hipStreamSynchronize");  // queued steps read the old fiber
-    // the slots' gathers of the separate passes hold their fiber's lists and mix: made anew
-    if (!s->use_fused && !s->products) return remake_solver(s, params);
+    // the slots' gathers of the separate passes hold their fiber's lists and mix: made anew, as a solver is for a
+    // fiber that takes the other gather
+    if (!s->use_fused && !(s->products && Pf.products)) return remake_solver(s, params);
     if (s->products && Pf.need_im && !s->need_im) {
       // the first fiber whose couplings need the Im products: the step takes their lines too (the other
       // fibers' Im coefficients are zero, and their Re products' arithmetic stays the same)

@@ -163,3 +163,20 @@ def test_a_loaded_fiber_brings_its_couplings(M, nt, precision, raman):
     assert np.array_equal(other.result(0), untouched.result(0))
     for x in (g, b, other, untouched):
         x.close()
+
+
+@pytest.mark.parametrize("raman", [True, False])
+@pytest.mark.parametrize("M,nt,lists", [(12, 1024, "own"), (13, 1024, "own"), (13, 4096, "one"), (16, 4096, "own"), (16, 1024, "one"),
+                                        (16, 4096, "full"), (20, 1024, "own"), (20, 1024, "one"), (32, 256, "one")])
+def test_lists_on_both_sides_of_the_gathers_choice(M, nt, lists, raman):
+    """FP64 on the separate passes (and without Raman the column kernel): self pairs alone, one coupling a pair
+    and the full list, on either side of the line between the sparse sum and the products."""
+    require_device()
+    sp = configs.grin_fiber(M=M, nt=nt, power_range=(1.0, 100.0), seed=6)
+    if lists != "full":
+        sp = with_lists(sp, lambda p: [(p, l, l) for l in range(M)]) if lists == "own" else one_k_per_pair(sp)
+    cls = MultimodePropagationGPU_RamanON if raman else MultimodePropagationGPU_RamanOFF
+    note(f"case gather choice M={M} nt={nt} lists={lists} raman={raman}")
+    s = cls(sp)
+    check(s, sp, 3, 1, 1e-12)
+    s.close()
