@@ -252,8 +252,8 @@ std::vector<double> product_blocks(const Problem& P, const std::vector<double>& 
 // parity structure) unless the list is far from full. The products cost all their coefficients
 // whatever the list holds; the sparse gather its longest list's nonzeros and a mix of every slot; and
 // with Raman both a line for two products or slots (half as many where couplings are symmetric and only the Re
-// products run). Counted in FMAs of a sample: a nonzero 12 (20 up to 64 workgroups of 64 samples, where the
-// sums are a latency), a slot's mix 32, a Raman line's half 256; against the column kernel, which is worse beyond
+// products run). Counted in FMAs of a sample: a nonzero 12 and a slot's mix 32 (24 and 16 up to 64 tiles of 64
+// samples, where the sums are a latency), a Raman line's half 256; against the column kernel, which is worse beyond
 // 12 modes than its passes saved, a nonzero 6 and a mix 64. Fitted on 520 lists of 13 to 32 modes at NT = 1024 to
 // 65536: within 1 % of the better one in the mean, 1.2x at worst. One MI355X, us per step, sparse and products: 32
 // modes, NT = 16384, one nonzero a slot, no Raman 367 and 3067; 20 modes, NT = 4096, 3 % of a symmetric
@@ -268,7 +268,9 @@ static bool choose_products(const Problem& P, const mmp_options& opt) {
   const bool columns = !P.raman && P.N1 == 64 && (int)P.M <= colstage_max_modes() && !separate;
   double longest = 0.;
   for (uint32_t p = 0; p < P.M; p++) longest = std::max(longest, (double)(P.off[p + 1] - P.off[p]));
-  const double line = P.raman ? 256. : 0., nonzero = columns ? 6. : (P.N <= 4096 ? 20. : 12.), mix = columns ? 64. : 32.;
+  const bool small = P.N <= 4096;
+  const double line = P.raman ? 256. : 0.;
+  const double nonzero = columns ? 6. : (small ? 24. : 12.), mix = columns ? 64. : (small ? 16. : 32.);
   return P.active_products(P.need_im) * (P.M * (double)colstage_coef_pad((int)P.M, P.parity) + line) <=
          nonzero * P.M * longest + (mix + line) * P.P;
 }
