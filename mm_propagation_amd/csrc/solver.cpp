@@ -123,6 +123,7 @@ struct mmp_solver {
   double* qdense = nullptr;
   std::vector<uint32_t> step_table;  // the vector gather's steps, whose order the coupling blocks follow
   bool loaded = false;       // every fiber's data is on the device
+  bool lines_ok = true;      // lines, steps and coupling blocks on the device are those of one plan
   bool need_im = false;      // the step runs the Im products (a fiber's couplings need them)
   uint32_t plan_id = 0;      // counts changes of the kernels' plan: graphs captured before are stale
   // work arrays of the step in the work precision (the FP64 buffers above in FP64 mode)
@@ -362,7 +363,15 @@ mmp_status enqueue_step_w(mmp_solver* s) {
   return MMP_OK;
 }
 
-mmp_status enqueue_step(mmp_solver* s) { return s->mixed ? enqueue_step_w<float>(s) : enqueue_step_w<double>(s); }
+// A load that failed half-way left lines and coupling blocks of two plans.
+mmp_status check_lines(const mmp_solver* s) {
+  return s->lines_ok ? MMP_OK : fail(MMP_ERR_STATE, "a fiber's load failed half-way: load it again");
+}
+
+mmp_status enqueue_step(mmp_solver* s) {
+  MMP_TRY(check_lines(s));
+  return s->mixed ? enqueue_step_w<float>(s) : enqueue_step_w<double>(s);
+}
 
 mmp_status capture_steps(mmp_solver* s, int steps, hipGraph_t* graph_out, hipGraphExec_t* exec_out) {
   hipStream_t st = s->ctx->stream;
@@ -654,6 +663,8 @@ mmp_status upload_couplings(mmp_solver* s, uint32_t f, const Problem& Pf) {
 // products, or of all products where s->need_im, and the products' steps; mixed: the slots'.
 mmp_status install_lines(mmp_solver* s, int max_lines) {
   Problem& P = s->P;
+  const bool partial = !s->lines_ok;  // an earlier call ended half-way
+  s->lines_ok = false;
   if (!s->use_fused) plan_product_chunks(P, max_lines, s->need_im);
   else if (!plan_colstage_chunks(P, max_lines, s->need_im))
     return fail(MMP_ERR_INVALID_ARGUMENT, "no chunk plan for these limits");
@@ -670,6 +681,7 @@ mmp_status install_lines(mmp_solver* s, int max_lines) {
     sa.max_chunk_slots = P.fused_max_slots;
     sa.first_lines = (int)P.fused_line[1];
     sa.first_slots = (int)P.fused_slot[1];
+    s->lines_ok = true;
     return MMP_OK;
   }
   ProductArgs& fa = s->fused;
@@ -687,7 +699,7 @@ mmp_status install_lines(mmp_solver* s, int max_lines) {
   fa.n_steps = (int)table.size();
   fa.odd_step = 0;
   while (fa.odd_step < fa.n_steps && !(table[fa.odd_step] >> 28 & 1u)) fa.odd_step++;
-  const bool changed = table != s->step_table;
+  const bool changed = partial || table != s->step_table;
   s->step_table = table;
   table.resize(step_table_size(P), 0u);
   MMP_TRY(upload(s, const_cast<uint32_t*>(fa.steps), table.data(), table.size() * 4));
@@ -695,6 +707,7 @@ mmp_status install_lines(mmp_solver* s, int max_lines) {
   // the coupling blocks follow the steps' order
   if (changed && s->loaded)
     for (uint32_t f = 0; f < s->F; f++) MMP_TRY(upload_couplings(s, f, s->fib[f]));
+  s->lines_ok = true;
   return MMP_OK;
 }
 
@@ -1335,6 +1348,7 @@ void account_steps(mmp_solver* s, uint32_t n) {
 
 mmp_status advance_impl(mmp_solver* s, uint32_t n) {
   MMP_TRY(set_device(s));
+  MMP_TRY(check_lines(s));
   if (n > 0 && s->chain) MMP_TRY(enqueue_head(s, 0));  // stage 0 of the first step
   uint32_t left = n;
   if (n > 0) MMP_TRY(build_graph(s));
@@ -1776,20 +1790,21 @@ mmp_status mmp_fiber_load(mmp_solver* s, uint32_t f, const mmp_params* params) {
     // the slots' gathers of the separate passes hold their fiber's lists and mix: made anew, as a solver is for a
     // fiber that takes the other gather
     if (!s->use_fused && !(s->products && Pf.products)) return remake_solver(s, params);
-    if (s->products && Pf.need_im && !s->need_im) {
+    if (s->products && ((Pf.need_im && !s->need_im) || !s->lines_ok)) {
       // the first fiber whose couplings need the Im products: the step takes their lines too (the other
-      // fibers' Im coefficients are zero, and their Re products' arithmetic stays the same)
+      // fibers' Im coefficients are zero, and their Re products' arithmetic stays the same). The graphs go
+      // first: after a failure nothing steps until a load has gone through
       int lines = s->chunk_lines;
       if (s->use_fused || s->kerr_cols) lines = std::min(lines, colstage_chunk_lines(s->P, true));
       if (lines < 1) return fail(MMP_ERR_UNSUPPORTED, "the fiber's couplings do not fit the batch's kernels");
+      s->plan_id++;
+      drop_graph(s);
       s->need_im = true;
       MMP_TRY(install_lines(s, lines));
       if (s->kerr_cols || (s->use_fused && !plan_valid(s, current_plan(s)))) {  // more lines than the workgroup's LDS holds at these columns
         s->fused.cols = gather_cols(s);
         s->fused.waves = gather_waves(s);
       }
-      s->plan_id++;
-      drop_graph(s);
       MMP_TRY(build_graph(s));
     }
     MMP_TRY(load_fiber(s, f, Pf));
