@@ -836,9 +836,9 @@ struct ColStageCfg {
 
 int colstage_max_modes() { return kColStageMaxM; }
 
-// Columns per C2 workgroup: one, two up to 10 modes (a wavefront pair per column; beyond, the sums'
-// registers leave one wavefront per SIMD), four up to 4 modes in the vector form
-constexpr int kColStageMaxM2 = 10, kColStageMaxM4 = 4;
+// Columns per FP64 C2 workgroup: one, two up to 6 modes (a wavefront pair per column; at 7 and 8 modes two were
+// 4 and 7 % slower than one on every grid, beyond the lines do not fit), four up to 2 modes (beyond they do not fit)
+constexpr int kColStageMaxM2 = 6, kColStageMaxM4 = 2;
 bool colstage_cols_ok(int M, int cols) {
   return cols == 1 || (cols == 2 && M <= kColStageMaxM2) || (cols == 4 && M <= kColStageMaxM4);
 }
@@ -2332,7 +2332,7 @@ static hipError_t c2_launch(const Geometry& g, const Twiddles& tw, const cd* U, 
 template <int M, bool PAR, bool RAMAN>
 static hipError_t c2_variant(const Geometry& g, const Twiddles& tw, const cd* U, const cd* conv, cd* yout,
                              const ProductArgs& fa, const double* Qp, double scale, const Batch& b, int F, hipStream_t s) {
-  if constexpr (RAMAN && M <= kColStageMaxM4) {  // (without Raman one fiber's columns, at most 1024)
+  if constexpr (RAMAN && M <= kColStageMaxM4) {  // (without Raman one fiber's columns: one a workgroup)
     if (fa.cols == 4) return c2_launch<M, 4, 4, PAR, RAMAN>(g, tw, U, conv, yout, fa, Qp, scale, b, F, s);
   }
   if constexpr (RAMAN && M <= kColStageMaxM2) {

@@ -567,12 +567,15 @@ size_t planned_device_bytes(const Problem& P, const mmp_options& opt, size_t F) 
   return b;
 }
 
-// FP64: wavefronts of the column-stage gather's workgroup. On grids that leave a CU one or two workgroups
-// it takes eight (12 at 5 and 6 modes where the Im products double the sums, `both`): a wavefront per
-// mode, up to 4 modes (12: 6) one per mode and parity class. Larger grids hide the sums' latency with
-// other workgroups.
+// FP64: wavefronts of the column-stage gather's workgroup of one column. On grids of one workgroup a CU or less it
+// takes eight (12 at 5 and 6 modes where the Im products double the sums, `both`): a wavefront per mode, up to
+// 4 modes (12: 6) one per mode and parity class. Larger grids hide the sums' latency with other workgroups, up
+// to 12 modes; beyond, four wavefronts have up to four modes each. One MI355X, us per step with four and eight
+// (and 12), all products: 256 columns, 3 modes 91.9 and 89.4, 5 modes 109.3 and 106.9 (103.7), 10 modes 233 and 222; 512
+// columns, 3 modes 104.8 and 110.6, 5 modes 139 and 150 (145), 10 modes 372 and 432, 13 modes (symmetric) 481 and
+// 435; 1024 columns, 10 modes 745 and 868, 13 modes 955 and 864; 4096 columns, 16 modes 4809 and 4229.
 int products_waves(int M, long columns, bool both) {
-  if (columns > 512) return 4;
+  if (M <= 12 && columns > 256) return 4;
   return (M == 5 || M == 6) && both ? 12 : 8;
 }
 
@@ -711,12 +714,18 @@ mmp_status install_lines(mmp_solver* s, int max_lines) {
   return MMP_OK;
 }
 
-// FP64: columns per gather workgroup for the solver's grid.
+// FP64: columns per gather workgroup for the solver's grid: two on 1024 columns and more, four on 2048, where the
+// sizes and the LDS allow them. Neighbouring columns share the cache lines of the fields' and sigma's rows; fewer
+// workgroups would leave CUs idle. One MI355X, us per step with one column (the better of four and eight
+// wavefronts), two and four: 512 columns, 2 modes 88 86 90, 5 modes 120 126; 1024, 2 modes 125 113 113, 5 modes 202 186,
+// 6 modes 233 210; 2048, 2 modes 156 141 131, 6 modes 384 345; 4096, 1 mode 209 175 168, 2 modes 274 235 228, 6
+// modes 807 738.
 int gather_cols(const mmp_solver* s) {
   const int M = (int)s->P.M;
   const long columns = (long)s->g.N2 * s->F;
+  if (s->kerr_cols) return 1;  // (its instances)
   for (int cols : {4, 2})
-    if (columns >= 1024 * cols && colstage_cols_ok(M, cols) &&
+    if (columns >= 512 * cols && colstage_cols_ok(M, cols) &&
         colstage_products_lds_bytes(M, cols, s->fused.max_chunk_lines, s->fused.stride, s->P.parity) <=
             kColStageLds)
       return cols;

@@ -180,3 +180,25 @@ def test_lists_on_both_sides_of_the_gathers_choice(M, nt, lists, raman):
     s = cls(sp)
     check(s, sp, 3, 1, 1e-12)
     s.close()
+
+
+@pytest.mark.parametrize("symmetric", [True, False])
+@pytest.mark.parametrize("M,fibers", [(1, 17), (1, 32), (2, 16), (2, 32), (2, 64), (3, 32), (4, 16), (5, 16), (6, 16), (6, 64),
+                                      (8, 32), (13, 9)])
+def test_gather_forms_of_large_grids(M, fibers, symmetric):
+    """FP64 batches on 576 to 4096 columns: one, two and four columns a workgroup, four and eight wavefronts. Every
+    fiber equals itself alone (one column, eight or 12 wavefronts) bit for bit."""
+    require_device()
+    sps = [configs.grin_fiber(M=M, nt=4096, fiber_length=0.5 + 0.01 * i, seed=50 + i, symmetric=symmetric, power_range=(1.0, 100.0))
+           for i in range(3)]
+    note(f"case gather forms M={M} fibers={fibers} symmetric={symmetric}")
+    b = MultimodePropagationBatch([sps[i % 3] for i in range(fibers)])
+    b.advance(4)
+    for i, sp in enumerate(sps):
+        s = MultimodePropagationGPU_RamanON(sp)
+        s.advance(4)
+        want = s.getResult()
+        for f in (i, i + (fibers - 1 - i) // 3 * 3):  # its first and its last copy
+            assert np.array_equal(b.result(f), want), f
+        s.close()
+    b.close()
