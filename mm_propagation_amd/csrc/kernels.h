@@ -210,14 +210,14 @@ bool colstage_cols_ok(int M, int cols);
 int colstage_coef_pad(int M, bool parity);
 // FP32: whether the 8-wavefront and the three-workgroups-per-CU 4-wavefront gathers exist.
 bool colstage_wide_ok(int M);
-bool colstage_hi_occupancy_ok(int M, bool mixed, bool parity);
+bool colstage_hi_occupancy_ok(int M, bool parity);
 // Whether the matrix-core gather exists (SlotArgs::matrix_cores): FP32, 4 to 16 modes with
 // parity-structured coupling blocks, 4 to 10 without.
-bool colstage_matrix_cores_ok(int M, bool mixed, bool parity);
+bool colstage_matrix_cores_ok(int M, bool parity);
 int colstage_lines_per_chunk(int M);  // Raman lines of one LDS chunk at most
 // FP32: slots and coupling coefficients of one chunk at most.
 int colstage_slots_per_chunk();
-int colstage_coefficients_per_chunk(int M, bool mixed);
+int colstage_coefficients_per_chunk(int M);
 constexpr size_t kColStageLds = 65536;      // dynamic LDS of one gather workgroup at most
 size_t colstage_products_lds_bytes(int M, int cols, int lines, int steps, bool parity);
 constexpr size_t kColStagePairsLds = 65536;
@@ -282,12 +282,11 @@ hipError_t launch_colstage_products(const Geometry& g, const Twiddles& tw, const
 hipError_t launch_colstage_raman_gather(const Geometry& g, const Twiddles& tw, const cf* U, const cf* conv, cf* yout,
                                         const SlotArgs& fa, const float* Qd, double scale, const Batch& b, int F,
                                         hipStream_t s);
-// Dense-block gather (FP32, M <= 16): Qd is [P][M][M] with Qd[s][p][k] = sum of Q/max|Q| over the
+// Dense-block gather (FP32, M <= 12): Qd is [P][M][M] with Qd[s][p][k] = sum of Q/max|Q| over the
 // nonzeros (k, slot s) of Q^(p). dense_gather_chunk(M) is 0 when M is out of range.
 int dense_gather_chunk(int M);
-template <class W>
-hipError_t launch_gather_dense(const Geometry& g, const cpx<W>* U, const cpx<W>* VR, cpx<W>* sigma,
-                               const GatherArgs& a, const W* Qd, hipStream_t s);
+hipError_t launch_gather_dense(const Geometry& g, const cf* U, const cf* VR, cf* sigma, const GatherArgs& a, const float* Qd,
+                               hipStream_t s);
 // The no-allocation entry point's device scratch: a file-scope __device__ array of
 // kStaticScratchBytes per device (kernels.hip). static_scratch_resolve looks up its address on
 // `device` (which must be current) once; static_scratch returns it (nullptr before that).

@@ -808,18 +808,12 @@ constexpr int kColStageMaxM = 16;    // modes kept in registers by the gather
 // LDS limits of one chunk, by mode count: a few modes have few lines and small coupling
 // blocks, and a small LDS footprint lets more workgroups share a CU (batched fibers)
 constexpr int colstage_lines_cap(int M) { return M <= 4 ? 16 : (M <= 6 ? 24 : 40); }  // Raman lines
-// coupling coefficients held in LDS (64 KB FP64 would crowd out the lines)
-constexpr int colstage_qcap(int M, bool mixed) {
-  return M <= 4 ? 1024 : (M <= 6 ? 2048 : ((mixed && M > 10) ? 8192 : 4096));
-}
-template <int M, class W>
-constexpr int kColStageQCapOf = colstage_qcap(M, std::is_same<W, float>::value);
+// FP32: coupling coefficients held in LDS
+constexpr int colstage_qcap(int M) { return M <= 4 ? 1024 : (M <= 6 ? 2048 : (M <= 10 ? 4096 : 8192)); }
 // of those, prefetched into registers before the chunk's barrier (the rest go straight to LDS):
 // what a small tensor needs in all (up to 4 modes: 512, up to 6: 1024, parity-compact), 4096
-// where the registers allow it (FP32, 7 to 12 modes), else 2048
-template <int M, class W>
-constexpr int kColStageQPreOf =
-    M <= 4 ? 512 : (M <= 6 ? 1024 : ((std::is_same<W, float>::value && M <= 12) ? 4096 : 2048));
+// where the registers allow it (7 to 12 modes), else 2048
+constexpr int colstage_qpre(int M) { return M <= 4 ? 512 : (M <= 6 ? 1024 : (M <= 12 ? 4096 : 2048)); }
 constexpr int kColStageSCap = 128;   // slots of one chunk
 constexpr int kColStageRS = LineSlots<kColStageL, 1>::value;  // LDS row stride of a line (72)
 // LDS rows for the lines of a chunk: every wavefront of a round transforms 8 line slots, so
@@ -843,13 +837,12 @@ bool colstage_cols_ok(int M, int cols) {
   return cols == 1 || (cols == 2 && M <= kColStageMaxM2) || (cols == 4 && M <= kColStageMaxM4);
 }
 int colstage_lines_per_chunk(int M) { return colstage_lines_cap(M); }
-int colstage_coefficients_per_chunk(int M, bool mixed) { return colstage_qcap(M, mixed); }
+int colstage_coefficients_per_chunk(int M) { return colstage_qcap(M); }
 int colstage_slots_per_chunk() { return kColStageSCap; }
 // FP32: 8-wavefront gather workgroups up to 12 modes (beyond, the registers of a 512-lane
 // workgroup would spill)
-template <int M, class W>
-constexpr bool kColStageWide = M <= 12;
-bool colstage_wide_ok(int M) { return M <= 12; }
+constexpr bool wide_gather(int M) { return M <= 12; }
+bool colstage_wide_ok(int M) { return wide_gather(M); }
 
 // C1 over CW neighbouring columns per workgroup, the column block's Raman lines dealt to
 // `groups` workgroups (each transforms every field of the block, group 0 stores them to U).
@@ -986,14 +979,10 @@ int colstage_coef_pad(int M, bool parity) { return coef_pad(parity ? (M + 1) / 2
     asm("s_nop 1" MMP_BC(OP, 0, n0) MMP_BC(OP, 1, n1) MMP_BC(OP, 2, n2) MMP_BC(OP, 3, n3)                              \
         : "+v"(B[0]), "+v"(B[1]), "+v"(B[2]), "+v"(B[3])                                                               \
         : [c] "v"(c), [x] "v"(x), [n0] "n"(N), [n1] "n"(N + 1), [n2] "n"(N + 2), [n3] "n"(N + 3));
-template <int Q, int N, class W>
-__device__ __forceinline__ void fmac_bcast(W* B, W c, W x) {
+template <int Q, int N>
+__device__ __forceinline__ void fmac_bcast(double* B, double c, double x) {
   static_assert(Q >= 1 && N + Q <= 16, "coefficients of one register");
-  if constexpr (std::is_same<W, float>::value) {
-    MMP_FMAC_BCAST("v_fmac_f32_dpp")
-  } else {
-    MMP_FMAC_BCAST("v_fmac_f64_dpp")
-  }
+  MMP_FMAC_BCAST("v_fmac_f64_dpp")
   if constexpr (Q > 4) fmac_bcast<Q - 4, N + 4>(B + 4, c, x);
 }
 #undef MMP_FMAC_BCAST
@@ -1011,13 +1000,13 @@ constexpr int steps_cap(int M, bool parity) {
 // all products: up to 6 modes with the parity structure, up to 5 without (6 modes: 18 lines in 24 rows and 19
 // steps would take 65,792 bytes; sigma in the lines' rows leaves 51,968)
 constexpr bool own_sigma(int M, int cols, bool parity) { return cols == 1 && M <= (parity ? 6 : 5); }
-template <int M, int COLS, class W, bool PAR>
+template <int M, int COLS, bool PAR>
 struct C2Cfg {
   static constexpr int UR = (M + 7) / 8 * 8;
   static constexpr int STEPS = steps_cap(M, PAR);
   static __host__ __device__ size_t q_offset(int lines) {
     const int jw = 8 / COLS, rows = (lines + jw - 1) / jw * jw, sig = 2 * M;
-    return (size_t)(UR + (OWN ? rows + sig : (rows > sig ? rows : sig))) * COLS * kColStageRS * sizeof(cpx<W>);
+    return (size_t)(UR + (OWN ? rows + sig : (rows > sig ? rows : sig))) * COLS * kColStageRS * sizeof(cd);
   }
   static constexpr bool OWN = own_sigma(M, COLS, PAR);
   // vector form with two wavefronts per mode and column, one for each parity class
@@ -1032,8 +1021,8 @@ size_t colstage_products_lds_bytes(int M, int cols, int lines, int steps, bool p
 }
 
 // B[kk] += over the G = 16 / QP products of one coefficient register
-template <int QROW, int QP, int I = 0, class W>
-__device__ __forceinline__ void group_fmac(W* B, W c, const W* x) {
+template <int QROW, int QP, int I = 0>
+__device__ __forceinline__ void group_fmac(double* B, double c, const double* x) {
   fmac_bcast<QROW, I * QP>(B, c, x[I]);
   if constexpr ((I + 1) * QP < 16) group_fmac<QROW, QP, I + 1>(B, c, x);
 }
@@ -1043,20 +1032,19 @@ __device__ __forceinline__ void group_fmac(W* B, W c, const W* x) {
 // acc (even parity class) or acc2 (odd) += U_k B. Xc: the sample in the chunk's first X row (rows of
 // RS reals, the two products of a line together, COLS columns per line); Uc: in field row 0. The
 // coefficients come from LDS (QL) or by `coefs`, PD steps ahead. CS: parity class `cls` only.
-template <int QROW, int NP, int PD, int WPC, int COLS, int RS, bool PAR, bool QL, bool CS, class W, class Coefs, int PQ,
+template <int QROW, int NP, int PD, int WPC, int COLS, int RS, bool PAR, bool QL, bool CS, class Coefs, int PQ,
           int P2>
-__device__ __forceinline__ void product_sums(const ProductArgs& fa, const W* Qsh, const W* Xc, const cpx<W>* Uc, int xc0,
+__device__ __forceinline__ void product_sums(const ProductArgs& fa, const double* Qsh, const double* Xc, const cd* Uc, int xc0,
                                              int xc1, int M, int sub, int cls, bool busy, int lane, int& step,
-                                             uint32_t& sdesc, W (&cq)[PQ][NP], const Coefs& coefs, cpx<W> (&acc)[NP],
-                                             cpx<W> (&acc2)[P2]) {
-  using cw = cpx<W>;
+                                             uint32_t& sdesc, double (&cq)[PQ][NP], const Coefs& coefs, cd (&acc)[NP],
+                                             cd (&acc2)[P2]) {
   constexpr int QP = coef_pad(QROW), G = 16 / QP;
   auto xrow = [&](int x) { return ((x >> 1) * COLS * 2 + (x & 1)) * RS; };  // of product xc0 + x
-  W B[NP][QROW];
+  double B[NP][QROW];
 #pragma unroll
   for (int j = 0; j < NP; j++)
 #pragma unroll
-    for (int kk = 0; kk < QROW; kk++) B[j][kk] = (W)0;
+    for (int kk = 0; kk < QROW; kk++) B[j][kk] = 0.;
   // PD steps with their coefficients in PD fixed registers, each loaded again for the step PD
   // further on as soon as it is used
   // lane i: step i of its 64: offset of its X values (G products of one line, or of two neighbouring
@@ -1067,9 +1055,9 @@ __device__ __forceinline__ void product_sums(const ProductArgs& fa, const W* Qsh
     sx = (sdesc & 0xf0000000u) | (uint32_t)xrow(x >= xc0 && x < xc1 ? x - xc0 : 0);
   };
   describe();
-  W xv[PD][G], cl[PD][NP];
+  double xv[PD][G], cl[PD][NP];
   uint32_t sd[PD];
-  const W* ql[NP];  // QL: step's coefficients
+  const double* ql[NP];  // QL: step's coefficients
 #pragma unroll
   for (int j = 0; j < NP; j++)
     ql[j] = Qsh + ((sub + j * WPC < M ? sub + j * WPC : 0) * fa.stride + step) * 16 + (lane & 15);
@@ -1081,7 +1069,7 @@ __device__ __forceinline__ void product_sums(const ProductArgs& fa, const W* Qsh
       }
     }
     sd[u] = __builtin_amdgcn_readlane(sx, QL ? s : s & 63);
-    const W* xs = Xc + (sd[u] & 0xfffffffu);
+    const double* xs = Xc + (sd[u] & 0xfffffffu);
 #pragma unroll
     for (int i = 0; i < G; i++) xv[u][i] = xs[xrow(i)];
     if constexpr (QL) {
@@ -1109,18 +1097,18 @@ __device__ __forceinline__ void product_sums(const ProductArgs& fa, const W* Qsh
 #pragma unroll
       for (int j = 0; j < NP; j++) {
         const int par = PAR ? ((sub + j * WPC + sg) & 1) : 0;
-        cw sum = {0, 0};
+        cd sum = {0, 0};
 #pragma unroll
         for (int kk = 0; kk < QROW; kk++) {
           sum = cadd(sum, cscale(Uc[((PAR ? 2 * kk : kk) + par) * COLS * RS], B[j][kk]));
-          B[j][kk] = (W)0;
+          B[j][kk] = 0.;
         }
         if (sg >= 2) sum = {-sum.im, sum.re};
         if constexpr (!CS && PAR) {  // (selects of values: of places would put the sums in scratch memory)
           const bool odd = sg & 1;
-          const cw even = cadd(acc[j], sum), odds = cadd(acc2[CS || !PAR ? 0 : j], sum);
+          const cd even = cadd(acc[j], sum), odds = cadd(acc2[CS || !PAR ? 0 : j], sum);
           acc[j] = {odd ? acc[j].re : even.re, odd ? acc[j].im : even.im};
-          cw& o = acc2[CS || !PAR ? 0 : j];
+          cd& o = acc2[CS || !PAR ? 0 : j];
           o = {odd ? odds.re : o.re, odd ? odds.im : o.im};
         } else {
           acc[j] = cadd(acc[j], sum);
@@ -1150,12 +1138,11 @@ __device__ __forceinline__ void product_sums(const ProductArgs& fa, const W* Qsh
 // themselves from `U` (row order; the same array as yout: a workgroup reads and writes its own columns only),
 // transforms them in their LDS rows, and the products have no line: 8 launches of 5-8 us an RK4 step in place
 // of 16, 6 modes, NT = 16384 78.7 -> 50.6 us per step. Bound by latency and its column access.
-template <int M, int NW, int COLS, class W, bool PAR, bool RAMAN>
+template <int M, int NW, int COLS, bool PAR, bool RAMAN>
 __global__ void __launch_bounds__(NW * 64) k_colstage_products(
-    Geometry g, const cpx<W>* __restrict__ coltw, const cpx<W>* __restrict__ fourtw, const cpx<W>* U,
-    const cpx<W>* __restrict__ conv, cpx<W>* yout, ProductArgs fa, const W* __restrict__ Qp, double scale, Batch b) {
-  using cw = cpx<W>;
-  using C2 = C2Cfg<M, COLS, W, PAR>;
+    Geometry g, const cd* __restrict__ coltw, const cd* __restrict__ fourtw, const cd* U,
+    const cd* __restrict__ conv, cd* yout, ProductArgs fa, const double* __restrict__ Qp, double scale, Batch b) {
+  using C2 = C2Cfg<M, COLS, PAR>;
   const int fib = blockIdx.y;
   const FiberParams fp = b.fp[fib];
   if (!fp.live) return;  // uniform over the workgroup
@@ -1171,11 +1158,11 @@ __global__ void __launch_bounds__(NW * 64) k_colstage_products(
   constexpr int UIN = (M * COLS * L + NT - 1) / NT;
   static_assert(M >= 1 && M <= kColStageMaxM && JW >= 1 && WPC >= 1 && JL >= M, "modes or columns out of range");
   extern __shared__ __align__(16) unsigned char c2_lds[];
-  cw* const Ush = reinterpret_cast<cw*>(c2_lds);  // field rows [UR][COLS] (zeros beyond M); transform rows of sigma
-  cw* const Rsh = Ush + UR * COLS * RS;           // line rows [lines][COLS], then their X rows; then sigma
-  W* const Xsh = reinterpret_cast<W*>(Rsh);
-  W* const Qsh = reinterpret_cast<W*>(c2_lds + C2::q_offset(fa.max_chunk_lines));  // coefficients (QL)
-  cw* const Ssh = C2::OWN ? Rsh + (fa.max_chunk_lines + 7) / 8 * 8 * RS : Rsh;  // sigma rows
+  cd* const Ush = reinterpret_cast<cd*>(c2_lds);  // field rows [UR][COLS] (zeros beyond M); transform rows of sigma
+  cd* const Rsh = Ush + UR * COLS * RS;           // line rows [lines][COLS], then their X rows; then sigma
+  double* const Xsh = reinterpret_cast<double*>(Rsh);
+  double* const Qsh = reinterpret_cast<double*>(c2_lds + C2::q_offset(fa.max_chunk_lines));  // coefficients (QL)
+  cd* const Ssh = C2::OWN ? Rsh + (fa.max_chunk_lines + 7) / 8 * 8 * RS : Rsh;  // sigma rows
   const int tid = threadIdx.x;
   const int c = tid % COLS, t = (tid / COLS) % T, jl = tid / (T * COLS);
   const int lane = tid % 64;
@@ -1185,8 +1172,8 @@ __global__ void __launch_bounds__(NW * 64) k_colstage_products(
   // waits on memory, each by the wavefronts that use it only: the vector memory pipe takes a
   // wavefront's 16-byte loads at 64 bytes a cycle, and eight wavefronts loading every twiddle kept
   // a lone workgroup's first line waiting for 3000 cycles.
-  cw v[8], uin[UIN], w4[8];
-  LineTw<L, W> lt;
+  cd v[8], uin[UIN], w4[8];
+  LineTw<L, double> lt;
   int l0 = 0, l1 = fa.first_lines;
   if (wave * JW < (RAMAN ? l1 : M)) {
     const int last = (RAMAN ? l1 : M) - 1, q = jl < last ? jl : last;  // lanes without a line read the last one's
@@ -1218,8 +1205,8 @@ __global__ void __launch_bounds__(NW * 64) k_colstage_products(
   // each wavefront reads its modes' ahead of use, from cache lines requested here
   constexpr bool QL = M <= 6;
   constexpr int PD = QL ? 2 : 4;          // steps read ahead
-  const W* qf = Qp + fib * b.sq + (lane & 15);
-  auto coefs = [&](int s, W (&q)[NP]) {  // step s's coefficients of this wavefront's modes
+  const double* qf = Qp + fib * b.sq + (lane & 15);
+  auto coefs = [&](int s, double (&q)[NP]) {  // step s's coefficients of this wavefront's modes
 #pragma unroll
     for (int j = 0; j < NP; j++) {
       const int p = sub0 + j * WPC < M ? sub0 + j * WPC : 0;
@@ -1227,7 +1214,7 @@ __global__ void __launch_bounds__(NW * 64) k_colstage_products(
     }
   };
   constexpr int QIN = QL ? (M * C2::STEPS * 16 + NT - 1) / NT : 1;
-  W cq[QL ? 1 : PD][NP], qin[QIN], touch[QL ? 1 : NP];
+  double cq[QL ? 1 : PD][NP], qin[QIN], touch[QL ? 1 : NP];
   uint32_t sdesc = fa.steps[lane];
   {
     if constexpr (QL) {
@@ -1240,7 +1227,7 @@ __global__ void __launch_bounds__(NW * 64) k_colstage_products(
       for (int u = 0; u < PD; u++) coefs(u, cq[u]);
 #pragma unroll
       for (int j = 0; j < NP; j++) {
-        const int p = sub0 + j * WPC < M ? sub0 + j * WPC : 0, e = lane * (128 / (int)sizeof(W));
+        const int p = sub0 + j * WPC < M ? sub0 + j * WPC : 0, e = lane * (128 / (int)sizeof(double));
         touch[j] = Qp[fib * b.sq + (size_t)p * fa.stride * 16 + (e < fa.stride * 16 ? e : 0)];
       }
     }
@@ -1254,15 +1241,15 @@ __global__ void __launch_bounds__(NW * 64) k_colstage_products(
     // the field row after the last one, which the coupling rows of an odd number of modes read with
     // zero coefficients
     constexpr int UZ = M % 2 && PAR ? M + 1 : M;
-    for (int e = M * COLS * L + tid; e < UZ * COLS * L; e += NT) Ush[(e / L) * RS + e % L] = cw{0, 0};
+    for (int e = M * COLS * L + tid; e < UZ * COLS * L; e += NT) Ush[(e / L) * RS + e % L] = cd{0, 0};
   } else if (wave * JW < M) {
     // the fields; the lanes beyond the last one leave zero rows (whole wavefronts: up to UR rows)
 #pragma unroll
     for (int i = 0; i < 8; i++) v[i] = cmulc(v[i], w4[i]);
-    cw* row = Ush + (jl * COLS + c) * RS;
-    line_fft<L, 1, 1, 1, W, true>(v, row, lt, t);
+    cd* row = Ush + (jl * COLS + c) * RS;
+    line_fft<L, 1, 1, 1, double, true>(v, row, lt, t);
 #pragma unroll
-    for (int i = 0; i < 8; i++) row[t + i * T] = jl < M ? cscale(v[i], (W)scale) : cw{0, 0};
+    for (int i = 0; i < 8; i++) row[t + i * T] = jl < M ? cscale(v[i], scale) : cd{0, 0};
   }
   if constexpr (QL) {
 #pragma unroll
@@ -1270,8 +1257,8 @@ __global__ void __launch_bounds__(NW * 64) k_colstage_products(
       if (tid + r * NT < M * fa.stride * 16) Qsh[tid + r * NT] = qin[r];
     for (int e = tid + QIN * NT; e < M * fa.stride * 16; e += NT) Qsh[e] = Qp[fib * b.sq + e];
   }
-  const W sc = (W)scale, kv = (W)fp.kv, kr = (W)fp.kr;
-  cw acc[NP], acc2[CS || !PAR ? 1 : NP];  // sums of the even (CS: its own) and of the odd parity class
+  const double sc = scale, kv = fp.kv, kr = fp.kr;
+  cd acc[NP], acc2[CS || !PAR ? 1 : NP];  // sums of the even (CS: its own) and of the odd parity class
 #pragma unroll
   for (int p = 0; p < NP; p++) acc[p] = {0, 0};
 #pragma unroll
@@ -1304,8 +1291,8 @@ __global__ void __launch_bounds__(NW * 64) k_colstage_products(
       }
 #pragma unroll
       for (int i = 0; i < 8; i++) v[i] = cmulc(v[i], w4[i]);
-      cw* row = Rsh + ((q - l0) * COLS + c) * RS;
-      line_fft<L, 1, 1, 1, W, true>(v, row, lt, t);
+      cd* row = Rsh + ((q - l0) * COLS + c) * RS;
+      line_fft<L, 1, 1, 1, double, true>(v, row, lt, t);
 #pragma unroll
       for (int i = 0; i < 8; i++) row[t + i * T] = v[i];
     }
@@ -1315,12 +1302,12 @@ __global__ void __launch_bounds__(NW * 64) k_colstage_products(
 #pragma unroll 1
     for (int i = 0, r = wave; r < rows; i++, r += NW) {
       const uint32_t d0 = __builtin_amdgcn_readlane(dl.x, i), d1 = __builtin_amdgcn_readlane(dl.y, i);
-      const cw* uc = Ush + (COLS > 1 ? r % COLS : 0) * RS + lane;
-      const cw V0 = cmulc(uc[(d0 & 255u) * COLS * RS], uc[((d0 >> 8) & 255u) * COLS * RS]);
-      const cw V1 = cmulc(uc[(d1 & 255u) * COLS * RS], uc[((d1 >> 8) & 255u) * COLS * RS]);
-      W* x0 = Xsh + r * 2 * RS + lane;
+      const cd* uc = Ush + (COLS > 1 ? r % COLS : 0) * RS + lane;
+      const cd V0 = cmulc(uc[(d0 & 255u) * COLS * RS], uc[((d0 >> 8) & 255u) * COLS * RS]);
+      const cd V1 = cmulc(uc[(d1 & 255u) * COLS * RS], uc[((d1 >> 8) & 255u) * COLS * RS]);
+      double* x0 = Xsh + r * 2 * RS + lane;
       if constexpr (RAMAN) {
-        const cw vr = Rsh[r * RS + lane];
+        const cd vr = Rsh[r * RS + lane];
         x0[0] = kv * ((d0 >> 16) & 1u ? V0.im : V0.re) + kr * (vr.re * sc);
         x0[RS] = kv * ((d1 >> 16) & 1u ? V1.im : V1.re) + kr * (vr.im * sc);
       } else {
@@ -1334,8 +1321,8 @@ __global__ void __launch_bounds__(NW * 64) k_colstage_products(
     }
     __syncthreads();
     const int xc0 = 2 * l0, xc1 = 2 * l1 < fa.n_products ? 2 * l1 : fa.n_products;  // products of the chunk
-    const W* const Xc = Xsh + col * 2 * RS + lane;  // this lane's sample of the chunk's first X row
-    const cw* const Uc = Ush + col * RS + lane;     // this lane's sample of field k: Uc[k * COLS * RS]
+    const double* const Xc = Xsh + col * 2 * RS + lane;  // this lane's sample of the chunk's first X row
+    const cd* const Uc = Ush + col * RS + lane;     // this lane's sample of field k: Uc[k * COLS * RS]
     product_sums<QROW, NP, PD, WPC, COLS, RS, PAR, QL, CS>(fa, Qsh, Xc, Uc, xc0, xc1, M, sub0, cls, sub < 2 * M, lane, step,
                                                            sdesc, cq, coefs, acc, acc2);
   }
@@ -1351,13 +1338,13 @@ __global__ void __launch_bounds__(NW * 64) k_colstage_products(
   if (wave * JW < M) {
     const int q = jl;
     const bool valid = q < M;
-    const cw* in = Ssh + ((valid ? q : 0) * COLS + c) * RS;
+    const cd* in = Ssh + ((valid ? q : 0) * COLS + c) * RS;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
       v[i] = in[t + i * T];
       if constexpr (SETS == 2) v[i] = cadd(v[i], in[M * COLS * RS + t + i * T]);
     }
-    line_fft<L, -1, 1, 1, W, true>(v, Ush + (q * COLS + c) * RS, lt, t);
+    line_fft<L, -1, 1, 1, double, true>(v, Ush + (q * COLS + c) * RS, lt, t);
     if (valid) {
       const size_t base = (size_t)q * g.N + n2;
 #pragma unroll
@@ -1505,9 +1492,8 @@ __global__ void __launch_bounds__(kProductsMaxWaves * 64) k_gather_products(
 // for large grids only: batched M = 10, NT = 16384 x 36 fibers 563 -> 480 us, M = 8 x 16
 // fibers 125 -> 102 us; one fiber at NT = 65536 (1024 workgroups) 65 -> 67 us. Beyond 10
 // modes (and without parity blocks at 10) the bound spills hundreds of bytes per lane.
-template <int M, class W, bool PAR>
-constexpr bool kColStageHiOcc = std::is_same<W, float>::value && M >= 7 && (M <= 9 || (M == 10 && PAR));
-bool colstage_hi_occupancy_ok(int M, bool mixed, bool parity) { return mixed && M >= 7 && (M <= 9 || (M == 10 && parity)); }
+constexpr bool hi_occupancy(int M, bool parity) { return M >= 7 && (M <= 9 || (M == 10 && parity)); }
+bool colstage_hi_occupancy_ok(int M, bool parity) { return hi_occupancy(M, parity); }
 
 // The slot sums on the matrix cores (MF, FP32): per sample, B[p][k] = sum over slots s of
 // Qd[s][p][k] X_s is a real-by-complex matrix product with the rows (p, k) of one coupling parity
@@ -1529,10 +1515,10 @@ struct MfmaRows {
   static constexpr bool TSPLIT = RT > 2;      // the wavefront pairs split the tiles
   static constexpr int TPW = TSPLIT ? 2 : RT;  // tiles per wavefront
 };
-template <int M, class W, bool PAR>
-constexpr bool kColStageMfma = std::is_same<W, float>::value && M >= 4 && MfmaRows<M, PAR>::RT <= 4;
-bool colstage_matrix_cores_ok(int M, bool mixed, bool parity) {
-  if (!mixed || M < 4 || M > kColStageMaxM) return false;
+template <int M, bool PAR>
+constexpr bool kColStageMfma = M >= 4 && MfmaRows<M, PAR>::RT <= 4;
+bool colstage_matrix_cores_ok(int M, bool parity) {
+  if (M < 4 || M > kColStageMaxM) return false;
   const int qrow = parity ? (M + 1) / 2 : M, khh = (qrow + 1) / 2;
   return (M * khh + 15) / 16 <= 4;
 }
@@ -1543,14 +1529,13 @@ typedef float mfma_acc_t __attribute__((ext_vector_type(16)));
 // FP32) the slot sums run on the matrix cores: wavefront w takes the samples 32 (w % 2) .. + 31
 // and, with up to two 32-row tiles, every other pair of its parity class's slots (from pair
 // w / 2); with three or four tiles, tiles 2 (w / 2) and 2 (w / 2) + 1 over every pair.
-template <int M, int NW, class W, bool PAR, bool HI = false, bool MF = false>
-__global__ void __launch_bounds__(NW * 64, HI ? 3 : (MF ? (MfmaRows<M, PAR>::RT == 1 ? 3 : 2) : 1)) k_colstage_raman_gather(Geometry g, const cpx<W>* __restrict__ coltw,
-                                                                   const cpx<W>* __restrict__ fourtw,
-                                                                   const cpx<W>* __restrict__ U,
-                                                                   const cpx<W>* __restrict__ conv,
-                                                                   cpx<W>* __restrict__ yout, SlotArgs fa, const W* __restrict__ Qd,
+template <int M, int NW, bool PAR, bool HI = false, bool MF = false>
+__global__ void __launch_bounds__(NW * 64, HI ? 3 : (MF ? (MfmaRows<M, PAR>::RT == 1 ? 3 : 2) : 1)) k_colstage_raman_gather(Geometry g, const cf* __restrict__ coltw,
+                                                                   const cf* __restrict__ fourtw,
+                                                                   const cf* __restrict__ U,
+                                                                   const cf* __restrict__ conv,
+                                                                   cf* __restrict__ yout, SlotArgs fa, const float* __restrict__ Qd,
                                                                    double scale, Batch b) {
-  using cw = cpx<W>;
   const int fib = blockIdx.y;
   const FiberParams fp = b.fp[fib];
   if (!fp.live) return;  // uniform over the workgroup
@@ -1568,10 +1553,10 @@ __global__ void __launch_bounds__(NW * 64, HI ? 3 : (MF ? (MfmaRows<M, PAR>::RT 
   // Raman line rows of a chunk, or the NW partial sums of M modes after the gather
   constexpr int RCAP = colstage_rows(M) * RS > NW * M * L ? colstage_rows(M) * RS : NW * M * L;
   static_assert(M >= 1 && M <= kColStageMaxM, "modes out of range");
-  static_assert(!MF || (NW == 4 && !HI && kColStageMfma<M, W, PAR>), "matrix-core gather: FP32, 4 wavefronts");
-  __shared__ cw Ush[UR * RS];   // field rows; sigma rows after the gather
-  __shared__ cw Rsh[RCAP];      // Raman line rows of the chunk; partial sums after the gather
-  __shared__ W Qsh[kColStageQCapOf<M, W>];  // [slots of the chunk][M][M] coupling blocks
+  static_assert(!MF || (NW == 4 && !HI && kColStageMfma<M, PAR>), "matrix-core gather: 4 wavefronts");
+  __shared__ cf Ush[UR * RS];   // field rows; sigma rows after the gather
+  __shared__ cf Rsh[RCAP];      // Raman line rows of the chunk; partial sums after the gather
+  __shared__ float Qsh[colstage_qcap(M)];  // [slots of the chunk][M][M] coupling blocks
   __shared__ uint32_t Msh[kColStageSCap];  // slot metadata of the chunk
   // MF: the chunk's slots of each parity class in order (metadata, offset in the chunk), and
   // their counts
@@ -1584,11 +1569,11 @@ __global__ void __launch_bounds__(NW * 64, HI ? 3 : (MF ? (MfmaRows<M, PAR>::RT 
   const int n2 = xcd_block(blockIdx.x, gridDim.x);
   // the first chunk's lines, this lane's field samples, coupling blocks and slot metadata are
   // all requested before anything waits on memory
-  cw v[8], uin[UIN];
+  cf v[8], uin[UIN];
   // (each by the wavefronts that use it only: see the products' C2)
   int l0 = 0, l1 = fa.first_lines, s0 = 0, s1 = fa.first_slots;
-  LineTw<L, W> lt;
-  cw w4[8];
+  LineTw<L, float> lt;
+  cf w4[8];
   if (wave * (64 / T) < l1) {
     const size_t base = (size_t)(job < l1 ? job : l1 - 1) * g.N + (size_t)n2 * L;
 #pragma unroll
@@ -1599,13 +1584,13 @@ __global__ void __launch_bounds__(NW * 64, HI ? 3 : (MF ? (MfmaRows<M, PAR>::RT 
     const int e = tid + r * NT;
     if (wave * 64 + r * NT < M * L) uin[r] = U[(size_t)(e / L) * g.N + (size_t)n2 * L + e % L];
   }
-  constexpr int QIN = kColStageQPreOf<M, W> / NT;
-  W qin[QIN];
+  constexpr int QIN = colstage_qpre(M) / NT;
+  float qin[QIN];
   uint32_t min_ = 0;
 #pragma unroll
   for (int r = 0; r < QIN; r++) {
     const int e = tid + r * NT;
-    qin[r] = e < (s1 - s0) * MM ? Qd[(size_t)s0 * MM + e] : (W)0;
+    qin[r] = e < (s1 - s0) * MM ? Qd[(size_t)s0 * MM + e] : 0.f;
   }
   if (tid < s1 - s0) min_ = fa.slot_meta[s0 + tid];
   // (a later chunk may hold more lines than the first one: its limit is on slots, one or two a line)
@@ -1619,8 +1604,8 @@ __global__ void __launch_bounds__(NW * 64, HI ? 3 : (MF ? (MfmaRows<M, PAR>::RT 
     const int e = tid + r * NT;
     if (wave * 64 + r * NT < M * L) Ush[(e / L) * RS + e % L] = uin[r];
   }
-  const W sc = (W)scale, kv = (W)fp.kv, kr = (W)fp.kr;
-  cw u[MF ? 1 : M], acc[M];
+  const float sc = (float)scale, kv = (float)fp.kv, kr = (float)fp.kr;
+  cf u[MF ? 1 : M], acc[M];
 #pragma unroll
   for (int p = 0; p < M; p++) acc[p] = {0, 0};
   // MF: this lane's sample and lane half, and the coupling offset of its A-operand row in each
@@ -1653,7 +1638,7 @@ __global__ void __launch_bounds__(NW * 64, HI ? 3 : (MF ? (MfmaRows<M, PAR>::RT 
 #pragma unroll
       for (int r = 0; r < QIN; r++) {
         const int e = tid + r * NT;
-        qin[r] = e < (s1 - s0) * MM ? Qd[(size_t)s0 * MM + e] : (W)0;
+        qin[r] = e < (s1 - s0) * MM ? Qd[(size_t)s0 * MM + e] : 0.f;
       }
       if (tid < s1 - s0) min_ = fa.slot_meta[s0 + tid];
     }
@@ -1698,8 +1683,8 @@ __global__ void __launch_bounds__(NW * 64, HI ? 3 : (MF ? (MfmaRows<M, PAR>::RT 
       }
 #pragma unroll
       for (int i = 0; i < 8; i++) v[i] = cmulc(v[i], w4[i]);
-      cw* row = Rsh + (q - l0) * RS;
-      line_fft<L, 1, 1, 1, W, true>(v, row, lt, t);
+      cf* row = Rsh + (q - l0) * RS;
+      line_fft<L, 1, 1, 1, float, true>(v, row, lt, t);
       if (valid) {
 #pragma unroll
         for (int i = 0; i < 8; i++) row[t + i * T] = cscale(v[i], sc);
@@ -1725,38 +1710,38 @@ __global__ void __launch_bounds__(NW * 64, HI ? 3 : (MF ? (MfmaRows<M, PAR>::RT 
         meta_next = sl + NW < s1 ? Msh[sl + NW - s0] : 0u;
         if (PAR && (int)((meta >> 18) & 1u) != par) continue;
         const int pa = meta & 255u, pb = (meta >> 8) & 255u, kind = (meta >> 16) & 3u, line = (int)(meta >> 19);
-        const W* qb = Qsh + (sl - s0) * MM;
-        const cw r = Rsh[(line - l0) * RS + lane];
-        const cw V = cmulc(Ush[pa * RS + lane], Ush[pb * RS + lane]);
-        cw vr;
+        const float* qb = Qsh + (sl - s0) * MM;
+        const cf r = Rsh[(line - l0) * RS + lane];
+        const cf V = cmulc(Ush[pa * RS + lane], Ush[pb * RS + lane]);
+        cf vr;
         switch (kind) {
           case kDirect: vr = r; break;
           case kConj: vr = cconj(r); break;
           case kRe: vr = {r.re, 0}; break;
           default: vr = {r.im, 0}; break;
         }
-        const cw X = cadd(cscale(V, kv), cscale(vr, kr));
-        cw y[M];
+        const cf X = cadd(cscale(V, kv), cscale(vr, kr));
+        cf y[M];
 #pragma unroll
         for (int k = 0; k < M; k++) y[k] = cmul(X, u[k]);
-        // the block's rows in groups of about 224 bytes (128 for FP32 beyond 10 modes, whose
+        // the block's rows in groups of about 224 bytes (128 beyond 10 modes, whose
         // registers are fuller; 64 in the 168-VGPR variant): each group's LDS reads are issued together (the scheduling
         // barrier keeps them ahead of their uses), so one LDS latency is exposed per group
         // rather than one per pair of coefficients
         constexpr int QROW = PAR ? KH : M;  // coefficients per row p
-        constexpr int QGB = HI ? 64 : ((std::is_same<W, float>::value && M > 10) ? 128 : 224);
-        constexpr int PG = (int)(QGB / sizeof(W)) / QROW > 0 ? (int)(QGB / sizeof(W)) / QROW : 1;
+        constexpr int QGB = HI ? 64 : (M > 10 ? 128 : 224);
+        constexpr int PG = (int)(QGB / sizeof(float)) / QROW > 0 ? (int)(QGB / sizeof(float)) / QROW : 1;
 #pragma unroll
         for (int p0 = 0; p0 < M; p0 += PG) {
-          W qv[PG * QROW];
+          float qv[PG * QROW];
 #pragma unroll
-          for (int e = 0; e < PG * QROW; e++) qv[e] = p0 * QROW + e < M * QROW ? qb[p0 * QROW + e] : (W)0;
+          for (int e = 0; e < PG * QROW; e++) qv[e] = p0 * QROW + e < M * QROW ? qb[p0 * QROW + e] : 0.f;
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
           for (int pp = 0; pp < PG; pp++) {
             const int p = p0 + pp;
             if (p >= M) break;
-            cw tsum = acc[p];
+            cf tsum = acc[p];
             if constexpr (PAR) {
               // only k with (p + k) % 2 == the slot's parity: q[p][kk] belongs to k = 2 kk + ((p + par) % 2)
 #pragma unroll
@@ -1795,27 +1780,27 @@ __global__ void __launch_bounds__(NW * 64, HI ? 3 : (MF ? (MfmaRows<M, PAR>::RT 
       // that their LDS reads overlap the matrix-core work of the pair before; the slot's
       // descriptor (metadata, offset in the chunk) is read one pair before that
       auto descriptor = [&](int pi) { return Lsh[cc * kColStageSCap + (2 * pi + hh < n ? 2 * pi + hh : 0)]; };
-      auto operands = [&](int pi, uint2 d, W& xre, W& xim, W (&qa)[TPW]) {
+      auto operands = [&](int pi, uint2 d, float& xre, float& xim, float (&qa)[TPW]) {
         // past the last slot: slot 0's data (finite) times zero, so that no branch splits the reads
-        const W hm = 2 * pi + hh < n ? (W)1 : (W)0;
+        const float hm = 2 * pi + hh < n ? 1.f : 0.f;
         const uint32_t meta = d.x;
         const int x = (int)d.y;
         const int pa = meta & 255u, pb = (meta >> 8) & 255u, kind = (meta >> 16) & 3u, line = (int)(meta >> 19);
-        const cw r = Rsh[(line - l0) * RS + smp];
-        const cw ua = Ush[pa * RS + smp], ub = Ush[pb * RS + smp];
+        const cf r = Rsh[(line - l0) * RS + smp];
+        const cf ua = Ush[pa * RS + smp], ub = Ush[pb * RS + smp];
 #pragma unroll
         for (int t = 0; t < TPW; t++) {
           const int o = aoff[cc][t];
-          qa[t] = Qsh[x * MM + (o >= 0 ? o : 0)] * (o >= 0 ? hm : (W)0);
+          qa[t] = Qsh[x * MM + (o >= 0 ? o : 0)] * (o >= 0 ? hm : 0.f);
         }
-        const cw V = cmulc(ua, ub);
-        const W vre = kind == kIm ? r.im : r.re;
-        const W vim = kind == kDirect ? r.im : (kind == kConj ? -r.im : (W)0);
+        const cf V = cmulc(ua, ub);
+        const float vre = kind == kIm ? r.im : r.re;
+        const float vim = kind == kDirect ? r.im : (kind == kConj ? -r.im : 0.f);
         xre = (kv * V.re + kr * vre) * hm;
         xim = (kv * V.im + kr * vim) * hm;
       };
       int pi = MR::TSPLIT ? 0 : (wave >> 1);
-      W xre, xim, qa[TPW];
+      float xre, xim, qa[TPW];
       uint2 dn = {0u, 0u};
       if (n > 0) {
         operands(pi, descriptor(pi), xre, xim, qa);
@@ -1823,7 +1808,7 @@ __global__ void __launch_bounds__(NW * 64, HI ? 3 : (MF ? (MfmaRows<M, PAR>::RT 
       }
 #pragma nounroll
       for (; pi < npairs; pi += PSTEP) {  // wave-uniform
-        W nre, nim, nqa[TPW];
+        float nre, nim, nqa[TPW];
         const uint2 d2 = dn;
         dn = descriptor(pi + 2 * PSTEP);
         operands(pi + PSTEP, d2, nre, nim, nqa);
@@ -1857,8 +1842,8 @@ __global__ void __launch_bounds__(NW * 64, HI ? 3 : (MF ? (MfmaRows<M, PAR>::RT 
               // U_k of this lane's half from its LDS row (a padding row's products are zero: any
               // field row serves)
               const int row = kA >= M ? 0 : (kB < M ? kA + (kB - kA) * hh : kA);
-              const cw uk = Ush[row * RS + smp];
-              acc[p] = cadd(acc[p], cmul(uk, cw{ar[j][r], ai[j][r]}));
+              const cf uk = Ush[row * RS + smp];
+              acc[p] = cadd(acc[p], cmul(uk, cf{ar[j][r], ai[j][r]}));
             }
           }
         }
@@ -1890,7 +1875,7 @@ __global__ void __launch_bounds__(NW * 64, HI ? 3 : (MF ? (MfmaRows<M, PAR>::RT 
   __syncthreads();
   for (int e = tid; e < M * L; e += NT) {
     const int p = e / L, j = e % L;
-    cw tsum = Rsh[p * L + j];
+    cf tsum = Rsh[p * L + j];
 #pragma unroll
     for (int w = 1; w < NW; w++) tsum = cadd(tsum, Rsh[(w * M + p) * L + j]);
     Ush[p * RS + j] = tsum;
@@ -1899,10 +1884,10 @@ __global__ void __launch_bounds__(NW * 64, HI ? 3 : (MF ? (MfmaRows<M, PAR>::RT 
   if (wave * (64 / T) < M) {
     const int q = job;
     const bool valid = q < M;
-    cw* row = Ush + q * RS;
+    cf* row = Ush + q * RS;
 #pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = valid ? row[t + i * T] : cw{0, 0};
-    line_fft<L, -1, 1, 1, W, true>(v, row, lt, t);
+    for (int i = 0; i < 8; i++) v[i] = valid ? row[t + i * T] : cf{0, 0};
+    line_fft<L, -1, 1, 1, float, true>(v, row, lt, t);
     if (valid) {
       const size_t base = (size_t)q * g.N + n2;
 #pragma unroll
@@ -1927,22 +1912,21 @@ int dense_gather_chunk(int M) {
   return room >= 4 * M ? room : 0;
 }
 
-template <int M, class W>
-__global__ void __launch_bounds__(256) k_gather_dense(Geometry g, const cpx<W>* __restrict__ U,
-                                                      const cpx<W>* __restrict__ VR, cpx<W>* __restrict__ sigma,
-                                                      GatherArgs a, const W* __restrict__ Qd, int chunk) {
-  using cw = cpx<W>;
-  __shared__ cw sh[kDenseCap];
+template <int M>
+__global__ void __launch_bounds__(256) k_gather_dense(Geometry g, const cf* __restrict__ U,
+                                                      const cf* __restrict__ VR, cf* __restrict__ sigma,
+                                                      GatherArgs a, const float* __restrict__ Qd, int chunk) {
+  __shared__ cf sh[kDenseCap];
   constexpr int TS = 64;
-  cw* Ush = sh;           // [M][TS]
-  cw* Xsh = sh + M * TS;  // [chunk][TS]; reused for the partial sums
+  cf* Ush = sh;           // [M][TS]
+  cf* Xsh = sh + M * TS;  // [chunk][TS]; reused for the partial sums
   const int t0 = blockIdx.x * TS;
   const int tid = threadIdx.x, lane = tid % TS;
   const int wave = __builtin_amdgcn_readfirstlane(tid / TS);
 #pragma unroll 4
   for (int e = tid; e < M * TS; e += 256) Ush[e] = U[(size_t)(e / TS) * g.N + t0 + e % TS];
   __syncthreads();
-  cw u[M], acc[M];
+  cf u[M], acc[M];
 #pragma unroll
   for (int k = 0; k < M; k++) {
     u[k] = Ush[k * TS + lane];
@@ -1954,14 +1938,14 @@ __global__ void __launch_bounds__(256) k_gather_dense(Geometry g, const cpx<W>* 
     slot_mix_tile(a, g, VR, Ush, Xsh, s0, ns, t0, tid, 256);
     __syncthreads();
     for (int sl = s0 + wave; sl < s0 + ns; sl += 4) {
-      const cw X = Xsh[(sl - s0) * TS + lane];
-      const W* qb = Qd + (size_t)sl * M * M;
-      cw y[M];
+      const cf X = Xsh[(sl - s0) * TS + lane];
+      const float* qb = Qd + (size_t)sl * M * M;
+      cf y[M];
 #pragma unroll
       for (int k = 0; k < M; k++) y[k] = cmul(X, u[k]);
 #pragma unroll
       for (int p = 0; p < M; p++) {
-        cw t = acc[p];
+        cf t = acc[p];
 #pragma unroll
         for (int k = 0; k < M; k++) t = cadd(t, cscale(y[k], qb[p * M + k]));
         acc[p] = t;
@@ -1974,7 +1958,7 @@ __global__ void __launch_bounds__(256) k_gather_dense(Geometry g, const cpx<W>* 
   __syncthreads();
   for (int e = tid; e < M * TS; e += 256) {
     const int p = e / TS, j = e % TS;
-    cw t = Xsh[p * TS + j];
+    cf t = Xsh[p * TS + j];
 #pragma unroll
     for (int w = 1; w < 4; w++) t = cadd(t, Xsh[(w * M + p) * TS + j]);
     sigma[(size_t)p * g.N + t0 + j] = t;
@@ -2325,7 +2309,7 @@ static hipError_t c2_launch(const Geometry& g, const Twiddles& tw, const cd* U, 
                             const ProductArgs& fa, const double* Qp, double scale, const Batch& b, int F, hipStream_t s) {
   const size_t lds = colstage_products_lds_bytes(M, COLS, fa.max_chunk_lines, fa.stride, PAR);
   if (g.N2 % COLS || lds > kColStageLds) return hipErrorInvalidValue;
-  MMP_LAUNCH((k_colstage_products<M, NW, COLS, double, PAR, RAMAN>), dim3(g.N2 / COLS, F), dim3(NW * 64), lds, s, g, tw.coltw,
+  MMP_LAUNCH((k_colstage_products<M, NW, COLS, PAR, RAMAN>), dim3(g.N2 / COLS, F), dim3(NW * 64), lds, s, g, tw.coltw,
              tw.fourtw, U, conv, yout, fa, Qp, scale, b);
   return hipGetLastError();
 }
@@ -2377,19 +2361,19 @@ hipError_t launch_colstage_products(const Geometry& g, const Twiddles& tw, const
 
 // C2 in FP32, on the complex slots
 #define MMP_COLSTAGE_GO(MV, NWV, PARV, ...)                                                                        \
-  MMP_LAUNCH((k_colstage_raman_gather<MV, NWV, float, PARV __VA_ARGS__>), dim3(g.N2, F), dim3(NWV * 64), 0, s, g,  \
+  MMP_LAUNCH((k_colstage_raman_gather<MV, NWV, PARV __VA_ARGS__>), dim3(g.N2, F), dim3(NWV * 64), 0, s, g,  \
              tw.coltw32, tw.fourtw32, U, conv, yout, fa, Qd, scale, b);                                            \
   break;
 #define MMP_COLSTAGE_LAUNCH(MV, PARV)                                                                              \
-  if constexpr (kColStageMfma<MV, float, PARV>)                                                                    \
+  if constexpr (kColStageMfma<MV, PARV>)                                                                           \
     if (fa.waves == 4 && fa.matrix_cores) {                                                                        \
       MMP_COLSTAGE_GO(MV, 4, PARV, , false, true)                                                                  \
     }                                                                                                              \
-  if constexpr (kColStageHiOcc<MV, float, PARV>)                                                                   \
+  if constexpr (hi_occupancy(MV, PARV))                                                                            \
     if (fa.waves == 4 && fa.hi_occupancy) {                                                                        \
       MMP_COLSTAGE_GO(MV, 4, PARV, , true)                                                                         \
     }                                                                                                              \
-  if constexpr (kColStageWide<MV, float>)                                                                          \
+  if constexpr (wide_gather(MV))                                                                                   \
     if (fa.waves == 8) {                                                                                           \
       MMP_COLSTAGE_GO(MV, 8, PARV)                                                                                 \
     }                                                                                                              \
@@ -2408,7 +2392,7 @@ hipError_t launch_colstage_raman_gather(const Geometry& g, const Twiddles& tw, c
   const int block = fa.parity ? g.M * ((g.M + 1) / 2) : g.M * g.M;
   if (fa.n_chunks < 1 || fa.max_chunk_lines < 1 || fa.max_chunk_lines > colstage_lines_per_chunk(g.M) ||
       fa.max_chunk_slots < 1 || fa.max_chunk_slots > colstage_slots_per_chunk() ||
-      fa.max_chunk_slots * block > colstage_coefficients_per_chunk(g.M, true))
+      fa.max_chunk_slots * block > colstage_coefficients_per_chunk(g.M))
     return hipErrorInvalidValue;
   switch (g.M) {
     MMP_COLSTAGE_CASE(1) MMP_COLSTAGE_CASE(2) MMP_COLSTAGE_CASE(3) MMP_COLSTAGE_CASE(4) MMP_COLSTAGE_CASE(5)
@@ -2422,18 +2406,16 @@ hipError_t launch_colstage_raman_gather(const Geometry& g, const Twiddles& tw, c
 
 #define MMP_DENSE_CASE(MV)                                                                                     \
   case MV:                                                                                                      \
-    MMP_LAUNCH((k_gather_dense<MV, W>), dim3(g.N / 64), dim3(256), 0, s, g, U, VR, sigma, a, Qd, chunk); \
+    MMP_LAUNCH((k_gather_dense<MV>), dim3(g.N / 64), dim3(256), 0, s, g, U, VR, sigma, a, Qd, chunk);           \
     break;
 
-template <class W>
-hipError_t launch_gather_dense(const Geometry& g, const cpx<W>* U, const cpx<W>* VR, cpx<W>* sigma,
-                               const GatherArgs& a, const W* Qd, hipStream_t s) {
+hipError_t launch_gather_dense(const Geometry& g, const cf* U, const cf* VR, cf* sigma, const GatherArgs& a, const float* Qd,
+                               hipStream_t s) {
   const int chunk = dense_gather_chunk(g.M);
   if (!chunk || g.N % 64) return hipErrorInvalidValue;
   switch (g.M) {
     MMP_DENSE_CASE(1) MMP_DENSE_CASE(2) MMP_DENSE_CASE(3) MMP_DENSE_CASE(4) MMP_DENSE_CASE(5) MMP_DENSE_CASE(6)
     MMP_DENSE_CASE(7) MMP_DENSE_CASE(8) MMP_DENSE_CASE(9) MMP_DENSE_CASE(10) MMP_DENSE_CASE(11) MMP_DENSE_CASE(12)
-    MMP_DENSE_CASE(13) MMP_DENSE_CASE(14) MMP_DENSE_CASE(15) MMP_DENSE_CASE(16)
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -2514,8 +2496,6 @@ hipError_t launch_photon_number(const Geometry& g, const cd* spectra, double* ou
                                                       cpx<W>*, const uint2*, int, double, const Batch&, int, int,  \
                                                       int, int, hipStream_t);
 MMP_INSTANTIATE_W(double)
-template hipError_t launch_gather_dense<float>(const Geometry&, const cf*, const cf*, cf*, const GatherArgs&, const float*,
-                                               hipStream_t);
 MMP_INSTANTIATE_W(float)
 
 }  // namespace mmp

@@ -581,7 +581,7 @@ static bool plan_slot_chunks(Problem& P, int max_lines) {
   if (nl > 0 && P.line_slot0.size() == (size_t)nl + 1 && P.line_slot0[0] == 0 && P.line_slot0[nl] == P.P) {
     const int block = P.parity ? (int)(M * ((M + 1) / 2)) : (int)(M * M);  // coefficients per slot
     const int max_slots =
-        std::min(colstage_slots_per_chunk(), colstage_coefficients_per_chunk((int)M, P.mixed) / block);
+        std::min(colstage_slots_per_chunk(), colstage_coefficients_per_chunk((int)M) / block);
     bool ok = max_slots >= 2;
     P.fused_line.push_back(0);
     P.fused_slot.push_back(0);

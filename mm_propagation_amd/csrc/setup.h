@@ -70,7 +70,6 @@ struct Problem {
   // of odd parity. A pair whose two slots differ in parity lies in both (the segments then overlap).
   // Without the parity structure all products lie in the even segments.
   uint32_t seg_b[4] = {0, 0, 0, 0}, seg_e[4] = {0, 0, 0, 0};
-  uint32_t seg_products() const { return seg_e[0] - seg_b[0] + seg_e[1] - seg_b[1] + seg_e[2] - seg_b[2] + seg_e[3] - seg_b[3]; }
   bool need_im = false;                             // some Q1 - Q2 is not zero
   bool products = false;                            // the gather sums the real products (choose_products)
   // chunks of Raman lines (0 chunks: the column-stage kernels do not apply) and the largest chunk

@@ -353,7 +353,7 @@ mmp_status enqueue_step_w(mmp_solver* s) {
       if constexpr (std::is_same<W, double>::value) {
         if (s->products) return launch_gather_products(g, U, conv, ybuf, s->fused, qdense, s->batch, P.raman, st);
       } else {
-        if (qdense) return launch_gather_dense<W>(g, U, conv, ybuf, s->gather, qdense, st);
+        if (qdense) return launch_gather_dense(g, U, conv, ybuf, s->gather, qdense, st);
       }
       return launch_gather<W>(g, U, conv, ybuf, s->gather, st);
     }));
@@ -1033,7 +1033,7 @@ mmp_status create_impl(mmp_ctx* ctx, uint32_t n_fibers, const mmp_params* params
       // (measured, 29 fibers of 3 modes at NT = 16384: 71 us with eight, 38 us with four)
       s->slots.waves = M >= 4 && M <= 6 ? 8 : 4;
       // grids of 8 or more workgroups per CU
-      s->slots.hi_occupancy = colstage_hi_occupancy_ok(M, true, compact) && (long)s->g.N2 * s->F >= 2048;
+      s->slots.hi_occupancy = colstage_hi_occupancy_ok(M, compact) && (long)s->g.N2 * s->F >= 2048;
       // the coupling sums on the matrix cores (FP32) by default at 4 to 10 and 13 to 16 modes,
       // whatever the number of fibers (a batch runs the arithmetic of its fibers alone). Measured on
       // one MI355X, gather per launch against the vector gather: 7-8 modes 1.03-1.23x (one 32-row
@@ -1045,7 +1045,7 @@ mmp_status create_impl(mmp_ctx* ctx, uint32_t n_fibers, const mmp_params* params
       // four tiles, the wavefront pairs splitting them).
       const bool want = (opt.flags & MMP_FLAG_MATRIX_CORES) || (M >= 4 && M <= 10) || M >= 13;
       s->slots.matrix_cores =
-          !(opt.flags & MMP_FLAG_NO_MATRIX_CORES) && want && colstage_matrix_cores_ok(M, true, compact) ? 1 : 0;
+          !(opt.flags & MMP_FLAG_NO_MATRIX_CORES) && want && colstage_matrix_cores_ok(M, compact) ? 1 : 0;
       if (s->slots.matrix_cores) {
         s->slots.waves = 4;
         s->slots.hi_occupancy = 0;
@@ -1159,8 +1159,8 @@ bool plan_valid(const mmp_solver* s, const ColPlan& c) {
   const int M = (int)s->P.M;
   if (s->mixed) {
     if (c.cols != 1 || (c.waves != 4 && !(c.waves == 8 && colstage_wide_ok(M)))) return false;
-    if (c.hi && !(c.waves == 4 && colstage_hi_occupancy_ok(M, true, s->slots.parity != 0))) return false;
-    const bool mf_ok = colstage_matrix_cores_ok(M, true, s->slots.parity != 0);
+    if (c.hi && !(c.waves == 4 && colstage_hi_occupancy_ok(M, s->slots.parity != 0))) return false;
+    const bool mf_ok = colstage_matrix_cores_ok(M, s->slots.parity != 0);
     if (c.mf && (c.waves != 4 || c.hi || (s->opt.flags & MMP_FLAG_NO_MATRIX_CORES) || !mf_ok)) return false;
     if (!c.mf && mf_ok && (s->opt.flags & MMP_FLAG_MATRIX_CORES)) return false;
   } else {
