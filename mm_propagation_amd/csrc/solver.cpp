@@ -111,7 +111,7 @@ struct mmp_solver {
   SlotArgs slots{};
   bool use_fused = false;
   bool kerr_cols = false;    // FP64 without Raman: one column kernel per stage (one fiber)
-  bool products = false;     // the gather sums the real products (FP64; beyond its sizes the sparse slots)
+  bool products = false;     // the gather sums the real products (Problem::products; else FP64 sums the sparse slots)
   int chunk_lines = 0;       // column-stage gather: Raman lines per LDS chunk at most
   bool tuned = false;        // MMP_FLAG_AUTOTUNE chose fused.waves and chunk_lines
   int pair_columns = 1;      // column-stage pair pass: columns per workgroup and line groups
@@ -569,13 +569,16 @@ size_t planned_device_bytes(const Problem& P, const mmp_options& opt, size_t F) 
 
 // FP64: wavefronts of the column-stage gather's workgroup of one column. On grids of one workgroup a CU or less it
 // takes eight (12 at 5 and 6 modes where the Im products double the sums, `both`): a wavefront per mode, up to
-// 4 modes (12: 6) one per mode and parity class. Larger grids hide the sums' latency with other workgroups, up
-// to 12 modes; beyond, four wavefronts have up to four modes each. One MI355X, us per step with four and eight
-// (and 12), all products: 256 columns, 3 modes 91.9 and 89.4, 5 modes 109.3 and 106.9 (103.7), 10 modes 233 and 222; 512
-// columns, 3 modes 104.8 and 110.6, 5 modes 139 and 150 (145), 10 modes 372 and 432, 13 modes (symmetric) 481 and
-// 435; 1024 columns, 10 modes 745 and 868, 13 modes 955 and 864; 4096 columns, 16 modes 4809 and 4229.
-int products_waves(int M, long columns, bool both) {
-  if (M <= 12 && columns > 256) return 4;
+// 4 modes (12: 6) one per mode and parity class. Larger grids hide the sums' latency with other workgroups; with
+// Raman not beyond 12 modes, where four wavefronts have up to four modes each. Without Raman up to 4 modes stay
+// with eight on two workgroups a CU. One MI355X, us per step with four and eight (and 12), all products. Raman: 256
+// columns, 3 modes 91.9 and 89.4, 5 modes 109.3 and 106.9 (103.7), 10 modes 233 and 222; 512 columns, 3 modes 104.8
+// and 110.6, 5 modes 139 and 150 (145), 10 modes 372 and 432, 13 modes (symmetric) 481 and 435; 1024 columns, 10
+// modes 745 and 868, 13 modes 955 and 864; 4096 columns, 16 modes 4809 and 4229. No Raman: 256 columns, 5 modes 54.4
+// and 52.0 (49.3), 10 modes 120 and 113; 512 columns, 3 modes 53.9 and 52.1, 5 modes 67.9 and 67.6 (72.0), 10 modes
+// 161 and 207; 1024 columns, 3 modes 74.1 and 81.8, 13 modes (symmetric) 358 and 429.
+int products_waves(int M, long columns, bool both, bool raman) {
+  if (raman ? M <= 12 && columns > 256 : columns > (M <= 4 ? 512 : 256)) return 4;
   return (M == 5 || M == 6) && both ? 12 : 8;
 }
 
@@ -605,7 +608,7 @@ void fill_info(const Problem& P, const mmp_options& opt, mmp_info* o) {
   const bool fused = P.fused_chunks > 0 && !(opt.flags & MMP_FLAG_SEPARATE_COLUMNS);
   // the defaults, before any tuning
   const bool both = P.need_im && P.parity && P.fused_chunks == 1;
-  o->gather_waves = !fused ? 0u : (P.mixed ? (P.M <= 6 ? 8u : 4u) : (uint32_t)products_waves((int)P.M, (long)P.N2, both));
+  o->gather_waves = !fused ? 0u : (P.mixed ? (P.M <= 6 ? 8u : 4u) : (uint32_t)products_waves((int)P.M, (long)P.N2, both, true));
   o->chunk_lines = fused ? (uint32_t)colstage_chunk_lines(P, P.need_im) : 0u;
   if (fused) {  // a solver of one fiber (a batch may choose differently; results do not depend on it)
     int columns = 1, groups = 1;
@@ -734,7 +737,8 @@ int gather_cols(const mmp_solver* s) {
 
 int gather_waves(const mmp_solver* s) {
   if (s->fused.cols > 1) return 4;
-  return products_waves((int)s->P.M, (long)s->g.N2 * s->F, s->need_im && s->fused.parity && s->fused.n_chunks == 1);
+  return products_waves((int)s->P.M, (long)s->g.N2 * s->F, s->need_im && s->fused.parity && s->fused.n_chunks == 1,
+                        s->P.raman);
 }
 
 // Uploads fiber f's own data (operators, couplings, Raman spectrum, initial state, scalars),

@@ -202,3 +202,14 @@ def test_gather_forms_of_large_grids(M, fibers, symmetric):
             assert np.array_equal(b.result(f), want), f
         s.close()
     b.close()
+
+
+@pytest.mark.parametrize("M,nt", [(1, 65536), (4, 32768), (5, 32768), (7, 32768), (13, 32768)])
+def test_column_kernel_without_raman_on_large_grids(M, nt):
+    """512 and 1024 columns: eight wavefronts up to 4 modes on the first, four else."""
+    require_device()
+    sp = configs.grin_fiber(M=M, nt=nt, power_range=(1.0, 100.0), seed=12)
+    note(f"case columns without Raman M={M} nt={nt}")
+    s = MultimodePropagationGPU_RamanOFF(sp)
+    check(s, sp, 2, 1, 1e-12)
+    s.close()
