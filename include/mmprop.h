@@ -70,7 +70,8 @@ enum {
   MMP_FLAG_SEPARATE_COLUMNS = 1u << 2, /* keep every column pass a kernel of its own (7 passes per stage)
                                           where the column-stage kernels would run (4 passes per stage:
                                           Raman on, 64-sample columns, n_modes <= 16; 2 for one FP64
-                                          fiber with Raman off) */
+                                          fiber with Raman off, unless it has more than 12 modes
+                                          and lists far from full) */
   MMP_FLAG_AUTOTUNE = 1u << 3 /* at creation, time the column-stage gather variants (wavefronts per
                                  workgroup, Raman lines per LDS chunk) on this solver's own data and
                                  keep the fastest; the choice is cached per structure for the process.
@@ -226,7 +227,10 @@ MMP_API mmp_status mmp_fiber_energy(mmp_solver* solver, uint32_t fiber, double* 
 MMP_API mmp_status mmp_fiber_info(mmp_solver* solver, uint32_t fiber, mmp_info* info_out);
 /* Replaces fiber f by a new problem of the same structure (a serving slot taking a new
  * request): its inputs are uploaded, it restarts at z = 0; the other fibers keep their state.
- * Waits for the work already queued on the context's stream. */
+ * Waits for the work already queued on the context's stream. A solver of one fiber whose sums run over
+ * a nonzero list, or would for the new fiber, is made anew in its place (it allocates and frees device
+ * memory, and on a failure stays as it was). After a load that failed on the way, stepping may return
+ * MMP_ERR_STATE until a load has gone through. */
 MMP_API mmp_status mmp_fiber_load(mmp_solver* solver, uint32_t fiber, const mmp_params* params);
 /* Parks (live = 0) or resumes (live = 1) fiber f: the steps leave a parked fiber's field, z and
  * Lawson tables untouched, and its workgroups exit at once, so a batch whose slots are partly

@@ -790,15 +790,15 @@ __global__ void __launch_bounds__(512) k_gather(Geometry g, const cpx<W>* __rest
 }
 
 // ---------------------------------------------------------------------------
-// Column-stage kernels (Raman on, N1 = 64, M <= 16). One workgroup of 256 (or 512) lanes
-// owns one column n2 and does every column-side step of a stage there, with the
-// column of each field and Raman line held in LDS between the steps:
+// Column-stage kernels (N1 = 64, M <= 16; with Raman, and C2 in FP64 also without). One workgroup of 256 lanes
+// or more owns one column n2, or a few neighbouring ones, and does every column-side step of a stage there, with
+// the column of each field and Raman line held in LDS between the steps:
 //   C1  inverse column DFT of the M fields -> U (HBM, column order, and LDS) -> pair
 //       products -> forward column DFT of the Raman lines -> conv (row order, or column
 //       order on large grids; the Raman row pass reads them so and writes column order)
 //   C2  inverse column DFT of the Raman lines (column order; kept in LDS) -> dense Kerr +
 //       Raman gather of the 64 samples, forming each slot mix X_s on the way -> forward
-//       column DFT of sigma -> yout
+//       column DFT of sigma -> yout; without Raman the inverse column DFT of the fields takes the lines' place
 // Column order: sample (n1, n2) of an array at n2 * N1 + n1, so that a column is one
 // contiguous run of N1 samples.
 // Lanes form 32 line slots of 8 lanes; a round transforms up to 32 lines.
@@ -988,10 +988,9 @@ __device__ __forceinline__ void fmac_bcast(double* B, double c, double x) {
 #undef MMP_FMAC_BCAST
 #undef MMP_BC
 
-// LDS of the products' C2: field rows (whole wavefronts of line slots, so that the transform of sigma has its
-// rows there), then the rows of a chunk's lines, which sigma takes over.
-// Steps of the vector gather whose coefficients are preloaded in registers (up to 6 modes): every
-// product once, and a shared group per further segment.
+// Steps of the vector gather whose coefficients pass through registers on their way to LDS (up to 6 modes): every
+// product once, and a shared group per further segment. Pairs whose slots differ in parity lie in two segments
+// and add steps (16 at 6 modes under the reference pair decode, where this is 12): those go straight to LDS.
 constexpr int steps_cap(int M, bool parity) {
   const int G = 16 / coef_pad(parity ? (M + 1) / 2 : M);
   return (M * M + G - 1) / G + 3;
@@ -1000,6 +999,9 @@ constexpr int steps_cap(int M, bool parity) {
 // all products: up to 6 modes with the parity structure, up to 5 without (6 modes: 18 lines in 24 rows and 19
 // steps would take 65,792 bytes; sigma in the lines' rows leaves 51,968)
 constexpr bool own_sigma(int M, int cols, bool parity) { return cols == 1 && M <= (parity ? 6 : 5); }
+// LDS of the products' C2: field rows (whole wavefronts of line slots, so that the transform of sigma has its
+// rows there), the rows of a chunk's lines, sigma's (in the lines' place where they are not its own), and up to 6 modes
+// the steps' coefficients.
 template <int M, int COLS, bool PAR>
 struct C2Cfg {
   static constexpr int UR = (M + 7) / 8 * 8;
@@ -2270,7 +2272,11 @@ size_t colstage_pairs_lds_bytes(int M, int columns, bool mixed) {
 // Measured on one MI355X (M = 2..15, NT = 4096..65536, 1 to 36 fibers): four columns per
 // workgroup took the pass from 0.6-1.5 TB/s to 2-3.4 TB/s; eight gained nothing over four
 // (twice the LDS, lower occupancy). Line groups fill the CUs when the column blocks alone are
-// too few, but each group transforms every field again, so a group keeps at least 4 lines.
+// too few, but each group transforms every field again, so a group keeps at least 4 lines of the general count.
+// FP64 with couplings symmetric in the pair runs about half of those (11 of 18 at 6 modes: groups of 2 and 3);
+// groups planned on the lines that run measured the same within 1 % over 232 forms (NT = 4096, us per step: 4
+// modes 72.7 as planned and 73.8, 6 modes 80.7 and 81.5, 13 modes 164 and 158), so one layout serves
+// the fiber whatever its couplings and whichever fibers join it.
 void colstage_pairs_plan(int M, int N2, int n_lines, int F, bool mixed, int& columns, int& groups) {
   columns = 1;
   for (int cw : {4, 2})
