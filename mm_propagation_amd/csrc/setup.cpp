@@ -255,7 +255,7 @@ std::vector<double> product_blocks(const Problem& P, const std::vector<double>& 
 // products run). Counted in FMAs of a sample: a nonzero 12 and a slot's mix 32 (24 and 16 up to 64 tiles of 64
 // samples, where the sums are a latency), a Raman line's half 256; against the column kernel, which is worse beyond
 // 12 modes than its passes saved, a nonzero 6 and a mix 64. Fitted on 520 lists of 13 to 32 modes at NT = 1024 to
-// 65536: within 1 % of the better one in the mean, 1.2x at worst. One MI355X, us per step, sparse and products: 32
+// 65536: 0.4 % from the better one in the mean, 1.2x at worst. One MI355X, us per step, sparse and products: 32
 // modes, NT = 16384, one nonzero a slot, no Raman 367 and 3067; 20 modes, NT = 4096, 3 % of a symmetric
 // list, no Raman 171 and 145; full lists 2995 and 254. Up to 12 modes the products won on every
 // list tried.
